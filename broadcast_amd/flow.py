@@ -305,6 +305,11 @@ class Flow:
         nz, zp = (1, int(self.case.kind == "cyl")) if split is None else (2, split)
         bufs = getattr(self, "_csr_bufs", None)
         if bufs is None:
+            # The library knows the arrays of its last CSR by their addresses,
+            # and the context outlives this Flow: new arrays may lie where an
+            # earlier Flow's were, with anything in them.  They are filled by
+            # a full build before a refresh may find them.
+            refresh = False
             # ~145 entries per interior row (29-cell stencil x 5 variables)
             cap = 160 * n
             bufs = (t.empty(n + 1, dtype=t.int32, device="cuda"), t.empty(cap, dtype=t.int32, device="cuda"),

@@ -361,7 +361,10 @@ int bca_jacobian_colored_csr(bca_ctx *ctx, const double *w, bca_metrics g, const
  * is checked against that call's; if no row changed only data is rewritten
  * (indptr and indices already hold this CSR) and *rebuilt = 0, otherwise the
  * whole CSR is rebuilt as bca_jacobian_colored_csr does and *rebuilt = 1.
- * The result is identical to bca_jacobian_colored_csr either way. */
+ * The result is identical to bca_jacobian_colored_csr either way.  The arrays
+ * are recognised by their addresses: the first call on newly allocated arrays
+ * is bca_jacobian_colored_csr's, since memory freed and handed out again can
+ * have the old addresses and other contents. */
 int bca_jacobian_colored_csr_refresh(bca_ctx *ctx, const double *w, bca_metrics g, const bca_phys *phys,
                                      const bca_bc_op *ops, int nops, const double *coefdiag, int nzones,
                                      int zparam, double mini, int *indptr, int *indices, double *data, long cap,
