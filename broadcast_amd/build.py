@@ -16,6 +16,9 @@ FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-fPIC", "-shared", "-std=c++17",
     # packed FP32 forms are kept out of the generated code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # matrix instructions accumulate in ordinary registers: without it every
+    # accumulator lane read by other instructions is copied out of an AGPR
+    "-mllvm", "-amdgpu-mfma-vgpr-form=1",
     "-Wno-unused-result",
 ]
 

@@ -174,145 +174,349 @@ __global__ void __launch_bounds__(256) k_gemm_f64_sub(int M, int N, int K, const
 // for i, j outside kk.  Every entry is one product out = A' - T U of a
 // GJ_T x GJ_T output tile, with T = A(i, kk) P^-1 (rows of kk: T = -P^-1)
 // and U = A(kk, j) (columns of kk: U = the identity), A' = A off the panel
-// rows and columns and 0 on them.  A workgroup (4 waves, one 64 x 64
-// quadrant each, v_mfma_f64_16x16x4f64) first issues the loads of its A'
-// tile into registers and of A(i, kk), A(kk, j) into LDS; meanwhile wave 0
-// inverts P in registers (lane r + 32 h holds row r, columns 16 h .. 16 h +
-// 15; each elimination step broadcasts the pivot row by lane shuffles).
-// Workgroup (0, 0) reports a pivot below tiny times the tile's largest
-// |entry| in *bad.  After n / GJ_NB steps Aout holds A^-1 (2 n^3 flops).
-// The Newton driver multiplies the off-diagonal blocks of its block row by
-// this inverse (one GEMM instead of two triangular solves) and applies it to
-// the right-hand sides of its solves.
+// rows and columns and 0 on them.  Panels are processed in turn, so the steps
+// are a serial chain and what bounds a block of 500-1000 unknowns is the
+// latency of one step, first of all the inversion of P.  That inversion is
+// therefore taken out of the step: nothing but the next step needs the next
+// pivot tile, so one extra workgroup of each launch forms that tile's update
+// from the same inputs, inverts it and stores the inverse in the tile's
+// place, beside the workgroups of the update; the step after it finds P^-1
+// where P would be (the first panel's comes from a launch of its own).  A step
+// on 640 unknowns takes 11 us against 37 with P inverted in every workgroup of
+// the step, column by column through lane shuffles, and 128 x 128 tiles; the
+// inverse 0.22 against 0.73 ms (480: 0.18 / 0.57, 1920: 1.33 / 2.29 ms).
 constexpr int GJ_NB = 32;
-constexpr int GJ_T = 128;
-__global__ void __launch_bounds__(256) k_gj_step(const double* __restrict__ Ain, long lda, double* __restrict__ Aout,
-                                                 long ldo, int n, int k0, int nb, double tiny, int* __restrict__ bad) {
-  __shared__ double P[GJ_NB][GJ_NB + 1];
-  // A(i, kk) of the tile's rows, overwritten by T (each wave reads and then
-  // writes only its own 32 rows)
-  __shared__ double AT[GJ_T][GJ_NB + 1];
-  __shared__ double U[GJ_NB][GJ_T + 1];
-  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-  const int lr = lane % 16, lk = lane / 16;
-  const int i0 = blockIdx.y * GJ_T, j0 = blockIdx.x * GJ_T;
-  const int wm = (wave / 2) * 64, wn = (wave % 2) * 64;
-  auto in_panel = [&](int g) { return g >= k0 && g < k0 + nb; };
-  // A' of this thread's output entries: D(lk + 4 t, lr) of MFMA tile (a, b)
-  double a0[4][4][4];
+constexpr int GJ_T = 64;
+
+// Doubles of a row-major tile through a buffer descriptor of its rows: an
+// index of NOWHERE is out of the descriptor's range, so such a load gives 0
+// and such a store is dropped, without a branch around either (a branch per
+// guarded load serialises the loads of a tile).
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+constexpr unsigned NOWHERE = ~0u;
+struct TileBuf {
+  __amdgpu_buffer_rsrc_t r;
+  // rows rows of pitch ld from p, n columns (at least one row)
+  __device__ TileBuf(const double* p, int rows, long ld, int n)
+      : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(p), 0, (int)(unsigned)(((rows - 1) * ld + n) * 8L),
+                                            0x00027000)) {}
+  __device__ double load(unsigned off) const {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+  }
+  __device__ void store(unsigned off, double v) const {
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, off, 0, 0);
+  }
+  __device__ double load(bool in, int row, long ld, int col) const {
+    return load(in ? (unsigned)(row * (int)ld + col) * 8u : NOWHERE);
+  }
+  __device__ void store(bool in, int row, long ld, int col, double v) const {
+    store(in ? (unsigned)(row * (int)ld + col) * 8u : NOWHERE, v);
+  }
+};
+
+__device__ inline double rcp64(double x) {
+  // v_rcp_f64 and two Newton steps: the reciprocal to within an ulp
+  double r = __builtin_amdgcn_rcp(x);
+  r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+  return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+}
+__device__ inline double readlane_f64(double x, int l) {
+  const long long b = __double_as_longlong(x);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, l);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), l);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// Inverse of a 2 x 2 block; amin / rmax: its two pivots |a| and |det / a| go
+// into the smallest |a| and the largest 1 / |det / a| seen.
+__device__ inline void inv2(double (&m)[2][2], double& amin, double& rmax) {
+  const double a = m[0][0], b = m[0][1], c = m[1][0], d = m[1][1];
+  const double r = rcp64(__builtin_fma(a, d, -(b * c)));
+  amin = fmin(amin, fabs(a));
+  rmax = fmax(rmax, fabs(a * r));
+  m[0][0] = d * r;
+  m[0][1] = -b * r;
+  m[1][0] = -c * r;
+  m[1][1] = a * r;
+}
+__device__ inline void mul2(const double (&x)[2][2], const double (&y)[2][2], double (&z)[2][2]) {
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int j = 0; j < 2; ++j) z[i][j] = __builtin_fma(x[i][1], y[1][j], x[i][0] * y[0][j]);
+}
+
+// In-place inverse of a 32 x 32 tile held by one wave in the accumulator
+// layout of v_mfma_f64_16x16x4f64 -- X[a][b][t] of lane l is S(16 a + l / 16 +
+// 4 t, 16 b + l % 16) -- by Gauss-Jordan steps on 4 pivots at a time.  In that
+// layout the register X[a][b][t] holds the rows 16 a + 4 t .. + 3, one per 16
+// lanes, which is the layout of a B operand (4 x 16), and the same register of
+// the transpose is the A operand (16 x 4) of the columns: with Y = S^T kept
+// beside X the rank-4 update is S -= C W with C from Y and W = Q R (R the
+// four pivot rows, Q the inverse of the 4 x 4 pivot block, by its 2 x 2
+// blocks), and Y -= W^T C^T swaps the operands; no value crosses lanes but the
+// 16 entries of the pivot block.  A chain of 8 such steps, against 32 of a
+// column-by-column elimination whose pivot rows go through lane shuffles.
+// Returns the smallest |pivot|, 0 where the inverse is not finite.
+__device__ inline double gj_inv32(f64x4 (&X)[2][2], f64x4 (&Y)[2][2]) {
+  const int lane = threadIdx.x % 64, lk = lane / 16;
+  const bool dg = lane % 4 == lk;
+  double amin = 1.7976931348623157e308, rmax = 0.0;
+#pragma unroll
+  for (int g = 0; g < 8; ++g) {
+    constexpr f64x4 zero4 = {0.0, 0.0, 0.0, 0.0};
+    const int ga = g / 4, gt = g % 4;
+    // the pivot block in 2 x 2 blocks (uniform over the wave)
+    double q[2][2][2][2];
+    const double piv = X[ga][ga][gt];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) q[i / 2][j / 2][i % 2][j % 2] = readlane_f64(piv, 16 * i + 4 * gt + j);
+    // this lane's column lies in the pivot columns of block column ga
+    const bool pc = lane % 16 / 4 == gt;
+    double br[2], ac[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      br[b] = X[ga][b][gt];
+      ac[b] = -Y[ga][b][gt];
+    }
+    // pivot columns of R: the identity; pivot rows of -C: the identity; both
+    // panels of the old tile: zero
+    br[ga] = pc ? (dg ? 1.0 : 0.0) : br[ga];
+    ac[ga] = pc ? (dg ? 1.0 : 0.0) : ac[ga];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      X[ga][a][gt] = 0.0;
+      Y[ga][a][gt] = 0.0;
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        const int gi = i0 + wm + 16 * a + lk + 4 * t, gj = j0 + wn + 16 * b + lr;
-        a0[a][b][t] = (gi < n && gj < n && !in_panel(gi) && !in_panel(gj)) ? Ain[(long)gi * lda + gj] : 0.0;
+        if (a == ga && t == gt) continue;
+        X[a][ga][t] = pc ? 0.0 : X[a][ga][t];
+        Y[a][ga][t] = pc ? 0.0 : Y[a][ga][t];
       }
-  for (int x = tid; x < GJ_T * GJ_NB; x += 256) {
-    const int r = x / GJ_NB, c = x % GJ_NB;
-    const int gi = i0 + r;
-    AT[r][c] = (gi < n && c < nb) ? Ain[(long)gi * lda + k0 + c] : 0.0;
-    const int q = x / GJ_T, cc = x % GJ_T;
-    const int gj = j0 + cc;
-    double u = 0.0;
-    if (in_panel(gj)) u = (q == gj - k0) ? 1.0 : 0.0;
-    else if (gj < n && q < nb) u = Ain[(long)(k0 + q) * lda + gj];
-    U[q][cc] = u;
+    }
+    // Q = inverse of [A B; C D]: A^-1, S = D - C A^-1 B, S^-1, then the blocks
+    double ab[2][2], ca[2][2], cab[2][2], z[2][2];
+    inv2(q[0][0], amin, rmax);
+    mul2(q[0][0], q[0][1], ab);
+    mul2(q[1][0], q[0][0], ca);
+    mul2(q[1][0], ab, cab);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) q[1][1][i][j] -= cab[i][j];
+    inv2(q[1][1], amin, rmax);
+    mul2(ab, q[1][1], q[0][1]);
+    mul2(q[1][1], ca, q[1][0]);
+    mul2(q[0][1], ca, z);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        q[0][0][i][j] += z[i][j];
+        q[0][1][i][j] = -q[0][1][i][j];
+        q[1][0][i][j] = -q[1][0][i][j];
+      }
+    // Q as an A operand: row l % 16 (rows past 3 zero), k = l / 16
+    double qr[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const double lo = lk % 2 ? q[i / 2][0][i % 2][1] : q[i / 2][0][i % 2][0];
+      const double hi = lk % 2 ? q[i / 2][1][i % 2][1] : q[i / 2][1][i % 2][0];
+      qr[i] = lk / 2 ? hi : lo;
+    }
+    const double q01 = lane % 2 ? qr[1] : qr[0], q23 = lane % 2 ? qr[3] : qr[2];
+    const double qa = lane % 16 < 4 ? (lane % 4 / 2 ? q23 : q01) : 0.0;
+    double w[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) w[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(qa, br[b], zero4, 0, 0, 0)[0];
+    // the next pivot block's tile first
+    const int na = (g + 1) / 4 % 2;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int a = (s / 2 + na) % 2, b = (s % 2 + na) % 2;
+      X[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ac[a], w[b], X[a][b], 0, 0, 0);
+      Y[b][a] = __builtin_amdgcn_mfma_f64_16x16x4f64(w[b], ac[a], Y[b][a], 0, 0, 0);
+    }
   }
-  if (wave == 0) {
-    const int r = lane % 32, h = lane / 32;
-    double p[16];
-    double amax = 0.0;
+  double nan = 0.0;
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int c = 16 * h + q;
-      const bool in = r < nb && c < nb;
-      p[q] = in ? Ain[(long)(k0 + r) * lda + k0 + c] : (r == c ? 1.0 : 0.0);
-      amax = fmax(amax, in ? fabs(p[q]) : 0.0);
-    }
+  for (int x = 0; x < 16; ++x) nan = __builtin_fma(X[x / 8][x / 4 % 2][x % 4], 0.0, nan);
+  return __ballot(nan != nan) ? 0.0 : fmin(amin, 1.0 / rmax);
+}
+
+// LDS of one workgroup: P^-1, A(i, kk) (then T) and U.  The pitches keep the
+// 32 lanes of a b64 access on 32 different bank pairs: an A operand reads
+// (row l % 16, k l / 16), so its pitch is 2 mod 32 doubles, a B operand (k,
+// column), pitch 16 mod 32.
+struct GjSmem {
+  double P[GJ_NB][GJ_NB + 16];
+  double AT[GJ_T][GJ_NB + 2];
+  double U[GJ_NB][GJ_T + 16];
+};
+
+// The inverse of the nb x nb tile S(r, c) = get(in, r, c) (identity where in is
+// false), read by one wave in both layouts, stored through put(in, r, c, value); a pivot
+// below tiny times the tile's largest |entry| sets *bad.
+template <class Get, class Put>
+__device__ inline void gj_invert_tile(int nb, double tiny, int* bad, const Get& get, const Put& put) {
+  const int lane = threadIdx.x % 64, lr = lane % 16, lk = lane / 16;
+  f64x4 X[2][2], Y[2][2];
+  double amax = 0.0;
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) amax = fmax(amax, __shfl_xor(amax, off));
-    const double thr = tiny * amax;
+  for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int k = 0; k < GJ_NB; ++k) {
-      const int kh = k / 16, kq = k % 16;
-      double rowk[16];
+    for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int q = 0; q < 16; ++q) rowk[q] = __shfl(p[q], k + 32 * h);
-      const double piv = __shfl(p[kq], k + 32 * kh);
-      const double f = __shfl(p[kq], r + 32 * kh);
-      if (k < nb && blockIdx.x == 0 && blockIdx.y == 0 && lane == 0 && !(fabs(piv) > thr)) *bad = 1;
-      const double pinv = 1.0 / piv;
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int c = 16 * h + q;
-        const double nk = rowk[q] * pinv;
-        if (r == k) p[q] = (c == k) ? pinv : nk;
-        else p[q] = (c == k) ? -f * pinv : p[q] - f * nk;
+      for (int t = 0; t < 4; ++t) {
+        const int r = 16 * a + lk + 4 * t, c = 16 * b + lr;
+        const bool in = r < nb && c < nb;
+        const double x = get(in, r, c), y = get(in, c, r);
+        X[a][b][t] = in ? x : (r == c ? 1.0 : 0.0);
+        Y[a][b][t] = in ? y : (r == c ? 1.0 : 0.0);
+        amax = fmax(amax, in ? fabs(x) : 0.0);
       }
-    }
+  const double pmin = gj_inv32(X, Y);
 #pragma unroll
-    for (int q = 0; q < 16; ++q) P[r][16 * h + q] = p[q];
+  for (int off = 32; off > 0; off >>= 1) amax = fmax(amax, __shfl_xor(amax, off));
+  // padded pivots are 1: only a tile of tiny entries could be judged by them
+  if (lane == 0 && !(pmin > tiny * amax)) *bad = 1;
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int r = 16 * a + lk + 4 * t, c = 16 * b + lr;
+        put(r < nb && c < nb, r, c, X[a][b][t]);
+      }
+}
+
+// The first panel's pivot tile, inverted in place (one wave).
+__global__ void __launch_bounds__(64) k_gj_first(double* __restrict__ A, long lda, int nb, double tiny,
+                                                 int* __restrict__ bad) {
+  const TileBuf t(A, nb, lda, nb);
+  gj_invert_tile(nb, tiny, bad, [&](bool in, int r, int c) { return t.load(in, r, lda, c); },
+                 [&](bool in, int r, int c, double v) { t.store(in, r, lda, c, v); });
+}
+
+// One step, panel k0 .. k0 + nb - 1 (its pivot tile in Ain already inverted);
+// nb2 columns in the panel after it (0: none), whose pivot tile the last
+// workgroup updates and inverts.
+__global__ void __launch_bounds__(256) k_gj_step(const double* __restrict__ Ain, long lda, double* __restrict__ Aout,
+                                                 long ldo, int n, int k0, int nb, int nb2, double tiny,
+                                                 int* __restrict__ bad) {
+  __shared__ GjSmem sm;
+  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+  const int lr = lane % 16, lk = lane / 16;
+  const int nt = (n + GJ_T - 1) / GJ_T;
+  const bool ahead = (int)blockIdx.x == nt * nt;  // the look-ahead workgroup
+  const int kn = k0 + nb;                         // next panel
+  const int i0 = ahead ? kn : (int)blockIdx.x / nt * GJ_T, j0 = ahead ? kn : (int)blockIdx.x % nt * GJ_T;
+  const int ni = ahead ? nb2 : n - i0, nj = ahead ? nb2 : n - j0;  // rows and columns present
+  auto in_panel = [&](int g) { return g >= k0 && g < kn; };
+  // the tile's rows and the panel's rows
+  const TileBuf rows(Ain + (long)i0 * lda, ni < GJ_T ? ni : GJ_T, lda, n), kk(Ain + (long)k0 * lda, nb, lda, n);
+#pragma unroll
+  for (int x = 0; x < GJ_T * GJ_NB / 256; ++x) {
+    const int r = x * 8 + tid / GJ_NB, c = tid % GJ_NB;
+    sm.AT[r][c] = rows.load(r < ni && c < nb, r, lda, k0 + c);
+    const int q = x * 4 + tid / GJ_T, cc = tid % GJ_T;
+    const double u = kk.load(cc < nj && q < nb, q, lda, j0 + cc);
+    sm.U[q][cc] = in_panel(j0 + cc) ? (q == j0 + cc - k0 ? 1.0 : 0.0) : u;
+  }
+#pragma unroll
+  for (int x = 0; x < GJ_NB * GJ_NB / 256; ++x) {
+    const int r = x * 8 + tid / GJ_NB, c = tid % GJ_NB;
+    sm.P[r][c] = kk.load(r < nb && c < nb, r, lda, k0 + c);
+  }
+  // A' of this thread's outputs: D(lk + 4 t, lr) of the wave's 2 x 2 MFMA
+  // tiles (the look-ahead tile: one 16 x 16 quadrant per wave)
+  const int wm = ahead ? wave / 2 * 16 : wave / 2 * 32, wn = ahead ? wave % 2 * 16 : wave % 2 * 32;
+  f64x4 acc[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int r = wm + 16 * a + lk + 4 * t, c = wn + 16 * b + lr;
+        const bool in = r < ni && c < nj && !in_panel(i0 + r) && !in_panel(j0 + c);
+        acc[a][b][t] = rows.load(in, r, lda, j0 + c);
+      }
+  __syncthreads();
+  // -T = -A(i, kk) P^-1 in place of A(i, kk): wave w its rows 16 w .. 16 w + 15
+  // (the look-ahead tile's 32 rows: waves 0 and 1); rows of kk: P^-1
+  if (!ahead || wave < 2) {
+    f64x4 t2[2] = {f64x4{0.0, 0.0, 0.0, 0.0}, f64x4{0.0, 0.0, 0.0, 0.0}};
+    double av[GJ_NB / 4], pv[GJ_NB / 4][2];
+#pragma unroll
+    for (int k = 0; k < GJ_NB / 4; ++k) {
+      av[k] = sm.AT[16 * wave + lr][4 * k + lk];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) pv[k][b] = sm.P[4 * k + lk][16 * b + lr];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < GJ_NB / 4; ++k)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) t2[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[k], pv[k][b], t2[b], 0, 0, 0);
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int r = 16 * wave + lk + 4 * t, c = 16 * b + lr;
+        sm.AT[r][c] = in_panel(i0 + r) ? sm.P[i0 + r - k0][c] : -t2[b][t];
+      }
   }
   __syncthreads();
-  // T = A(i, kk) P^-1: wave w rows 32 w .. 32 w + 31
-  {
-    f64x4 acc[2][2];
+  const TileBuf out(Aout + (long)i0 * ldo, ni < GJ_T ? ni : GJ_T, ldo, n);
+  if (ahead) {
+    // S = A(next, next) - T U, through LDS to wave 0, which inverts it
+    double av[GJ_NB / 4], bv[GJ_NB / 4];
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int b = 0; b < 2; ++b) acc[a][b] = f64x4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int k = 0; k < GJ_NB; k += 4) {
-      double av[2], bv[2];
-#pragma unroll
-      for (int a = 0; a < 2; ++a) av[a] = AT[32 * wave + 16 * a + lr][k + lk];
-#pragma unroll
-      for (int b = 0; b < 2; ++b) bv[b] = P[k + lk][16 * b + lr];
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a], bv[b], acc[a][b], 0, 0, 0);
+    for (int k = 0; k < GJ_NB / 4; ++k) {
+      av[k] = sm.AT[wm + lr][4 * k + lk];
+      bv[k] = sm.U[4 * k + lk][wn + lr];
     }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < GJ_NB / 4; ++k)
+      acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[k], bv[k], acc[0][0], 0, 0, 0);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) sm.P[wm + lk + 4 * t][wn + lr] = acc[0][0][t];
+    __syncthreads();
+    if (wave == 0)
+      gj_invert_tile(nb2, tiny, bad, [&](bool, int r, int c) { return sm.P[r][c]; },
+                     [&](bool in, int r, int c, double v) { out.store(in, r, ldo, kn + c, v); });
+    return;
+  }
+  double av[GJ_NB / 4][2], bv[GJ_NB / 4][2];
+#pragma unroll
+  for (int k = 0; k < GJ_NB / 4; ++k)
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      av[k][a] = sm.AT[wm + 16 * a + lr][4 * k + lk];
+      bv[k][a] = sm.U[4 * k + lk][wn + 16 * a + lr];
+    }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int k = 0; k < GJ_NB / 4; ++k)
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
       for (int b = 0; b < 2; ++b)
+        acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[k][a], bv[k][b], acc[a][b], 0, 0, 0);
+  auto next_tile = [&](int g) { return g >= kn && g < kn + nb2; };
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const int r = 32 * wave + 16 * a + lk + 4 * t, c = 16 * b + lr;
-          const int gi = i0 + r;
-          AT[r][c] = in_panel(gi) ? -P[gi - k0][c] : acc[a][b][t];
-        }
-  }
-  __syncthreads();
-  // out = A' - T U over the wave's 64 x 64 quadrant, 4 x 4 MFMA tiles
-  f64x4 acc[4][4];
+  for (int a = 0; a < 2; ++a)
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = f64x4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-  for (int k = 0; k < GJ_NB; k += 4) {
-    double av[4], bv[4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a) av[a] = AT[wm + 16 * a + lr][k + lk];
-#pragma unroll
-    for (int b = 0; b < 4; ++b) bv[b] = U[k + lk][wn + 16 * b + lr];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a], bv[b], acc[a][b], 0, 0, 0);
-  }
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        const int gi = i0 + wm + 16 * a + lk + 4 * t, gj = j0 + wn + 16 * b + lr;
-        if (gi < n && gj < n) Aout[(long)gi * ldo + gj] = a0[a][b][t] - acc[a][b][t];
+        const int r = wm + 16 * a + lk + 4 * t, c = wn + 16 * b + lr;
+        out.store(r < ni && c < nj && !(next_tile(i0 + r) && next_tile(j0 + c)), r, ldo, j0 + c, acc[a][b][t]);
       }
 }
 

@@ -1734,13 +1734,15 @@ int bca_inv_np(void* stream, double* A, int n, long ld, double* work, double tin
   if (!A || !bad || !work) return fail(-1, "null argument");
   if (n < 1 || ld < n) return fail(-1, "bca_inv_np: need n >= 1 and ld >= n");
   const hipStream_t s = (hipStream_t)stream;
-  const dim3 g((n + GJ_T - 1) / GJ_T, (n + GJ_T - 1) / GJ_T);
+  const int nt = (n + GJ_T - 1) / GJ_T;
   double* buf[2] = {A, work};
   const long ldb[2] = {ld, (long)n};
+  k_gj_first<<<1, 64, 0, s>>>(A, ld, std::min(GJ_NB, n), tiny, bad);
+  BCA_LAUNCHED();
+  if (n <= GJ_NB) return 0;  // one panel: its pivot tile is the block
   // Panels of GJ_NB columns; the steps alternate between A and work, so an
   // even number of them ends in A.  An odd count splits its last panel in
-  // two (or, when that panel is one column wide, the full panel before it),
-  // and n = 1 adds a step over no column (nb = 0 copies Ain to Aout).
+  // two (or, when that panel is one column wide, the full panel before it).
   std::vector<int> widths;
   for (int k0 = 0; k0 < n; k0 += GJ_NB) widths.push_back(std::min(GJ_NB, n - k0));
   if (widths.size() % 2 == 1) {
@@ -1748,16 +1750,16 @@ int bca_inv_np(void* stream, double* A, int n, long ld, double* work, double tin
     if (r >= 2) {
       widths.back() = r - r / 2;
       widths.push_back(r / 2);
-    } else if (widths.size() >= 2) {
+    } else {
       widths[widths.size() - 2] = GJ_NB / 2;
       widths.insert(widths.end() - 1, GJ_NB - GJ_NB / 2);
-    } else {
-      widths.push_back(0);
     }
   }
   int cur = 0, k0 = 0;
-  for (const int nb : widths) {
-    k_gj_step<<<g, 256, 0, s>>>(buf[cur], ldb[cur], buf[1 - cur], ldb[1 - cur], n, k0, nb, tiny, bad);
+  for (size_t q = 0; q < widths.size(); ++q) {
+    const int nb = widths[q], nb2 = q + 1 < widths.size() ? widths[q + 1] : 0;
+    k_gj_step<<<nt * nt + (nb2 ? 1 : 0), 256, 0, s>>>(buf[cur], ldb[cur], buf[1 - cur], ldb[1 - cur], n, k0, nb, nb2,
+                                                      tiny, bad);
     BCA_LAUNCHED();
     cur = 1 - cur;
     k0 += nb;
