@@ -99,9 +99,13 @@ _SIGS = {
     "bca_gemm_bf16": [_dp, C.c_int, C.c_int, C.c_int, _dp, C.c_long, C.c_long, _dp, C.c_long, C.c_long, _dp,
                       C.c_long, C.c_long, C.c_int, C.c_int],
     "bca_lu_np": [_dp, _dp, C.c_int, C.c_long, C.c_double, _dp, _dp],
+    "bca_band_factor": [C.POINTER(C.c_void_p), _dp, _dp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _dp, C.c_double,
+                        _dp],
+    "bca_band_solve": [_dp, _dp, _dp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _dp, _dp],
     "bca_inv_np": [_dp, _dp, C.c_int, C.c_long, _dp, C.c_double, _dp],
     "bca_gemm_f64_sub": [_dp, C.c_int, C.c_int, C.c_int, _dp, C.c_long, _dp, C.c_long, _dp, C.c_long],
     "bca_csr_spmv": [_dp, C.c_long, _dp, _dp, _dp, _dp, _dp],
+    "bca_csr_residual": [_dp, C.c_long, _dp, _dp, _dp, _dp, _dp, _dp],
 }
 
 _LONG_RESULT = ("bca_ctx_scratch_bytes", "bca_residual_noalloc_bytes")

@@ -23,6 +23,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "scheme.h"
+
 namespace bca {
 
 constexpr int LU_NB = 32;
@@ -393,9 +395,18 @@ __device__ inline void gj_invert_tile(int nb, double tiny, int* bad, const Get& 
       }
 }
 
+// The blocks of one launch (blockIdx.y): the two ends of a band go through
+// their steps together.
+constexpr int GJ_BATCH = 2;
+struct GjPair {
+  double* in[GJ_BATCH];
+  double* out[GJ_BATCH];
+};
+
 // The first panel's pivot tile, inverted in place (one wave).
-__global__ void __launch_bounds__(64) k_gj_first(double* __restrict__ A, long lda, int nb, double tiny,
-                                                 int* __restrict__ bad) {
+__global__ void __launch_bounds__(64) k_gj_first(GjPair m, long lda, int nb, double tiny, int* __restrict__ bad) {
+  __builtin_amdgcn_s_setprio(3);
+  double* A = m.in[blockIdx.y];
   const TileBuf t(A, nb, lda, nb);
   gj_invert_tile(nb, tiny, bad, [&](bool in, int r, int c) { return t.load(in, r, lda, c); },
                  [&](bool in, int r, int c, double v) { t.store(in, r, lda, c, v); });
@@ -404,10 +415,12 @@ __global__ void __launch_bounds__(64) k_gj_first(double* __restrict__ A, long ld
 // One step, panel k0 .. k0 + nb - 1 (its pivot tile in Ain already inverted);
 // nb2 columns in the panel after it (0: none), whose pivot tile the last
 // workgroup updates and inverts.
-__global__ void __launch_bounds__(256) k_gj_step(const double* __restrict__ Ain, long lda, double* __restrict__ Aout,
-                                                 long ldo, int n, int k0, int nb, int nb2, double tiny,
-                                                 int* __restrict__ bad) {
+__global__ void __launch_bounds__(256) k_gj_step(GjPair m, long lda, long ldo, int n, int k0, int nb, int nb2,
+                                                 double tiny, int* __restrict__ bad) {
   __shared__ GjSmem sm;
+  const double* Ain = m.in[blockIdx.y];
+  double* Aout = m.out[blockIdx.y];
+  __builtin_amdgcn_s_setprio(3);  // the chain goes before the bulk products on its CU
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
   const int lr = lane % 16, lk = lane / 16;
   const int nt = (n + GJ_T - 1) / GJ_T;
@@ -520,14 +533,208 @@ __global__ void __launch_bounds__(256) k_gj_step(const double* __restrict__ Ain,
       }
 }
 
-// y = A x for a CSR matrix (one row per thread).
-__global__ void k_csr_spmv(long n, const int* __restrict__ indptr, const int* __restrict__ indices,
-                           const double* __restrict__ data, const double* __restrict__ x, double* __restrict__ y) {
-  const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
+// ------------------------------------------------------------------ block products
+// C (=, or -=) A B for a list of B x B blocks in one launch, row-major with
+// their own pitches: the products of one block step are independent, and one
+// launch over all their tiles fills the chip where a launch per product leaves
+// a partly filled last round each.  A workgroup of 2 x 2 waves forms a
+// (32 MT) x (32 NT) tile of one product, each wave MT x NT MFMA tiles
+// (v_mfma_f64_16x16x4f64, 64 cycles each), K in slices of KS through two LDS
+// buffers, the next slice loaded into registers under the current one's
+// products.  Offsets within a slice are fixed per thread and only the
+// descriptors move: with the offsets formed anew for each slice a lone
+// workgroup on a CU spent as long on them as on its products.  64 x 64 tiles,
+// slices of 16 (four workgroups a CU): 8 products of 640^3 in 92 us (46
+// TFLOP/s: 800 tiles are 3.1 a CU), of 1920^3 in 1.71 ms (66; the card's
+// matrix cores sustain 69).  The elimination's chain has one product at a
+// time: 32 x 32 tiles and slices of 32 put 640^3 on every CU, 22 us against 41
+// with 64 x 64.
+// The bulk products ask for BG_RESERVE bytes of LDS they do not use: with two
+// of them on a CU instead of four there is room for a workgroup of the
+// elimination's chain, which would otherwise wait for one of them to end.
+constexpr int BG_MAX = 16;
+constexpr int BG_RESERVE = 16 * 1024;
+struct BlockProduct {
+  const double* A;
+  const double* B;
+  double* C;
+  int lda, ldb, ldc;
+};
+struct BlockProducts {
+  BlockProduct p[BG_MAX];
+};
+
+template <int MT, int NT, int KS, bool SUB>
+__global__ void __launch_bounds__(256) k_block_products(BlockProducts list, int n) {
+  constexpr int TM = 32 * MT, TN = 32 * NT;
+  // pitches: an A operand reads (row l % 16, k l / 16), a B operand (k l / 16,
+  // column l % 16); 2 mod 4 and 16 mod 32 doubles spread 32 lanes over all banks
+  __shared__ double As[2][TM][KS + 2];
+  __shared__ double Bs[2][KS][TN + 16];
+  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+  const int lr = lane % 16, lk = lane / 16;
+  const int ntn = (n + TN - 1) / TN;
+  int bx, by;
+  xcd_block(bx, by);
+  const BlockProduct q = list.p[by];
+  if constexpr (MT == 1) __builtin_amdgcn_s_setprio(3);
+  const int m0 = bx / ntn * TM, n0 = bx % ntn * TN;
+  const int mr = min(TM, n - m0);
+  const int wm = wave / 2 * 16 * MT, wn = wave % 2 * 16 * NT;
+  constexpr int NA = TM * KS / 256, NB = TN * KS / 256;
+  static_assert(256 % KS == 0 && 256 % TN == 0, "staging shape");
+  // this thread's elements of a slice: fixed offsets from its first one, which
+  // moves by a scalar amount from slice to slice
+  unsigned oa[NA], ob[NB];
+#pragma unroll
+  for (int x = 0; x < NA; ++x) {
+    const int r = x * (256 / KS) + tid / KS;
+    oa[x] = r < mr ? (unsigned)(r * q.lda + tid % KS) * 8u : NOWHERE;
+  }
+#pragma unroll
+  for (int x = 0; x < NB; ++x) {
+    const int r = x * (256 / TN) + tid / TN;
+    ob[x] = n0 + tid % TN < n ? (unsigned)(r * q.ldb + n0 + tid % TN) * 8u : NOWHERE;
+  }
+  double ra[NA], rb[NB];
+  auto fetch = [&](int k0) {
+    const int kr = min(KS, n - k0);
+    const TileBuf ta(q.A + (long)m0 * q.lda + k0, mr, q.lda, kr), tb(q.B + (long)k0 * q.ldb, kr, q.ldb, n);
+    if (kr == KS) {
+#pragma unroll
+      for (int x = 0; x < NA; ++x) ra[x] = ta.load(oa[x]);
+#pragma unroll
+      for (int x = 0; x < NB; ++x) rb[x] = tb.load(ob[x]);
+    } else {
+      // the last, shorter slice: zeros past it
+#pragma unroll
+      for (int x = 0; x < NA; ++x) ra[x] = ta.load(tid % KS < kr ? oa[x] : NOWHERE);
+#pragma unroll
+      for (int x = 0; x < NB; ++x) rb[x] = tb.load(x * (256 / TN) + tid / TN < kr ? ob[x] : NOWHERE);
+    }
+  };
+  auto stage = [&](int s) {
+#pragma unroll
+    for (int x = 0; x < NA; ++x) As[s][x * (256 / KS) + tid / KS][tid % KS] = ra[x];
+#pragma unroll
+    for (int x = 0; x < NB; ++x) Bs[s][x * (256 / TN) + tid / TN][tid % TN] = rb[x];
+  };
+  const TileBuf tc(q.C + (long)m0 * q.ldc, mr, q.ldc, n);
+  f64x4 acc[MT][NT], cv[MT][NT];
+#pragma unroll
+  for (int a = 0; a < MT; ++a)
+#pragma unroll
+    for (int b = 0; b < NT; ++b) acc[a][b] = f64x4{0.0, 0.0, 0.0, 0.0};
+  auto slice = [&](int k0, int s) {
+    const bool more = k0 + KS < n;
+    if (more) fetch(k0 + KS);
+#pragma unroll
+    for (int k = 0; k < KS; k += 4) {
+      double av[MT], bv[NT];
+#pragma unroll
+      for (int a = 0; a < MT; ++a) av[a] = As[s][wm + 16 * a + lr][k + lk];
+#pragma unroll
+      for (int b = 0; b < NT; ++b) bv[b] = Bs[s][k + lk][wn + 16 * b + lr];
+#pragma unroll
+      for (int a = 0; a < MT; ++a)
+#pragma unroll
+        for (int b = 0; b < NT; ++b) acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a], bv[b], acc[a][b], 0, 0, 0);
+    }
+    if (more) stage(s ^ 1);
+    __syncthreads();
+  };
+  fetch(0);
+  stage(0);
+  __syncthreads();
+  for (int k0 = 0; k0 < n; k0 += 2 * KS) {
+    slice(k0, 0);
+    if (k0 + KS < n) slice(k0 + KS, 1);
+  }
+  // all of C in flight together
+  auto coff = [&](int a, int b, int t) {
+    const int r = wm + 16 * a + lk + 4 * t, c = n0 + wn + 16 * b + lr;
+    return r < mr && c < n ? (unsigned)(r * q.ldc + c) * 8u : NOWHERE;
+  };
+  if constexpr (SUB)
+#pragma unroll
+    for (int x = 0; x < MT * NT * 4; ++x) cv[x / 4 / NT][x / 4 % NT][x % 4] = tc.load(coff(x / 4 / NT, x / 4 % NT, x % 4));
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int x = 0; x < MT * NT * 4; ++x) {
+    const int a = x / 4 / NT, b = x / 4 % NT, t = x % 4;
+    tc.store(coff(a, b, t), SUB ? cv[a][b][t] - acc[a][b][t] : acc[a][b][t]);
+  }
+}
+
+// Scratch blocks into place: dst(r, c) = src(r, c) for n x n blocks, a row per
+// workgroup.
+struct CopyRow {
+  const double* src;
+  double* dst;
+  int lds, ldd;
+};
+struct CopyRows {
+  CopyRow c[BG_MAX];
+};
+__global__ void __launch_bounds__(256) k_copy_rows(CopyRows list, int n) {
+  const CopyRow q = list.c[blockIdx.y];
+  const double* s = q.src + (long)blockIdx.x * q.lds;
+  double* d = q.dst + (long)blockIdx.x * q.ldd;
+  for (int c = threadIdx.x; c < n; c += 256) d[c] = s[c];
+}
+
+// ------------------------------------------------------------------ band solve
+// Matrix-vector products of one step of the band solve, one wave per row: for
+// every job, y(r) (=, or -=) sum_c A(r, c) x(c), r < rows, c < n.  A step's
+// jobs are independent (both ends of the band, all block rows a step reaches),
+// so they share a launch; what bounds the solve is the chain of launches, two
+// a block row forward and one back.
+constexpr int BV_MAX = 8;
+struct BandVec {
+  const double* A;
+  const double* x;
+  double* y;
+  long lda;
+  int n, sub;
+};
+struct BandVecs {
+  BandVec j[BV_MAX];
+};
+__global__ void __launch_bounds__(256) k_band_vec(BandVecs list, int rows) {
+  const BandVec q = list.j[blockIdx.y];
+  const int r = blockIdx.x * 4 + threadIdx.x / 64, lane = threadIdx.x % 64;
+  if (r >= rows) return;
+  const double* a = q.A + r * q.lda;
+  double s0 = 0.0, s1 = 0.0;
+  int c = lane;
+  for (; c + 64 < q.n; c += 128) {
+    s0 += a[c] * q.x[c];
+    s1 += a[c + 64] * q.x[c + 64];
+  }
+  if (c < q.n) s0 += a[c] * q.x[c];
+  s0 += s1;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s0 += __shfl_xor(s0, off);
+  if (lane == 0) q.y[r] = q.sub ? q.y[r] - s0 : s0;
+}
+
+// y = A x for a CSR matrix, or b - A x where b is given: one wave per row, so
+// that a row's ~145 entries are consecutive loads (with one row per thread
+// each lane walked its own row: 390 us for 164k rows of the 256 x 128 boundary
+// layer).
+__global__ void __launch_bounds__(256) k_csr_spmv(long n, const int* __restrict__ indptr,
+                                                  const int* __restrict__ indices, const double* __restrict__ data,
+                                                  const double* __restrict__ x, const double* __restrict__ b,
+                                                  double* __restrict__ y) {
+  const long r = (long)blockIdx.x * 4 + threadIdx.x / 64;
+  const int lane = threadIdx.x % 64;
   if (r >= n) return;
   double s = 0.0;
-  for (int p = indptr[r]; p < indptr[r + 1]; ++p) s += data[p] * x[indices[p]];
-  y[r] = s;
+  const int end = indptr[r + 1];
+  for (int p = indptr[r] + lane; p < end; p += 64) s += data[p] * x[indices[p]];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+  if (lane == 0) y[r] = b ? b[r] - s : s;
 }
 
 }  // namespace bca

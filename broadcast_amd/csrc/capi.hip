@@ -1730,14 +1730,20 @@ int bca_lu_np(void* stream, double* A, int n, long ld, double tiny, int* bad, do
   return 0;
 }
 
-int bca_inv_np(void* stream, double* A, int n, long ld, double* work, double tiny, int* bad) {
-  if (!A || !bad || !work) return fail(-1, "null argument");
-  if (n < 1 || ld < n) return fail(-1, "bca_inv_np: need n >= 1 and ld >= n");
-  const hipStream_t s = (hipStream_t)stream;
+}  // extern "C"
+
+namespace {
+
+// In-place inverses of `batch` n x n blocks (pitch ld), work n x n each.
+int invert_blocks(hipStream_t s, int batch, double* const A[], int n, long ld, double* const work[], double tiny,
+                  int* bad) {
   const int nt = (n + GJ_T - 1) / GJ_T;
-  double* buf[2] = {A, work};
-  const long ldb[2] = {ld, (long)n};
-  k_gj_first<<<1, 64, 0, s>>>(A, ld, std::min(GJ_NB, n), tiny, bad);
+  GjPair m{};
+  for (int q = 0; q < batch; ++q) {
+    m.in[q] = A[q];
+    m.out[q] = work[q];
+  }
+  k_gj_first<<<dim3(1, batch), 64, 0, s>>>(m, ld, std::min(GJ_NB, n), tiny, bad);
   BCA_LAUNCHED();
   if (n <= GJ_NB) return 0;  // one panel: its pivot tile is the block
   // Panels of GJ_NB columns; the steps alternate between A and work, so an
@@ -1755,16 +1761,282 @@ int bca_inv_np(void* stream, double* A, int n, long ld, double* work, double tin
       widths.insert(widths.end() - 1, GJ_NB - GJ_NB / 2);
     }
   }
-  int cur = 0, k0 = 0;
+  long ldi = ld, ldo = n;
+  int k0 = 0;
   for (size_t q = 0; q < widths.size(); ++q) {
     const int nb = widths[q], nb2 = q + 1 < widths.size() ? widths[q + 1] : 0;
-    k_gj_step<<<nt * nt + (nb2 ? 1 : 0), 256, 0, s>>>(buf[cur], ldb[cur], buf[1 - cur], ldb[1 - cur], n, k0, nb, nb2,
-                                                      tiny, bad);
+    k_gj_step<<<dim3(nt * nt + (nb2 ? 1 : 0), batch), 256, 0, s>>>(m, ldi, ldo, n, k0, nb, nb2, tiny, bad);
     BCA_LAUNCHED();
-    cur = 1 - cur;
+    std::swap(ldi, ldo);
+    for (int x = 0; x < batch; ++x) std::swap(m.in[x], m.out[x]);
     k0 += nb;
   }
-  if (cur != 0 || k0 != n) return fail(-3, "bca_inv_np: internal panel schedule");
+  if (widths.size() % 2 != 0 || k0 != n) return fail(-3, "inverse: internal panel schedule");
+  return 0;
+}
+
+}  // namespace
+
+extern "C" {
+
+int bca_inv_np(void* stream, double* A, int n, long ld, double* work, double tiny, int* bad) {
+  if (!A || !bad || !work) return fail(-1, "null argument");
+  if (n < 1 || ld < n) return fail(-1, "bca_inv_np: need n >= 1 and ld >= n");
+  return invert_blocks((hipStream_t)stream, 1, &A, n, ld, &work, tiny, bad);
+}
+
+}  // extern "C"
+
+namespace {
+
+// Block-banded elimination from both ends of the band at once.
+//
+// Block rows 0 .. mid - 1 are eliminated downwards, nb - 1 .. mid + kb
+// upwards, then the kb rows between them downwards; mid = nb eliminates
+// everything downwards.  The steps of one direction are a serial chain (the
+// inverse of a diagonal block needs the step before it) whose launches leave
+// most of the chip idle; the two directions are independent until they meet,
+// so every launch carries a step of both: half the chain with the same
+// products.  64 block rows of 480 unknowns, kb = 3: 10.3 ms against 16.7 ms
+// downwards only, of 640: 20.8 / 22.3 ms (there the products fill the chip).
+// With the products by rocBLAS (and torch's subtractions) one Newton iteration
+// on the 256 x 128 boundary layer took 128 ms, now 72 ms.
+//
+// Step I with neighbours K_d = I +- d, d = 1 .. h:
+//   chain stream  D_I^-1 in place, X_1 = D_I^-1 A(I, K_1) into the scratch
+//                 row, A(K_1, K_1) -= A(K_1, I) X_1, then the next step's
+//                 inverse
+//   main stream   X_d, d = 2 .. h, the other h^2 - 1 updates A(K_d, K_e) -=
+//                 A(K_d, I) X_e, and X into the place of A(I, K_d)
+// The chain waits for the main stream's updates of the step before (they
+// write A(I, K_1) and A(K_1, K_1), and read the scratch row).
+struct BandStreams {
+  hipStream_t chain, main;
+  hipEvent_t ready, upd;
+};
+struct BandStep {
+  int I, dir, h;
+  double *work, *X;  // B x B, B x (kb + nfar) B
+};
+
+struct BandMatrix {
+  double *R, *F;
+  int nb, B, kb, nfar;
+  long W() const { return (long)(2 * kb + 1) * B; }
+  double* at(int K, int J) const { return R + (long)K * B * W() + (long)(J - K + kb) * B; }
+};
+
+template <int MT, int NT, int KS, bool SUB>
+int block_products(hipStream_t s, const std::vector<BlockProduct>& v, int n) {
+  for (size_t q = 0; q < v.size(); q += BG_MAX) {
+    const int c = (int)std::min(v.size() - q, (size_t)BG_MAX);
+    BlockProducts l{};
+    for (int x = 0; x < c; ++x) l.p[x] = v[q + x];
+    const unsigned nt = (unsigned)((n + 32 * MT - 1) / (32 * MT)) * (unsigned)((n + 32 * NT - 1) / (32 * NT));
+    k_block_products<MT, NT, KS, SUB><<<dim3(nt, c), 256, MT == 1 ? 0 : BG_RESERVE, s>>>(l, n);
+    BCA_LAUNCHED();
+  }
+  return 0;
+}
+
+int band_step(const BandMatrix& a, const BandStreams& c, const std::vector<BandStep>& st, double tiny, int* bad) {
+  const int B = a.B, W = (int)a.W(), ldx = (a.kb + a.nfar) * B;
+  double *D[GJ_BATCH], *work[GJ_BATCH];
+  for (size_t q = 0; q < st.size(); ++q) {
+    D[q] = a.at(st[q].I, st[q].I);
+    work[q] = st[q].work;
+  }
+  int rc = invert_blocks(c.chain, (int)st.size(), D, B, W, work, tiny, bad);
+  if (rc) return rc;
+  // the first neighbour on the chain, everything else on the main stream
+  std::vector<BlockProduct> x1, u1, px, pu;
+  for (const BandStep& q : st) {
+    const int I = q.I;
+    auto K = [&](int d) { return I + q.dir * d; };
+    auto X = [&](int d) { return q.X + (long)(d - 1) * B; };
+    if (q.h == 0) continue;
+    x1.push_back({a.at(I, I), a.at(I, K(1)), X(1), W, W, ldx});
+    u1.push_back({a.at(K(1), I), X(1), a.at(K(1), K(1)), W, ldx, W});
+    // the far blocks of block row 0 (columns kb + 1 .. kb + nfar) ride along
+    const int far = (I == 0 && q.dir > 0) ? a.nfar : 0;
+    for (int d = 2; d <= q.h; ++d) px.push_back({a.at(I, I), a.at(I, K(d)), X(d), W, W, ldx});
+    for (int f = 1; f <= far; ++f)
+      px.push_back({a.at(I, I), a.F + (long)(f - 1) * B, X(a.kb + f), W, a.nfar * B, ldx});
+    for (int d = 1; d <= q.h; ++d) {
+      for (int e = 1; e <= q.h; ++e)
+        if (d > 1 || e > 1) pu.push_back({a.at(K(d), I), X(e), a.at(K(d), K(e)), W, ldx, W});
+      for (int f = 1; f <= far; ++f)
+        if (a.kb + f - K(d) <= a.kb) pu.push_back({a.at(K(d), I), X(a.kb + f), a.at(K(d), a.kb + f), W, ldx, W});
+    }
+  }
+  if (x1.empty()) return 0;
+  BCA_HIP(hipStreamWaitEvent(c.chain, c.upd, 0));
+  if ((rc = block_products<1, 1, 32, false>(c.chain, x1, B))) return rc;
+  if ((rc = block_products<1, 1, 32, true>(c.chain, u1, B))) return rc;
+  // the bulk starts when the chain is back in an inverse, which leaves most of
+  // the chip to it (beside the chain's own products it took longer than it won)
+  BCA_HIP(hipEventRecord(c.ready, c.chain));
+  BCA_HIP(hipStreamWaitEvent(c.main, c.ready, 0));
+  if ((rc = block_products<2, 2, 16, false>(c.main, px, B))) return rc;
+  if ((rc = block_products<2, 2, 16, true>(c.main, pu, B))) return rc;
+  // X into the place of A(I, K_d)
+  CopyRows cp{};
+  int nc = 0;
+  auto flush = [&]() -> int {
+    if (nc == 0) return 0;
+    k_copy_rows<<<dim3((unsigned)B, nc), 256, 0, c.main>>>(cp, B);
+    BCA_LAUNCHED();
+    nc = 0;
+    return 0;
+  };
+  for (const BandStep& q : st) {
+    const int far = (q.I == 0 && q.dir > 0) ? a.nfar : 0;
+    for (int d = 1; d <= q.h + far; ++d) {
+      const bool f = d > q.h;
+      cp.c[nc++] = f ? CopyRow{q.X + (long)(a.kb + d - q.h - 1) * B, a.F + (long)(d - q.h - 1) * B, ldx, a.nfar * B}
+                     : CopyRow{q.X + (long)(d - 1) * B, a.at(q.I, q.I + q.dir * d), ldx, W};
+      if (nc == BG_MAX && (rc = flush())) return rc;
+    }
+  }
+  if ((rc = flush())) return rc;
+  BCA_HIP(hipEventRecord(c.upd, c.main));
+  return 0;
+}
+
+int band_check(const BandMatrix& a, int mid) {
+  if (a.nb < 1 || a.B < 1 || a.kb < 0 || a.kb > a.nb || a.nfar < 0) return fail(-1, "band: bad block counts");
+  if (mid != a.nb && (mid < 1 || mid + a.kb >= a.nb)) return fail(-1, "band: mid must be nb or leave rows on both ends");
+  if (a.W() * 8L * 128 > 2147483647L) return fail(-1, "band: block row too wide");
+  return 0;
+}
+
+}  // namespace
+
+extern "C" {
+
+int bca_band_factor(void* const streams[3], double* R, double* F, int nb, int B, int kb, int nfar, int mid,
+                    double* scratch, double tiny, int* bad) {
+  if (!streams || !R || !scratch || !bad || (nfar > 0 && !F)) return fail(-1, "null argument");
+  const BandMatrix a{R, F, nb, B, kb, nfar};
+  int rc = band_check(a, mid);
+  if (rc) return rc;
+  hipEvent_t ev[3] = {};
+  auto done = [&](int r) {
+    for (hipEvent_t e : ev)
+      if (e) (void)hipEventDestroy(e);
+    return r;
+  };
+  for (hipEvent_t& e : ev)
+    if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return done(fail(-2, "hipEventCreate"));
+  const hipStream_t cur = (hipStream_t)streams[0];
+  const BandStreams c{(hipStream_t)streams[1], (hipStream_t)streams[2], ev[0], ev[1]};
+  auto order = [&](hipStream_t after, hipStream_t before) -> int {
+    if (after == before) return 0;
+    BCA_HIP(hipEventRecord(ev[2], before));
+    BCA_HIP(hipStreamWaitEvent(after, ev[2], 0));
+    return 0;
+  };
+  // everything starts after what is queued on the caller's stream
+  if ((rc = order(c.chain, cur)) || (rc = order(c.main, cur))) return done(rc);
+  const long per = (long)B * B * (1 + kb + nfar);
+  auto down = [&](int I, int h) { return BandStep{I, 1, h, scratch, scratch + (long)B * B}; };
+  auto up = [&](int t) { return BandStep{nb - 1 - t, -1, kb, scratch + per, scratch + per + (long)B * B}; };
+  const int top = mid, bottom = mid == nb ? 0 : nb - mid - kb;
+  // the rows between are written by both ends in their last kb steps: the
+  // upward end's go after the downward end
+  for (int t = 0; t < std::max(top, bottom - kb); ++t) {
+    std::vector<BandStep> st;
+    if (t < top) st.push_back(down(t, std::min(kb, nb - 1 - t)));
+    if (t < bottom - kb) st.push_back(up(t));
+    if ((rc = band_step(a, c, st, tiny, bad))) return done(rc);
+  }
+  for (int t = std::max(bottom - kb, 0); t < bottom; ++t)
+    if ((rc = band_step(a, c, {up(t)}, tiny, bad))) return done(rc);
+  if (bottom > 0) {
+    // row mid is not the last step's neighbour on the chain: its diagonal
+    // block was updated on the main stream too
+    if ((rc = order(c.chain, c.main))) return done(rc);
+    for (int I = mid; I < mid + kb; ++I)
+      if ((rc = band_step(a, c, {down(I, mid + kb - 1 - I)}, tiny, bad))) return done(rc);
+  }
+  if ((rc = order(cur, c.chain)) || (rc = order(cur, c.main))) return done(rc);
+  return done(0);
+}
+
+int bca_band_solve(void* stream, const double* R, const double* F, int nb, int B, int kb, int nfar, int mid, double* y,
+                   double* z) {
+  if (!R || !y || !z || (nfar > 0 && !F)) return fail(-1, "null argument");
+  const BandMatrix a{const_cast<double*>(R), const_cast<double*>(F), nb, B, kb, nfar};
+  int rc = band_check(a, mid);
+  if (rc) return rc;
+  const hipStream_t s = (hipStream_t)stream;
+  const long W = a.W();
+  auto launch = [&](const std::vector<BandVec>& v) -> int {
+    for (size_t q = 0; q < v.size(); q += BV_MAX) {
+      const int c = (int)std::min(v.size() - q, (size_t)BV_MAX);
+      BandVecs l{};
+      for (int x = 0; x < c; ++x) l.j[x] = v[q + x];
+      k_band_vec<<<dim3((unsigned)((B + 3) / 4), c), 256, 0, s>>>(l, B);
+      BCA_LAUNCHED();
+    }
+    return 0;
+  };
+  auto vec = [&](double* p, int K) { return p + (long)K * B; };
+  // z_I = D_I^-1 y_I, then y_K -= A(K, I) z_I for the rows I reaches
+  struct Step {
+    int I, dir, h;
+  };
+  auto forward = [&](const std::vector<Step>& st) -> int {
+    std::vector<BandVec> v;
+    for (const Step& q : st) v.push_back({a.at(q.I, q.I), vec(y, q.I), vec(z, q.I), W, B, 0});
+    if (int e = launch(v)) return e;
+    v.clear();
+    for (const Step& q : st)
+      for (int d = 1; d <= q.h; ++d) {
+        const int K = q.I + q.dir * d;
+        v.push_back({a.at(K, q.I), vec(z, q.I), vec(y, K), W, B, 1});
+      }
+    return launch(v);
+  };
+  // z_I -= sum_d X(I, K_d) z_K_d: the K_d are one run of columns
+  auto backward = [&](const std::vector<Step>& st) -> int {
+    std::vector<BandVec> v;
+    for (const Step& q : st) {
+      if (q.h == 0) continue;
+      const int K0 = q.dir > 0 ? q.I + 1 : q.I - q.h;
+      v.push_back({a.at(q.I, K0), vec(z, K0), vec(z, q.I), W, q.h * B, 1});
+    }
+    return launch(v);
+  };
+  const int top = mid, bottom = mid == nb ? 0 : nb - mid - kb;
+  auto down = [&](int t) { return Step{t, 1, std::min(kb, nb - 1 - t)}; };
+  auto up = [&](int t) { return Step{nb - 1 - t, -1, kb}; };
+  // both ends together; where their rows meet (the last kb steps) the upward
+  // end goes after the downward one
+  for (int t = 0; t < std::max(top, bottom - kb); ++t) {
+    std::vector<Step> st;
+    if (t < top) st.push_back(down(t));
+    if (t < bottom - kb) st.push_back(up(t));
+    if ((rc = forward(st))) return rc;
+  }
+  for (int t = std::max(bottom - kb, 0); t < bottom; ++t)
+    if ((rc = forward({up(t)}))) return rc;
+  if (bottom > 0) {
+    for (int I = mid; I < mid + kb; ++I)
+      if ((rc = forward({Step{I, 1, mid + kb - 1 - I}}))) return rc;
+    for (int I = mid + kb - 1; I >= mid; --I)
+      if ((rc = backward({Step{I, 1, mid + kb - 1 - I}}))) return rc;
+  }
+  for (int t = std::max(top, bottom) - 1; t >= 0; --t) {
+    std::vector<Step> st;
+    if (t < top) st.push_back(down(t));
+    if (t < bottom) st.push_back(up(t));
+    if ((rc = backward(st))) return rc;
+    if (t == 0 && nfar > 0) {
+      const int nf = std::min(nfar, nb - 1 - kb);
+      if (nf > 0 && (rc = launch({{F, vec(z, kb + 1), vec(z, 0), (long)nfar * B, nf * B, 1}}))) return rc;
+    }
+  }
   return 0;
 }
 
@@ -1785,7 +2057,15 @@ int bca_gemm_f64_sub(void* stream, int M, int N, int K, const double* A, long ld
 int bca_csr_spmv(void* stream, long n, const int* indptr, const int* indices, const double* data, const double* x,
                  double* y) {
   if (!indptr || !indices || !data || !x || !y) return fail(-1, "null argument");
-  k_csr_spmv<<<grid1(n, 256), 256, 0, (hipStream_t)stream>>>(n, indptr, indices, data, x, y);
+  k_csr_spmv<<<grid1(n, 4), 256, 0, (hipStream_t)stream>>>(n, indptr, indices, data, x, nullptr, y);
+  BCA_LAUNCHED();
+  return 0;
+}
+
+int bca_csr_residual(void* stream, long n, const int* indptr, const int* indices, const double* data, const double* x,
+                     const double* b, double* r) {
+  if (!indptr || !indices || !data || !x || !b || !r) return fail(-1, "null argument");
+  k_csr_spmv<<<grid1(n, 4), 256, 0, (hipStream_t)stream>>>(n, indptr, indices, data, x, b, r);
   BCA_LAUNCHED();
   return 0;
 }

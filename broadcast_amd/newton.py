@@ -23,14 +23,15 @@ by more than `growth`.
 Block-banded LU.  In the reference's unknown order (C-order ravel of
 (im, jm, 5), i outermost) the Jacobian couples i-lines at most 3 apart, so it
 is block banded with blocks of one i-line (5 jm unknowns).  The factorization
-is block Gaussian elimination: each diagonal block by LU with partial
-pivoting (rocSOLVER getrf through torch.linalg.lu_factor), the row blocks to
-its right by one solve with it, the band below updated by one GEMM per block
-row (rocBLAS); no fill leaves the band.  Storage is dense per block row,
+is block Gaussian elimination without pivoting across blocks, on the device by
+the library's own kernels from both ends of the band (bca_band_factor): each
+diagonal block is replaced by its inverse, the block rows by their products
+with it; no fill leaves the band.  Storage is dense per block row,
 R[K] = [A(K, K-kb) ... A(K, K+kb)], (nblocks, B, (2 kb + 1) B) doubles.
 An i-periodic mesh (the O-mesh) couples the first and last i-lines; it is
 solved with j outermost instead (blocks of one j-line), where the band is
-that of the radial stencil.
+that of the radial stencil.  Complex matrices, small pivots and CPU tensors
+take torch's pivoted LU of the diagonal blocks.
 """
 from __future__ import annotations
 
@@ -54,9 +55,9 @@ class BlockBandLU:
     block rows 1..kb), so the band stays 2 kb + 1 blocks wide: with kb = 3
     instead of 4, 9 instead of 16 Schur products per block step.
 
-    With look-ahead (device tensors), block step I updates the next diagonal
-    block first and factors it on a side stream while the remaining Schur
-    products of step I run on the current stream."""
+    With look-ahead (device tensors), the next diagonal block goes first and
+    the remaining products of a step run beside it on another stream; the
+    library's elimination then also works from both ends of the band at once."""
 
     def __init__(self, im, jm, outer="i", kb=None, group=1, lookahead=True, pivot=None, diag="inv"):
         self.t = dev.torch()
@@ -133,6 +134,10 @@ class BlockBandLU:
         if self.np_lu:
             self._bad = t.zeros(1, dtype=t.int32, device=dv)
             if self.np_factor(R, F):
+                # solve() corrects with the matrix: a copy, the caller's
+                # arrays may hold another one by then
+                if self.diag == "inv":
+                    self.csr, self.shift = (indptr.clone(), indices.clone(), data.clone()), shift
                 return self
             # a pivot came out too small: refactor with partial pivoting
             self.np_lu = False
@@ -189,14 +194,44 @@ class BlockBandLU:
         return self
 
     def np_factor(self, R, F):
-        """Block elimination with the project's unpivoted kernels for the
-        diagonal blocks: with diag="inv" each diagonal block is replaced by its
-        inverse (bca_inv_np) and the block row X = D^-1 A(I, J) is one GEMM;
-        with diag="lu" by its LU factors (bca_lu_np) and X comes from two
-        triangular solves.  The first block of X and the next diagonal
-        block's update go first; that block is then inverted/factored on a
-        side stream while the rest of the step's products run.  False if a
-        pivot was too small."""
+        """Block elimination with the project's unpivoted kernels: with
+        diag="inv" the whole elimination is bca_band_factor (each diagonal
+        block replaced by its inverse, from both ends of the band); with
+        diag="lu" each diagonal block is replaced by its LU factors
+        (bca_lu_np), the next one's on a side stream beside the rest of the
+        step's products.  False if a pivot was too small."""
+        self._bad.zero_()
+        (self._factor_band if self.diag == "inv" else self._factor_lu)(R, F)
+        return int(self._bad.item()) == 0
+
+    def _factor_band(self, R, F):
+        import ctypes as C
+        from . import _lib
+
+        t = self.t
+        nb, B, kb = self.nb, self.B, self.kb
+        # both ends need rows of their own beside the kb rows they meet in,
+        # and the far blocks of block row 0 lie on its side
+        # (they meet with the downward end kb steps behind: the upward end's
+        # last kb steps come after it)
+        self.mid = nb // 2 - kb
+        if not self.lookahead or self.mid < kb + self.nfar + 1:
+            self.mid = nb
+        scratch = t.empty(2 * (1 + kb + self.nfar) * B * B, dtype=t.float64, device=R.device)
+        cur = t.cuda.current_stream()
+        # the caller's stream may share a hardware queue with one of these:
+        # it only waits for the two that do the work
+        side = [t.cuda.Stream() for _ in range(2)] if self.lookahead else [cur] * 2
+        streams = (C.c_void_p * 3)(*[s.cuda_stream for s in (cur, *side)])
+        rc = _lib.lib().bca_band_factor(streams, C.c_void_p(R.data_ptr()), C.c_void_p(F.data_ptr()) if self.nfar else None,
+                                        nb, B, kb, self.nfar, self.mid, C.c_void_p(scratch.data_ptr()), 1e-14,
+                                        C.c_void_p(self._bad.data_ptr()))
+        # the scratch and the matrix are in use on the other streams until the
+        # caller's stream gets past them
+        t.cuda.synchronize(R.device)
+        _lib.check(rc, "bca_band_factor")
+
+    def _factor_lu(self, R, F):
         import ctypes as C
         from . import _lib
 
@@ -206,31 +241,20 @@ class BlockBandLU:
         W = R.shape[2]
         cur = t.cuda.current_stream()
         side = t.cuda.Stream() if self.lookahead else cur
-        self._bad.zero_()
-        inv = self.diag == "inv"
         # scratch of each stream the diagonal blocks are processed on
-        wsize = B * B if inv else 32 * 32
-        work = [t.empty(wsize, dtype=t.float64, device=R.device) for _ in range(2 if self.lookahead else 1)]
+        work = [t.empty(32 * 32, dtype=t.float64, device=R.device) for _ in range(2 if self.lookahead else 1)]
 
         def diag_np(I, stream):
             D = R[I, :, kb * B:(kb + 1) * B]
             wk = work[1 if (self.lookahead and stream is side) else 0]
-            sp = C.c_void_p(stream.cuda_stream)
-            if inv:
-                rc = L_.bca_inv_np(sp, C.c_void_p(D.data_ptr()), B, W, C.c_void_p(wk.data_ptr()), 1e-14,
-                                   C.c_void_p(self._bad.data_ptr()))
-            else:
-                rc = L_.bca_lu_np(sp, C.c_void_p(D.data_ptr()), B, W, 1e-14, C.c_void_p(self._bad.data_ptr()),
-                                  C.c_void_p(wk.data_ptr()))
-            _lib.check(rc, "bca_inv_np" if inv else "bca_lu_np")
+            rc = L_.bca_lu_np(C.c_void_p(stream.cuda_stream), C.c_void_p(D.data_ptr()), B, W, 1e-14,
+                              C.c_void_p(self._bad.data_ptr()), C.c_void_p(wk.data_ptr()))
+            _lib.check(rc, "bca_lu_np")
 
         def apply_inv(D, X):
             """X <- D^-1 X in place."""
-            if inv:
-                X.copy_(D @ X)
-            else:
-                X.copy_(t.linalg.solve_triangular(D, t.linalg.solve_triangular(D, X, upper=False,
-                                                                               unitriangular=True), upper=True))
+            X.copy_(t.linalg.solve_triangular(D, t.linalg.solve_triangular(D, X, upper=False, unitriangular=True),
+                                              upper=True))
 
         diag_np(0, cur)
         ready = None
@@ -273,7 +297,6 @@ class BlockBandLU:
                             R[K2, :, (kb + off) * B:(kb + off + 1) * B].sub_(L @ F[:, (f - 1) * B:f * B])
         if ready is not None:
             cur.wait_event(ready)
-        return int(self._bad.item()) == 0
 
     def _solve_diag(self, I, v):
         """D_I^-1 v for one block (v: (B,) or (B, k))."""
@@ -282,14 +305,25 @@ class BlockBandLU:
             return t.linalg.lu_solve(self.lu[I], self.piv[I], v.unsqueeze(1) if v.dim() == 1 else v).reshape(v.shape)
         kb, B = self.kb, self.B
         D = self.R[I, :, kb * B:(kb + 1) * B]
-        if self.diag == "inv":
-            return D @ v
         m = v.unsqueeze(1) if v.dim() == 1 else v
         y = t.linalg.solve_triangular(D, t.linalg.solve_triangular(D, m, upper=False, unitriangular=True), upper=True)
         return y.reshape(v.shape)
 
     def solve(self, b):
         """x with A x = b, b in the reference's unknown order."""
+        if self.np_lu and self.diag == "inv":
+            # one correction with the matrix itself belongs to the solve: the
+            # upward half of the elimination runs against the flow on a
+            # boundary layer, where (weakly relaxed) it loses some digits
+            x = self._apply(b)
+            r = csr_residual(self.csr, x, b.reshape(-1))
+            if self.shift is not None:
+                r += self.shift * x
+            return x + self._apply(r)
+        return self._apply(b)
+
+    def _apply(self, b):
+        """The factors applied to b once."""
         t = self.t
         B, kb, nb = self.B, self.kb, self.nb
         if self.outer == "i":
@@ -298,6 +332,9 @@ class BlockBandLU:
             y = b.reshape(self.im, self.jm, 5).permute(1, 0, 2).reshape(-1)
         y = t.cat((y, y.new_zeros(self.np - self.n))).reshape(nb, B)
         R = self.R
+        if self.np_lu and self.diag == "inv":
+            y = self._solve_band(y)
+            return self._unpermute(y)
         for I in range(nb):
             y[I] = self._solve_diag(I, y[I])
             for dd in range(1, min(kb, nb - 1 - I) + 1):
@@ -309,6 +346,21 @@ class BlockBandLU:
                 for f in range(1, self.nfar + 1):
                     if kb + f < nb:
                         y[0] -= self.F[:, (f - 1) * B:f * B] @ y[kb + f]
+        return self._unpermute(y)
+
+    def _solve_band(self, y):
+        """bca_band_solve; y is overwritten."""
+        import ctypes as C
+        from . import _lib
+
+        z = self.t.empty_like(y)
+        _lib.check(_lib.lib().bca_band_solve(
+            dev.current_stream_ptr(), C.c_void_p(self.R.data_ptr()),
+            C.c_void_p(self.F.data_ptr()) if self.nfar else None, self.nb, self.B, self.kb, self.nfar, self.mid,
+            C.c_void_p(y.data_ptr()), C.c_void_p(z.data_ptr())), "bca_band_solve")
+        return z
+
+    def _unpermute(self, y):
         y = y.reshape(-1)[:self.n]
         if self.outer == "i":
             return y
@@ -322,11 +374,12 @@ def csr_residual(csr, x, b):
 
     t = dev.torch()
     indptr, indices, data = csr
-    y = t.empty_like(b)
-    _lib.check(_lib.lib().bca_csr_spmv(dev.current_stream_ptr(), b.numel(), C.c_void_p(indptr.data_ptr()),
-                                       C.c_void_p(indices.data_ptr()), C.c_void_p(data.data_ptr()),
-                                       C.c_void_p(x.data_ptr()), C.c_void_p(y.data_ptr())), "bca_csr_spmv")
-    return b - y
+    r = t.empty_like(b)
+    _lib.check(_lib.lib().bca_csr_residual(dev.current_stream_ptr(), b.numel(), C.c_void_p(indptr.data_ptr()),
+                                           C.c_void_p(indices.data_ptr()), C.c_void_p(data.data_ptr()),
+                                           C.c_void_p(x.data_ptr()), C.c_void_p(b.data_ptr()),
+                                           C.c_void_p(r.data_ptr())), "bca_csr_residual")
+    return r
 
 
 def refine(lu, csr, b, x, rtol=1e-12, steps=3):

@@ -386,13 +386,30 @@ int bca_jacobian_colored_csr_refresh(bca_ctx *ctx, const double *w, bca_metrics 
  * multiplies its off-diagonal blocks and right-hand sides by it.  work:
  * device scratch of n x n doubles; *bad as for bca_lu_np.
  * bca_gemm_f64_sub: C -= A B, row-major, FP64 matrix cores.
- * bca_csr_spmv: y = A x for a CSR matrix (the residual of a refined solve). */
+ * bca_csr_spmv: y = A x for a CSR matrix; bca_csr_residual: r = b - A x (a
+ * refined solve's residual). */
 int bca_lu_np(void *hip_stream, double *A, int n, long ld, double tiny, int *bad, double *work);
 int bca_inv_np(void *hip_stream, double *A, int n, long ld, double *work, double tiny, int *bad);
+/* Block-banded elimination of nb block rows of B unknowns, kb blocks to either
+ * side: R holds row K as [A(K, K-kb) ... A(K, K+kb)] (B x (2 kb + 1) B,
+ * row-major, rows back to back), F (B x nfar B) the blocks kb+1 .. kb+nfar of
+ * block row 0.  Rows 0 .. mid-1 are eliminated downwards, nb-1 .. mid+kb
+ * upwards beside them, then the kb rows between (mid = nb: all downwards).
+ * In place: D_I^-1 on the diagonal, D_I^-1 A(I, J) for the blocks J a row
+ * still reaches, the others as given.  streams: the caller's (ordered before
+ * and after the work) and the two that do it; scratch: 2 (1 + kb +
+ * nfar) B^2 doubles, free again when the caller's stream gets there; *bad as
+ * for bca_lu_np.  bca_band_solve applies it: y (nb B, overwritten) to z. */
+int bca_band_factor(void *const hip_streams[3], double *R, double *F, int nb, int B, int kb, int nfar, int mid,
+                    double *scratch, double tiny, int *bad);
+int bca_band_solve(void *hip_stream, const double *R, const double *F, int nb, int B, int kb, int nfar, int mid,
+                   double *y, double *z);
 int bca_gemm_f64_sub(void *hip_stream, int M, int N, int K, const double *A, long lda, const double *B,
                      long ldb, double *C, long ldc);
 int bca_csr_spmv(void *hip_stream, long n, const int *indptr, const int *indices, const double *data,
                  const double *x, double *y);
+int bca_csr_residual(void *hip_stream, long n, const int *indptr, const int *indices, const double *data,
+                     const double *x, const double *b, double *r);
 
 /* ---- BF16 GEMM of the learned Newton guess ---------------------------------- */
 /* No reference counterpart (the reference has no learned part).  C (fp32,
