@@ -344,10 +344,10 @@ __host__ __device__ constexpr double euler_coef(int along) {
   }
 }
 
-// The face adjoint of one face for the offsets [O0, O1): J = false an
+// The face adjoint of one face: J = false an
 // i-face (compact viscous flux), true a centred j-face.  hb: the face's
 // adjoint hnb; out: out[(o * 5 + q) * nf + f].
-template <bool J, bool O4, int ROW, int O0, int O1>
+template <bool J, bool O4, int ROW>
 __device__ inline void face_reverse(const Mesh& m, const Phys& ph, const Metric& g, const double* w,
                                     const double* prim, const double* grad, int i, int j, const double hb[5],
                                     double* out, long nf, long f) {
@@ -407,7 +407,7 @@ __device__ inline void face_reverse(const Mesh& m, const Phys& ph, const Metric&
   const double cvm1 = 1.0 / ph.cv;
   const double betas = ph.muref * (ph.tref + ph.cs) / (sqrt(ph.tref) * ph.tref);
 
-  sfor<O0, O1>([&](auto O) {
+  sfor<0, NOFF>([&](auto O) {
     constexpr int o = decltype(O)::value;
     constexpr int SI = J ? joff_di(o) : ioff_di(o), SJ = J ? joff_dj(o) : ioff_dj(o);
     // the two extra offsets exist only on the faces the seeded passes store
@@ -501,31 +501,25 @@ __device__ inline void face_reverse(const Mesh& m, const Phys& ph, const Metric&
   });
 }
 
-// offsets per launch of the reverse kernels (the face-level part is
-// recomputed per launch)
-constexpr int REV_GROUP = 24;
-
-// One thread per face of rows [j0, j1], i = i0, i0 + istep, ...: J = false
-// i-faces (O4: rows j >= 3, the compact viscous flux; else rows 1, 2), J =
-// true j-faces (ROW 0: rows j >= 4, centred Euler flux; ROW 3, 2: the
-// off-centred rows 3 (compact viscous flux) and 2 (2nd-order)); offsets
-// [O0, O1) of the face's stencil.
-template <bool J, bool O4, int ROW, int O0 = 0, int O1 = NOFF>
+// One thread per face of rows [j0, j1]: J = false i-faces (O4: rows j >= 3, the
+// compact viscous flux; else rows 1, 2), J = true j-faces (ROW 0: rows j >= 4,
+// centred Euler flux; ROW 3, 2: the off-centred rows 3 (compact viscous flux)
+// and 2 (2nd-order)).
+template <bool J, bool O4, int ROW>
 __global__ void __launch_bounds__(256) k_face_reverse(Mesh m, Phys ph, Metric g, const double* __restrict__ w,
                                                       const double* __restrict__ prim,
                                                       const double* __restrict__ grad, double* __restrict__ out,
-                                                      const double* __restrict__ resb, int j0, int j1, int i0,
-                                                      int istep) {
+                                                      const double* __restrict__ resb, int j0, int j1) {
   int bx, by;
   xcd_block(bx, by);
-  const int i = i0 + (bx * (int)blockDim.x + (int)threadIdx.x) * istep;
+  const int i = 1 + bx * (int)blockDim.x + (int)threadIdx.x;
   const int j = j0 + by * blockDim.y + threadIdx.y;
   if (i > (J ? m.im : m.im + 1) || j > j1) return;
   const long nf = J ? (long)m.im * (m.jm + 1) : (long)(m.im + 1) * m.jm;
   const long f = J ? (i - 1) + (long)m.im * (j - 1) : (i - 1) + (long)(m.im + 1) * (j - 1);
   double hb[5];
   face_adjoint(m, resb, i, j, J ? 0 : 1, J ? 1 : 0, hb);
-  face_reverse<J, O4, ROW, O0, O1>(m, ph, g, w, prim, grad, i, j, hb, out, nf, f);
+  face_reverse<J, O4, ROW>(m, ph, g, w, prim, grad, i, j, hb, out, nf, f);
 }
 
 }  // namespace bca

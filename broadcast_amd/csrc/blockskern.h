@@ -1,10 +1,10 @@
-// Face-local Jacobian block kernels: B(face, o) = d hn(face) / d w(face + o)
-// for the 24 stencil offsets o of the face family, by compile-time sparse
-// forward mode (SeededAcc).  Two outputs of the same passes:
+// Stencil offsets of the face families, and the kernel of the wall faces'
+// blocks B(face, o) = d hn(face) / d w(face + o), by compile-time sparse
+// forward mode (SeededAcc; the other faces: fwdface.h).  Two outputs:
 //   MODE_BLOCKS  the blocks themselves (phase 1 of the colored assembly);
 //   MODE_VJP     hnb(face)^T B(face, o), 5 values per offset, with hnb the
 //                face adjoint of residub (the VJP, gathered per cell later).
-// Templates only: each variant is instantiated in its own object (blocks.hip).
+// Templates only, instantiated in objects of their own (blocks.hip).
 #pragma once
 #include "faces.h"
 
@@ -119,84 +119,30 @@ __device__ inline void face_adjoint(const Mesh& m, const double* resb, int i, in
   }
 }
 
-// The 24 seeded passes of an interior face are split into groups of
-// OFF_GROUP offsets, one kernel instantiation (and launch) per group: one
-// thread evaluating all 24 lets the compiler interleave them far beyond the
-// register file (hundreds of bytes of spills per lane).  Offsets [O0, O1) per
-// instantiation.  At 512 x 384, groups of 4 (one of six spills) take
-// 0.66 + 0.52 ms for the i- and j-face blocks, groups of 2 0.62 + 0.48 ms and
-// single offsets (no spills, 24 launches) 0.52 + 0.43 ms.
-constexpr int OFF_GROUP = 1;
-
-// i-faces (i, j), i = i0, i0 + istep, ... <= im+1, rows j in [j0, j1]; O4 selects the
-// compact viscous flux (rows j >= 3) over the 2nd-order one (rows 1, 2).
-// The two extra offsets (3, 0), (-4, 0) only exist for the faces i = 1 and
-// i = im+1 (extrapolated ghost gradients); elsewhere nothing is stored for
-// them and the assembly does not read them.
-template <bool O4, int MODE, int O0 = 0, int O1 = NOFF>
-__global__ void __launch_bounds__(256) k_iface_blocks(Mesh m, Phys ph, Metric g, const double* __restrict__ w,
-                                                      const double* __restrict__ prim,
-                                                      const double* __restrict__ grad,
-                                                      double* __restrict__ out, const double* __restrict__ resb,
-                                                      int j0, int j1, int i0, int istep) {
-  int bx, by;
-  xcd_block(bx, by);
-  const int i = i0 + (bx * (int)blockDim.x + (int)threadIdx.x) * istep;
-  const int j = j0 + by * blockDim.y + threadIdx.y;
-  if (i > m.im + 1 || j > j1) return;
-  const long nf = (long)(m.im + 1) * m.jm;
-  FaceSink<MODE> sink{out, nf, (i - 1) + (long)(m.im + 1) * (j - 1), {}};
-  if constexpr (MODE == MODE_VJP) face_adjoint(m, resb, i, j, 1, 0, sink.hb);
-  sfor<O0, O1>([&](auto O) {
-    constexpr int o = decltype(O)::value;
-    constexpr int SI = ioff_di(o), SJ = ioff_dj(o);
-    if (o == 22 && i != 1) return;
-    if (o == 23 && i != m.im + 1) return;
-    auto a = seeded<SI, SJ>(m, ph, g, w, prim, grad, i, j);
-    Dual<5> hn[5];
-    iface<O4>(a, hn);
-    sink.put(o, hn);
-  });
-}
-
-// j-faces (i, j), i = i0, i0 + istep, ... <= im, one row variant per launch: ROW 0 = centred
-// (rows j >= 4), 3, 2 = off-centred near-wall rows, 1 = the wall face.
-// Extra offsets: (0, 3) only for row 2, (0, -4) only for row jm+1; the wall
-// face depends on (0, 0) and (0, 1) only.
-template <int ROW, int MODE, int O0 = 0, int O1 = NOFF>
-__global__ void __launch_bounds__(256) k_jface_blocks(Mesh m, Phys ph, Metric g, const double* __restrict__ w,
-                                                      const double* __restrict__ prim,
-                                                      const double* __restrict__ grad,
-                                                      double* __restrict__ out, const double* __restrict__ resb,
-                                                      int j0, int j1, int i0, int istep) {
-  int bx, by;
-  xcd_block(bx, by);
-  const int i = i0 + (bx * (int)blockDim.x + (int)threadIdx.x) * istep;
-  const int j = j0 + by * blockDim.y + threadIdx.y;
+// Wall faces (i, 1) (adiabatic no-slip, fluxwall.F): they depend on the cells
+// (0, 0) and (0, 1) only; the other blocks are stored as explicit zeros where
+// the assembly may look for them.
+template <int MODE>
+__global__ void __launch_bounds__(256) k_jface_wall_blocks(Mesh m, Phys ph, Metric g, const double* __restrict__ w,
+                                                           const double* __restrict__ prim,
+                                                           const double* __restrict__ grad,
+                                                           double* __restrict__ out,
+                                                           const double* __restrict__ resb, int j0, int j1) {
+  const int i = 1 + blockIdx.x * (int)blockDim.x + (int)threadIdx.x;
+  const int j = j0 + blockIdx.y * blockDim.y + threadIdx.y;
   if (i > m.im || j > j1) return;
   const long nf = (long)m.im * (m.jm + 1);
   FaceSink<MODE> sink{out, nf, (i - 1) + (long)m.im * (j - 1), {}};
   if constexpr (MODE == MODE_VJP) face_adjoint(m, resb, i, j, 0, 1, sink.hb);
-  sfor<O0, O1>([&](auto O) {
+  sfor<0, 22>([&](auto O) {
     constexpr int o = decltype(O)::value;
     constexpr int SI = joff_di(o), SJ = joff_dj(o);
-    if constexpr (o == 22 && ROW != 2) return;
-    else if constexpr (ROW == 1 && !(SI == 0 && (SJ == 0 || SJ == 1))) {
-      // the wall face does not depend on this cell: store an explicit zero
-      // block where the assembly may look for one
-      Dual<5> z[5];
-      sink.put(o, z);
-      return;
-    } else {
-      if (o == 23 && !(ROW == 0 && j == m.jm + 1)) return;
+    Dual<5> hn[5];
+    if constexpr (SI == 0 && (SJ == 0 || SJ == 1)) {
       auto a = seeded<SI, SJ>(m, ph, g, w, prim, grad, i, j);
-      Dual<5> hn[5];
-      if constexpr (ROW == 0) jface<0, true>(a, hn);
-      else if constexpr (ROW == 3) jface<3, true>(a, hn);
-      else if constexpr (ROW == 2) jface<2, false>(a, hn);
-      else jface_wall(a, hn);
-      sink.put(o, hn);
+      jface_wall(a, hn);
     }
+    sink.put(o, hn);
   });
 }
 

@@ -95,6 +95,7 @@ struct bca_ctx {
   Work<Dual<1>> w1;
   double* norm_part = nullptr;
   double* norm_out = nullptr;
+  double* cellx = nullptr;  // 1 / rho and d mu / d T of every cell
   double* blki = nullptr;   // face-local Jacobian blocks, i-faces, one plane per offset
   double* blkj = nullptr;   // j-faces
   double* ghostT = nullptr; // ghost tangents per zone and color
@@ -482,7 +483,7 @@ int bca_ctx_destroy(bca_ctx* c) {
   free_work(c->w1);
   if (c->norm_part) (void)hipFree(c->norm_part);
   if (c->norm_out) (void)hipFree(c->norm_out);
-  for (double* p : {c->blki, c->blkj, c->ghostT, c->vjpi, c->vjpj})
+  for (double* p : {c->cellx, c->blki, c->blkj, c->ghostT, c->vjpi, c->vjpj})
     if (p) (void)hipFree(p);
   if (c->wcol) (void)hipFree(c->wcol);
   if (c->ghostnz) (void)hipFree(c->ghostnz);
@@ -979,6 +980,7 @@ int jacobian_phase1(bca_ctx* c, const double* w, bca_metrics g, const bca_phys* 
   if ((rc = check_ops_frame(m, ops, nops, g.nx, g.ny))) return rc;
   if ((rc = ensure_work(c, c->w0, false))) return rc;
   const long nfi = (long)(m.im + 1) * m.jm, nfj = (long)m.im * (m.jm + 1);
+  if ((rc = alloc_planes(c, &c->cellx, NCELLX * m.ncell))) return rc;
   if ((rc = alloc_planes(c, &c->blki, (long)NOFF * 25 * nfi))) return rc;
   if ((rc = alloc_planes(c, &c->blkj, (long)NOFF * 25 * nfj))) return rc;
   const Metric gm = to_metric(g);
@@ -992,21 +994,23 @@ int jacobian_phase1(bca_ctx* c, const double* w, bca_metrics g, const bca_phys* 
   BCA_LAUNCHED();
   k_grad_ghost<double><<<grid1(2 * m.im + m.jm, 256), 256, 0, s>>>(m, c->w0.grad);
   BCA_LAUNCHED();
+  k_cellx<<<grid1(m.ncell, 256), 256, 0, s>>>(m, ph, w, c->w0.prim, c->cellx);
+  BCA_LAUNCHED();
   // phase 1: face-local blocks (independent of the zones).  The edge rows
   // (i-face rows 1-2, j-face rows 1-3) write face rows the interior launches
   // do not, so they run on the side streams meanwhile, and so do the ghost
   // tangents.
   hipStream_t es[3];
   if ((rc = edge_fork(c, es))) return rc;
-  BlockArgs ae{m, ph, gm, w, c->w0.prim, c->w0.grad, c->blki, nullptr, 1, 2};
+  BlockArgs ae{m, ph, gm, w, c->w0.prim, c->w0.grad, c->blki, nullptr, 1, 2, c->cellx};
   launch_iface_blocks_o2(grid2(m.im + 1, 2, b), b, es[0], ae);
   ae.out = c->blkj;
-  ae.j0 = ae.j1 = 3;
-  launch_jface_blocks_r3(grid2(m.im, 1, b), b, es[1], ae);
   ae.j0 = ae.j1 = 2;
-  launch_jface_blocks_r2(grid2(m.im, 1, b), b, es[2], ae);
+  launch_jface_blocks_r2(grid2(m.im, 1, b), b, es[0], ae);
+  ae.j0 = ae.j1 = 3;
+  launch_jface_blocks_r3(grid2(m.im, 1, b), b, es[2], ae);
   ae.j0 = ae.j1 = 1;
-  launch_jface_blocks_wall(grid2(m.im, 1, b), b, es[0], ae);
+  launch_jface_blocks_wall(grid2(m.im, 1, b), b, es[2], ae);
   BCA_LAUNCHED();
   // the ghost tangents read w only and write their own planes: on side
   // stream 1 too (its launches go to c->stream, pointed there meanwhile)
@@ -1018,21 +1022,16 @@ int jacobian_phase1(bca_ctx* c, const double* w, bca_metrics g, const bca_phys* 
     (void)edge_join(c, es);
     return rc;
   }
-  BlockArgs ai{m, ph, gm, w, c->w0.prim, c->w0.grad, c->blki, nullptr, 3, m.jm};
+  BlockArgs ai{m, ph, gm, w, c->w0.prim, c->w0.grad, c->blki, nullptr, 3, m.jm, c->cellx};
   const dim3 bt = c->tune_blocks;
   {
-    // every second offset on side stream 0 (free once its edge rows are
-    // done); the timers cover the offsets on c->stream
     Timed t(c, "k_iface_blocks");
-    launch_iface_blocks_o4(grid2(m.im + 1, m.jm - 2, bt), bt, s, ai, es[0] == s ? nullptr : es[0]);
+    launch_iface_blocks_o4(grid2(m.im + 1, m.jm - 2, bt), bt, s, ai);
   }
-  BlockArgs aj{m, ph, gm, w, c->w0.prim, c->w0.grad, c->blkj, nullptr, 4, m.jm + 1};
+  BlockArgs aj{m, ph, gm, w, c->w0.prim, c->w0.grad, c->blkj, nullptr, 4, m.jm + 1, c->cellx};
   {
-    // likewise every second j-face offset on side stream 2: the one-offset
-    // launches (tens of microseconds each) leave most of the chip idle
-    // alone, so four of them run side by side
     Timed t(c, "k_jface_blocks");
-    launch_jface_blocks_c(grid2(m.im, m.jm - 2, bt), bt, s, aj, es[2] == s ? nullptr : es[2]);
+    launch_jface_blocks_c(grid2(m.im, m.jm - 2, bt), bt, s, aj);
   }
   BCA_LAUNCHED();
   return edge_join(c, es);
@@ -1125,18 +1124,18 @@ int bca_vjp_dnc5(bca_ctx* c, double* residub, double* wb, const double* w, bca_m
   // queue with c->stream does not hold them back
   hipStream_t es[3];
   if ((rc = edge_fork(c, es))) return rc;
-  BlockArgs ai{m, ph, gm, w, c->w0.prim, c->w0.grad, c->vjpi, residub, 3, m.jm};
+  BlockArgs ai{m, ph, gm, w, c->w0.prim, c->w0.grad, c->vjpi, residub, 3, m.jm, nullptr};
   {
     Timed t(c, "k_iface_vjp");
     launch_iface_vjp_rev(grid2(m.im + 1, m.jm - 2, b), b, s, ai);
   }
-  BlockArgs aj{m, ph, gm, w, c->w0.prim, c->w0.grad, c->vjpj, residub, 4, m.jm + 1};
+  BlockArgs aj{m, ph, gm, w, c->w0.prim, c->w0.grad, c->vjpj, residub, 4, m.jm + 1, nullptr};
   {
     Timed t(c, "k_jface_vjp");
     launch_jface_vjp_rev(grid2(m.im, m.jm - 2, b), b, s, aj);
   }
   BCA_LAUNCHED();
-  BlockArgs ae{m, ph, gm, w, c->w0.prim, c->w0.grad, c->vjpi, residub, 1, 2};
+  BlockArgs ae{m, ph, gm, w, c->w0.prim, c->w0.grad, c->vjpi, residub, 1, 2, nullptr};
   launch_iface_vjp_rev_o2(grid2(m.im + 1, 2, b), b, es[0], ae);
   ae.out = c->vjpj;
   ae.j0 = ae.j1 = 3;
@@ -2170,8 +2169,8 @@ int bca_autotune(bca_ctx* c, const double* w, bca_metrics g, const bca_phys* p, 
   // interior face blocks (both families share the shape)
   best = 1e30f;
   for (const dim3& b : shapes) {
-    BlockArgs ai{m, ph, gm, w, c->w0.prim, c->w0.grad, c->blki, nullptr, 3, m.jm};
-    BlockArgs aj{m, ph, gm, w, c->w0.prim, c->w0.grad, c->blkj, nullptr, 4, m.jm + 1};
+    BlockArgs ai{m, ph, gm, w, c->w0.prim, c->w0.grad, c->blki, nullptr, 3, m.jm, c->cellx};
+    BlockArgs aj{m, ph, gm, w, c->w0.prim, c->w0.grad, c->blkj, nullptr, 4, m.jm + 1, c->cellx};
     if ((rc = time_launch(c, reps, [&] {
            launch_iface_blocks_o4(grid2(m.im + 1, m.jm - 2, b), b, s, ai);
            launch_jface_blocks_c(grid2(m.im, m.jm - 2, b), b, s, aj);

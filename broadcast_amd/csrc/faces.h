@@ -4,14 +4,11 @@
 //
 //   PlainAcc<double>    the residual                (every value a double)
 //   PlainAcc<Dual<N>>   dense tangents (JVP)        (every value a Dual<N>)
-//   SeededAcc<SI, SJ>   face-local Jacobian block   (only the cell at offset
+//   SeededAcc<SI, SJ>   block of the wall face      (only the cell at offset
 //                       d hn(face) / d w(cell)       (SI, SJ) carries a 5-way
 //                                                     tangent; all else double)
 //
-// With SeededAcc, C++ typing carries the tangent exactly along the data flow
-// of the one seeded cell: a sum of six cell values becomes a Dual only at the
-// seeded term and everything that does not depend on it stays plain FP64, so
-// the 24 blocks of a face cost a fraction of 24 dense 5-way tangents.
+// (the blocks of the other faces: fwdface.h).
 //
 // Formulas: srcfv/rhs/flux_num_dnc5.F90 (expanded srcfv/prepro/flux_num_dnc5.f90)
 //   Euler        euler_o6_i.F / nearbndfluxes{3,5}demi_7p.F (coefnearbnd_7p.F)
@@ -95,45 +92,12 @@ struct PlainAcc : AccBase {
   template <int DI, int DJ> __device__ T G(int k) const { return grad[cidx(m, i + DI, j + DJ) + (long)k * m.ncell]; }
 };
 
-// 4th-order gradient (gradop_5pi/j.F + gradient.F) at the cell at offset
-// (GI, GJ), computed from the accessor's primitives so that it is typed by
-// whether the seeded cell is in its stencil.  k: G_UX, G_UY, G_VX, G_VY.
-template <int GI, int GJ, class A>
-__device__ inline auto grad_direct(const A& a, int k) {
-  const int q = (k < 2) ? P_U : P_V;
-  auto di = Coef::b1 * (a.template P<GI + 1, GJ>(q) - a.template P<GI - 1, GJ>(q)) +
-            Coef::b2 * (a.template P<GI + 2, GJ>(q) - a.template P<GI - 2, GJ>(q));
-  auto dj = Coef::b1 * (a.template P<GI, GJ + 1>(q) - a.template P<GI, GJ - 1>(q)) +
-            Coef::b2 * (a.template P<GI, GJ + 2>(q) - a.template P<GI, GJ - 2>(q));
-  const double volm1 = 1.0 / a.VOL(GI, GJ);
-  const bool xd = (k == G_UX || k == G_VX);
-  const double m1 = xd ? 0.5 * (a.NX(GI, GJ, 0) + a.NX(GI + 1, GJ, 0)) * volm1
-                       : 0.5 * (a.NY(GI, GJ, 0) + a.NY(GI + 1, GJ, 0)) * volm1;
-  const double m2 = xd ? 0.5 * (a.NX(GI, GJ, 1) + a.NX(GI, GJ + 1, 1)) * volm1
-                       : 0.5 * (a.NY(GI, GJ, 1) + a.NY(GI, GJ + 1, 1)) * volm1;
-  return m1 * di + m2 * dj;
-}
-
-__host__ __device__ constexpr bool in_grad_stencil(int dx, int dy) {
-  return (dy == 0 && (dx == 1 || dx == -1 || dx == 2 || dx == -2)) ||
-         (dx == 0 && (dy == 1 || dy == -1 || dy == 2 || dy == -2));
-}
-// can the gradient at offset (GI, GJ) -- directly, or through the one-layer
-// ghost extrapolation 2 g(a) - g(b) of gradveloingh.F -- depend on (SI, SJ)?
-__host__ __device__ constexpr bool grad_reach(int SI, int SJ, int GI, int GJ) {
-  return in_grad_stencil(SI - GI, SJ - GJ) || in_grad_stencil(SI - GI - 1, SJ - GJ) ||
-         in_grad_stencil(SI - GI - 2, SJ - GJ) || in_grad_stencil(SI - GI + 1, SJ - GJ) ||
-         in_grad_stencil(SI - GI + 2, SJ - GJ) || in_grad_stencil(SI - GI, SJ - GJ + 1) ||
-         in_grad_stencil(SI - GI, SJ - GJ + 2);
-}
-
 // Unit 5-way tangent on the cell at offset (SI, SJ) (the 5 conservative
 // variables of that cell), FP64 everywhere else.
 template <int SI, int SJ>
 struct SeededAcc : AccBase {
   using Out = Dual<5>;
   template <int DI, int DJ> using CT = std::conditional_t<(DI == SI && DJ == SJ), Dual<5>, double>;
-  template <int DI, int DJ> using GT = std::conditional_t<grad_reach(SI, SJ, DI, DJ), Dual<5>, double>;
   const double* w;
   const double* prim;
   const double* grad;
@@ -156,18 +120,6 @@ struct SeededAcc : AccBase {
   template <int DI, int DJ> __device__ CT<DI, DJ> P(int k) const {
     if constexpr (DI == SI && DJ == SJ) return sp[k];
     else return prim[cidx(m, i + DI, j + DJ) + (long)k * m.ncell];
-  }
-  template <int DI, int DJ> __device__ GT<DI, DJ> G(int k) const {
-    using R = GT<DI, DJ>;
-    if constexpr (!grad_reach(SI, SJ, DI, DJ)) {
-      return grad[cidx(m, i + DI, j + DJ) + (long)k * m.ncell];
-    } else {
-      const int gi = i + DI, gj = j + DJ;
-      if (gi == 0) return R(2.0 * grad_direct<DI + 1, DJ>(*this, k) - grad_direct<DI + 2, DJ>(*this, k));
-      if (gi == m.im + 1) return R(2.0 * grad_direct<DI - 1, DJ>(*this, k) - grad_direct<DI - 2, DJ>(*this, k));
-      if (gj == m.jm + 1) return R(2.0 * grad_direct<DI, DJ - 1>(*this, k) - grad_direct<DI, DJ - 2>(*this, k));
-      return R(grad_direct<DI, DJ>(*this, k));
-    }
   }
 };
 

@@ -24,10 +24,24 @@
 // the sum over its active inputs), so the COO values agree to rounding.
 #pragma once
 #include "bcs.h"
+#include "blocks.h"
 #include "blockskern.h"
 #include "misc.h"
 
 namespace bca {
+
+// 1 / rho and d mu / d T of every cell, for the blocks' d prim / d w.
+__global__ void __launch_bounds__(256) k_cellx(Mesh m, Phys ph, const double* __restrict__ w,
+                                               const double* __restrict__ prim, double* __restrict__ x) {
+  const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= m.ncell) return;
+  const double betas = ph.muref * (ph.tref + ph.cs) / (sqrt(ph.tref) * ph.tref);
+  const double t = prim[c + P_T * m.ncell];
+  // mu = (betas / (t + S)) sqrt(t) t
+  const double inv = 1.0 / (t + ph.s_suth);
+  x[c + X_RM * m.ncell] = 1.0 / w[c];
+  x[c + X_DMU * m.ncell] = (betas * inv) * sqrt(t) * (1.5 - t * inv);
+}
 
 // Seed zones in i.  One zone spanning the mesh is the reference's plain
 // coloring (testvector + computejacobianfromjv[_relaxed][_withjn]); two zones
