@@ -99,6 +99,7 @@ _SIGS = {
     "bca_gemm_bf16": [_dp, C.c_int, C.c_int, C.c_int, _dp, C.c_long, C.c_long, _dp, C.c_long, C.c_long, _dp,
                       C.c_long, C.c_long, C.c_int, C.c_int],
     "bca_lu_np": [_dp, _dp, C.c_int, C.c_long, C.c_double, _dp, _dp],
+    "bca_bc_sequence": [_dp, _dp, _dp, C.POINTER(BcOp), C.c_int, _dp, _dp],
     "bca_band_factor": [C.POINTER(C.c_void_p), _dp, _dp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _dp, C.c_double,
                         _dp],
     "bca_band_solve": [_dp, _dp, _dp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _dp, _dp],

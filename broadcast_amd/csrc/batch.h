@@ -87,18 +87,19 @@ __device__ inline void batch_pack(const BatchItem<T>& it, long c) {
 template <class T>
 __device__ inline void batch_bc(const BatchItem<T>& it, const BatchBc& op, int t) {
   const Mesh& m = it.m;
+  const StateView<T> w(m, it.ws);
   switch (op.kind) {
     case 0:  // inlet
-      bc_inlet_line(m, it.ws, op.loc, op.box, op.data, op.lm, it.g.nx, it.g.ny, op.gam, t + 1);
+      bc_inlet_line(w, op.loc, op.box, op.data, op.lm, it.g.nx, it.g.ny, op.gam, t + 1);
       break;
     case 1:  // no reflexion
-      bc_noref_line(m, it.ws, op.data, op.lm, op.loc, op.box, it.g.nx, it.g.ny, op.gam, t + 1);
+      bc_noref_line(w, op.data, op.lm, op.loc, op.box, it.g.nx, it.g.ny, op.gam, t + 1);
       break;
     case 2:
-      bc_extrap2_line(m, it.ws, op.loc, op.box, 5, t + 1);
+      bc_extrap2_line(w, op.loc, op.box, 5, t + 1);
       break;
     case 3:
-      bc_wall_line(m, it.ws, op.loc, op.box, op.gam, t + 1);
+      bc_wall_line(w, op.loc, op.box, op.gam, t + 1);
       break;
     default:
       join_cell(m, it.ws, op.box, op.box2, op.tr0, op.tr1, 5, m.ni, m.ncell, t);

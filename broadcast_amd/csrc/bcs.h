@@ -72,25 +72,47 @@ constexpr int BC_FRAME = 7;
 // the boundary conditions touch).
 template <class T, bool FR = false>
 struct StateView {
+  using Scalar = T;
   Mesh m;
   T* w;
   long plane;
-  __device__ StateView(const Mesh& mm, T* ww) : m(mm), w(ww), plane(FR ? frame_count(mm, BC_FRAME) : mm.ncell) {}
-  __device__ T& operator()(int i, int j, int e) const {
+  __host__ __device__ StateView(const Mesh& mm, T* ww) : m(mm), w(ww), plane(FR ? frame_count(mm, BC_FRAME) : mm.ncell) {}
+  __device__ long at(int i, int j, int e) const {
     const long c = FR ? frame_index(m, BC_FRAME, i + m.gh - 1, j + m.gh - 1) : cidx(m, i, j);
-    return w[c + (long)e * plane];
+    return c + (long)e * plane;
+  }
+  __device__ T operator()(int i, int j, int e) const { return w[at(i, j, e)]; }
+  __device__ void put(int i, int j, int e, const T& x) const { w[at(i, j, e)] = x; }
+};
+// A state and its tangent in their two arrays, as Dual<1>.
+struct PairView {
+  using Scalar = Dual<1>;
+  Mesh m;
+  double* v;
+  double* d;
+  __device__ Dual<1> operator()(int i, int j, int e) const {
+    const long c = cidx(m, i, j) + (long)e * m.ncell;
+    Dual<1> x(v[c]);
+    x.d[0] = d[c];
+    return x;
+  }
+  __device__ void put(int i, int j, int e, const Dual<1>& x) const {
+    const long c = cidx(m, i, j) + (long)e * m.ncell;
+    v[c] = x.v;
+    d[c] = x.d[0];
   }
 };
 
 // Characteristic sub/supersonic inflow.  Kept quirks of the reference:
 // the Roe-state pressure lacks the 1/2 (:49), velo2 uses ww unsquared (:69),
 // the ghost spanwise momentum is field(j, de, 4) (:160).
-template <class T, bool FR = false>
-__device__ inline void bc_inlet_line(const Mesh& m, T* __restrict__ wp, int loc, Box b,
+template <class V>
+__device__ inline void bc_inlet_line(const V& w, int loc, Box b,
                                      const double* __restrict__ field, int lm, const double* __restrict__ nxp,
                                      const double* __restrict__ nyp, double gam, int l) {
+  using T = typename V::Scalar;
+  const Mesh& m = w.m;
   const Side s = decode_side(loc, b.imin, b.jmin, b.imax, b.jmax);
-  StateView<T, FR> w{m, wp};
   auto F = [&](int a, int d, int e) { return field[(a - 1) + (long)lm * ((d - 1) + (long)m.gh * e)]; };
   const int i = b.imin + (l - 1) * s.j0 * s.j0;
   const int j = b.jmin + (l - 1) * s.i0 * s.i0;
@@ -126,27 +148,33 @@ __device__ inline void bc_inlet_line(const Mesh& m, T* __restrict__ wp, int loc,
     e0 = 0.5 + copysign(0.5, -rvn);
     ep = 0.5 + copysign(0.5, -rc - rvn);
   }
+  // inner state s: the layer before (kept in registers: a layer stored and
+  // read back costs its thread a round trip to memory)
+  T in[5];
+#pragma unroll
+  for (int e = 0; e < 5; ++e) in[e] = w(i, j, e);
   for (int de = 1; de <= m.gh; ++de) {
     const int ig = i - de * s.i0, jg = j - de * s.j0;
+    if (!sub) {
 #pragma unroll
-    for (int e = 0; e < 5; ++e) w(ig, jg, e) = T(F(l, de, e));
-    if (!sub) continue;
-    const int is = i - (de - 1) * s.i0, js = j - (de - 1) * s.j0;
-    // outer state d (the prescribed profile), inner state s (previous layer)
-    T rd = w(ig, jg, 0);
-    T rdm1 = 1.0 / rd;
-    T ud = w(ig, jg, 1) * rdm1, vd = w(ig, jg, 2) * rdm1, zd = w(ig, jg, 3) * rdm1;
-    T pd = g1 * (w(ig, jg, 4) - rd * 0.5 * (ud * ud + vd * vd + zd * zd));
-    T vnd = ud * nxn + vd * nyn;
-    T utd = ud - vnd * nxn, vtd = vd - vnd * nyn;
-    T hd = (w(ig, jg, 4) + pd) * rdm1;
-    T rs = w(is, js, 0);
+      for (int e = 0; e < 5; ++e) w.put(ig, jg, e, T(F(l, de, e)));
+      continue;
+    }
+    // outer state d: the prescribed profile
+    const double rd = F(l, de, 0);
+    const double rdm1 = 1.0 / rd;
+    const double ud = F(l, de, 1) * rdm1, vd = F(l, de, 2) * rdm1, zd = F(l, de, 3) * rdm1;
+    const double pd = g1 * (F(l, de, 4) - rd * 0.5 * (ud * ud + vd * vd + zd * zd));
+    const double vnd = ud * nxn + vd * nyn;
+    const double utd = ud - vnd * nxn, vtd = vd - vnd * nyn;
+    const double hd = (F(l, de, 4) + pd) * rdm1;
+    T rs = in[0];
     T rsm1 = 1.0 / rs;
-    T us = w(is, js, 1) * rsm1, vs = w(is, js, 2) * rsm1, zs = w(is, js, 3) * rsm1;
-    T ps = g1 * (w(is, js, 4) - rs * 0.5 * (us * us + vs * vs + zs * zs));
+    T us = in[1] * rsm1, vs = in[2] * rsm1, zs = in[3] * rsm1;
+    T ps = g1 * (in[4] - rs * 0.5 * (us * us + vs * vs + zs * zs));
     T vns = us * nxn + vs * nyn;
     T uts = us - vns * nxn, vts = vs - vns * nyn;
-    T hs = (w(is, js, 4) + ps) * rsm1;
+    T hs = (in[4] + ps) * rsm1;
     T sr2 = dsqrt(rs * rdm1);
     T rr2 = dsqrt(rs * rd);
     T wg2 = 1.0 / (sr2 + 1.0);
@@ -168,11 +196,10 @@ __device__ inline void bc_inlet_line(const Mesh& m, T* __restrict__ wp, int loc,
     T rou = ro * (ut + vn * nxn);
     T rov = ro * (vt + vn * nyn);
     T row = T(F(j, de, 3));
-    w(ig, jg, 0) = ro;
-    w(ig, jg, 1) = rou;
-    w(ig, jg, 2) = rov;
-    w(ig, jg, 3) = row;
-    w(ig, jg, 4) = p / g1 + 0.5 * (rou * rou + rov * rov + row * row) / ro;
+    in[0] = ro, in[1] = rou, in[2] = rov, in[3] = row;
+    in[4] = p / g1 + 0.5 * (rou * rou + rov * rov + row * row) / ro;
+#pragma unroll
+    for (int e = 0; e < 5; ++e) w.put(ig, jg, e, in[e]);
   }
 }
 
@@ -182,16 +209,17 @@ __global__ void k_bc_inlet(Mesh m, T* __restrict__ wbase, int loc, Box b, const 
                            double gam, long cstride) {
   const int l = 1 + blockIdx.x * blockDim.x + threadIdx.x;
   if (l <= decode_side(loc, b.imin, b.jmin, b.imax, b.jmax).lmax)
-    bc_inlet_line<T, FR>(m, wbase + (long)blockIdx.y * cstride, loc, b, field, lm, nxp, nyp, gam, l);
+    bc_inlet_line(StateView<T, FR>(m, wbase + (long)blockIdx.y * cstride), loc, b, field, lm, nxp, nyp, gam, l);
 }
 
 // Non-reflecting far field against the reference state wbd(l, :).
-template <class T, bool FR = false>
-__device__ inline void bc_noref_line(const Mesh& m, T* __restrict__ wp, const double* __restrict__ wbd, int lm,
+template <class V>
+__device__ inline void bc_noref_line(const V& w, const double* __restrict__ wbd, int lm,
                                      int loc, Box b, const double* __restrict__ nxp,
                                      const double* __restrict__ nyp, double gam, int l) {
+  using T = typename V::Scalar;
+  const Mesh& m = w.m;
   const Side s = decode_side(loc, b.imin, b.jmin, b.imax, b.jmax);
-  StateView<T, FR> w{m, wp};
   const int i1 = s.i0 * s.i0, j1 = s.j0 * s.j0;
   const int i = b.imin + (l - 1) * j1;
   const int j = b.jmin + (l - 1) * i1;
@@ -236,14 +264,16 @@ __device__ inline void bc_noref_line(const Mesh& m, T* __restrict__ wp, const do
   T row = ro * zt;
   T roe = p / g1 + 0.5 * rom1 * (rou * rou + rov * rov + row * row);
   // first ghost layer from the characteristics, the others linearly extrapolated
-  T q[5] = {ro, rou, rov, row, roe};
+  T q[5] = {ro, rou, rov, row, roe}, in[5];
+#pragma unroll
+  for (int e = 0; e < 5; ++e) in[e] = w(i, j, e);
   for (int de = 1; de <= m.gh; ++de) {
-    const int ig = i - de * s.i0, jg = j - de * s.j0;
-    const int ia = i - (de - 1) * s.i0, ja = j - (de - 1) * s.j0;
 #pragma unroll
     for (int e = 0; e < 5; ++e) {
-      w(ig, jg, e) = q[e];
-      q[e] = 2.0 * q[e] - w(ia, ja, e);
+      w.put(i - de * s.i0, j - de * s.j0, e, q[e]);
+      const T nx_ = 2.0 * q[e] - in[e];
+      in[e] = q[e];
+      q[e] = nx_;
     }
   }
 }
@@ -254,35 +284,42 @@ __global__ void k_bc_noref(Mesh m, T* __restrict__ wbase, const double* __restri
                            double gam, long cstride) {
   const int l = 1 + blockIdx.x * blockDim.x + threadIdx.x;
   if (l <= decode_side(loc, b.imin, b.jmin, b.imax, b.jmax).lmax)
-    bc_noref_line<T, FR>(m, wbase + (long)blockIdx.y * cstride, wbd, lm, loc, b, nxp, nyp, gam, l);
+    bc_noref_line(StateView<T, FR>(m, wbase + (long)blockIdx.y * cstride), wbd, lm, loc, b, nxp, nyp, gam, l);
 }
 
-template <class T, bool FR = false>
-__device__ inline void bc_extrap2_line(const Mesh& m, T* __restrict__ wp, int loc, Box b, int em, int l) {
+template <class V>
+__device__ inline void bc_extrap2_line(const V& w, int loc, Box b, int em, int l) {
+  using T = typename V::Scalar;
+  const Mesh& m = w.m;
   const Side s = decode_side(loc, b.imin, b.jmin, b.imax, b.jmax);
-  StateView<T, FR> w{m, wp};
   const int i = b.imin + (l - 1) * s.j0 * s.j0;
   const int j = b.jmin + (l - 1) * s.i0 * s.i0;
-  for (int de = 1; de <= m.gh; ++de)
-    for (int e = 0; e < em; ++e)
-      w(i - s.i0 * de, j - s.j0 * de, e) =
-          2.0 * w(i - s.i0 * (de - 1), j - s.j0 * (de - 1), e) - w(i - s.i0 * (de - 2), j - s.j0 * (de - 2), e);
+  for (int e = 0; e < em; ++e) {
+    T in = w(i + s.i0, j + s.j0, e), q = w(i, j, e);
+    for (int de = 1; de <= m.gh; ++de) {
+      const T next = 2.0 * q - in;
+      w.put(i - s.i0 * de, j - s.j0 * de, e, next);
+      in = q;
+      q = next;
+    }
+  }
 }
 
 template <class T, bool FR = false>
 __global__ void k_bc_extrap2(Mesh m, T* __restrict__ wbase, int loc, Box b, int em, long cstride) {
   const int l = 1 + blockIdx.x * blockDim.x + threadIdx.x;
   if (l <= decode_side(loc, b.imin, b.jmin, b.imax, b.jmax).lmax)
-    bc_extrap2_line<T, FR>(m, wbase + (long)blockIdx.y * cstride, loc, b, em, l);
+    bc_extrap2_line(StateView<T, FR>(m, wbase + (long)blockIdx.y * cstride), loc, b, em, l);
 }
 
 // Adiabatic no-slip wall: first ghost from the 2nd-order zero-normal-gradient
 // pressure and the isentropic density, the deeper ones mirror interior cells
 // with reversed velocity.
-template <class T, bool FR = false>
-__device__ inline void bc_wall_line(const Mesh& m, T* __restrict__ wp, int loc, Box b, double gam, int l) {
+template <class V>
+__device__ inline void bc_wall_line(const V& w, int loc, Box b, double gam, int l) {
+  using T = typename V::Scalar;
+  const Mesh& m = w.m;
   const Side s = decode_side(loc, b.imin, b.jmin, b.imax, b.jmax);
-  StateView<T, FR> w{m, wp};
   const int i = b.imin + (l - 1) * s.j0 * s.j0;
   const int j = b.jmin + (l - 1) * s.i0 * s.i0;
   const double g1 = gam - 1.0;
@@ -301,11 +338,11 @@ __device__ inline void bc_wall_line(const Mesh& m, T* __restrict__ wp, int loc, 
   T ei = pi / g1 + 0.5 * ri * (ui * ui + vi * vi);
   for (int de = 1; de <= m.gh; ++de) {
     const int ig = i - de * s.i0, jg = j - de * s.j0;
-    w(ig, jg, 0) = ri;
-    w(ig, jg, 1) = ri * ui;
-    w(ig, jg, 2) = ri * vi;
-    w(ig, jg, 3) = ri * zi;
-    w(ig, jg, 4) = ei;
+    w.put(ig, jg, 0, ri);
+    w.put(ig, jg, 1, ri * ui);
+    w.put(ig, jg, 2, ri * vi);
+    w.put(ig, jg, 3, ri * zi);
+    w.put(ig, jg, 4, ei);
     const int ii = i + de * s.i0, jj = j + de * s.j0;
     ri = w(ii, jj, 0);
     T rim1 = 1.0 / ri;
@@ -320,7 +357,7 @@ template <class T, bool FR = false>
 __global__ void k_bc_wall(Mesh m, T* __restrict__ wbase, int loc, Box b, double gam, long cstride) {
   const int l = 1 + blockIdx.x * blockDim.x + threadIdx.x;
   if (l <= decode_side(loc, b.imin, b.jmin, b.imax, b.jmax).lmax)
-    bc_wall_line<T, FR>(m, wbase + (long)blockIdx.y * cstride, loc, b, gam, l);
+    bc_wall_line(StateView<T, FR>(m, wbase + (long)blockIdx.y * cstride), loc, b, gam, l);
 }
 
 // Block copy between two boxes of one block (the periodic join of the O-mesh).
@@ -357,6 +394,100 @@ __global__ void k_join(Mesh m, T* __restrict__ wbase, Box prr, Box prd, int tr0,
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t < join_count(prd, tr0, tr1))
     join_cell<T, FR>(m, wbase + (long)blockIdx.y * cstride, prr, prd, tr0, tr1, em, ni_arr, plane, t);
+}
+
+// ------------------------------------------------------------------ sequence
+// A whole BC sequence in one launch.  A line away from the corners reads
+// interior cells and its own ghosts only, so the lines of all operations run
+// side by side; only near a corner does an operation read what an earlier one
+// wrote (a ghost column continued into the corner).  Each corner therefore has
+// a workgroup of its own, one wave that takes the corner's lines of every
+// operation in sequence order, a barrier between them -- those of the lines
+// within gh + 1 cells of the corner that the corner's ghosts are made from
+// among them, which the other workgroups leave out.  bc_sequence_plan (host)
+// admits the sequences for which this order is the sequential one.  What
+// bounds it is the latency of the longest chain (a corner's lines of each
+// operation).  Against one launch per operation (and, with a tangent, the
+// packing of both arrays and a join of each): residual 96x64 45.9 -> 38.6 us,
+// 383x255 O-mesh 126 -> 80 us, tangent 509x381 O-mesh 127 -> 93 us.
+constexpr int BC_SEQ = 8;
+constexpr int BC_SEQ_THREADS = 64;
+struct BcSeqOp {
+  int kind, loc;
+  Box box, box2;
+  const double* data;
+  int lm;
+  double gam;
+  int lo, hi;     // tangential coordinates of the lines away from the corners
+  int first;      // first workgroup of those lines
+  int side;       // join: 0 fills the low i ghosts, 1 the high ones
+};
+struct BcSeq {
+  int n, blocks;  // operations; workgroups before the four corners
+  BcSeqOp op[BC_SEQ];
+  int donor[2];   // a join fills the i ghosts of side 0 / 1: its donors' columns belong to that corner too
+};
+enum { SEQ_INLET = 0, SEQ_NOREF, SEQ_EXTRAP2, SEQ_WALL, SEQ_JOIN };
+
+// tangential extent of an operation's lines, and the line of coordinate t
+__host__ __device__ inline void bc_seq_range(const BcSeqOp& q, int& lo, int& hi) {
+  const bool rows = q.kind == SEQ_JOIN || q.loc < 2;  // lines numbered by j
+  lo = rows ? q.box.jmin : q.box.imin;
+  hi = rows ? q.box.jmax : q.box.imax;
+}
+// cells of a join per row
+__host__ __device__ inline int bc_seq_width(const BcSeqOp& q) {
+  return q.kind == SEQ_JOIN ? q.box.imax - q.box.imin + 1 : 1;
+}
+
+template <class V>
+__device__ inline void bc_seq_line(const V& w, const BcSeqOp& q, const double* nx, const double* ny, int t, int col) {
+  int lo, hi;
+  bc_seq_range(q, lo, hi);
+  if (t < lo || t > hi) return;
+  const int l = t - lo + 1;
+  switch (q.kind) {
+    case SEQ_INLET: bc_inlet_line(w, q.loc, q.box, q.data, q.lm, nx, ny, q.gam, l); break;
+    case SEQ_NOREF: bc_noref_line(w, q.data, q.lm, q.loc, q.box, nx, ny, q.gam, l); break;
+    case SEQ_EXTRAP2: bc_extrap2_line(w, q.loc, q.box, 5, l); break;
+    case SEQ_WALL: bc_wall_line(w, q.loc, q.box, q.gam, l); break;
+    default:
+      for (int e = 0; e < 5; ++e) w.put(q.box.imin + col, t, e, w(q.box2.imin + col, t, e));
+  }
+}
+
+template <class V>
+__global__ void __launch_bounds__(BC_SEQ_THREADS) k_bc_sequence(V w, BcSeq seq, const double* __restrict__ nx,
+                                                                const double* __restrict__ ny) {
+  const int tid = threadIdx.x;
+  const Mesh& m = w.m;
+  if ((int)blockIdx.x < seq.blocks) {
+    int k = 0;
+    while (k + 1 < seq.n && (int)blockIdx.x >= seq.op[k + 1].first) ++k;
+    const BcSeqOp& q = seq.op[k];
+    const int x = ((int)blockIdx.x - q.first) * BC_SEQ_THREADS + tid, wd = bc_seq_width(q);
+    const int t = q.lo + x / wd;
+    if (t <= q.hi) bc_seq_line(w, q, nx, ny, t, x % wd);
+    return;
+  }
+  const int c = blockIdx.x - seq.blocks, is = c % 2, js = c / 2;
+  for (int k = 0; k < seq.n; ++k) {
+    const BcSeqOp& q = seq.op[k];
+    const bool rows = q.kind == SEQ_JOIN || q.loc < 2;
+    const int side = q.kind == SEQ_JOIN ? q.side : q.loc % 2;
+    if (side == (rows ? is : js)) {
+      // the corner's lines, ghosts included: 2 gh + 1 of them
+      const int n = rows ? m.jm : m.im, high = rows ? js : is, wd = bc_seq_width(q);
+      const int t0 = high ? n - m.gh : 1 - m.gh;
+      for (int x = tid; x < (2 * m.gh + 1) * wd; x += BC_SEQ_THREADS)
+        bc_seq_line(w, q, nx, ny, t0 + x / wd, x % wd);
+      // the lines over the donors of this corner's join
+      if (!rows && seq.donor[is] && tid >= 32 && tid < 32 + m.gh)
+        bc_seq_line(w, q, nx, ny, (is ? 1 : m.im - m.gh + 1) + tid - 32, 0);
+    }
+    __threadfence_block();
+    __syncthreads();
+  }
 }
 
 }  // namespace bca

@@ -754,6 +754,114 @@ static int bc_entry(bca_ctx* c, double* w, double* wd, const bca_bc_op& op, cons
   return 0;
 }
 
+}  // extern "C"
+
+namespace {
+
+// The one-launch form of a checked BC sequence (k_bc_sequence), or false where
+// its order could differ from the sequential one.  Admitted: operations on the
+// block's own edges, one per side, or periodic joins of the i sides row by
+// row (a repeated join is one: its donors are interior columns, which nothing
+// between writes but what it already copied); and where an operation's lines
+// run on into the ghosts of a side, nothing later in the sequence fills that
+// side.
+bool bc_sequence_plan(const Mesh& m, const bca_bc_op* ops, int nops, BcSeq& seq) {
+  seq = BcSeq{};
+  if (m.im < 2 * m.gh || m.jm < 2 * m.gh) return false;
+  for (int k = 0; k < nops; ++k) {
+    const bca_bc_op& o = ops[k];
+    BcSeqOp q{};
+    q.kind = o.kind == BCA_BC_INLET ? SEQ_INLET : o.kind == BCA_BC_NOREF ? SEQ_NOREF
+           : o.kind == BCA_BC_EXTRAP2 ? SEQ_EXTRAP2 : o.kind == BCA_BC_WALL_ADIA ? SEQ_WALL : SEQ_JOIN;
+    q.loc = o.loc;
+    q.box = Box{o.box[0], o.box[1], o.box[2], o.box[3]};
+    q.box2 = Box{o.box2[0], o.box2[1], o.box2[2], o.box2[3]};
+    q.data = o.data;
+    q.lm = o.lm;
+    q.gam = o.gam;
+    if (q.kind == SEQ_JOIN) {
+      const Box &r = q.box, &d = q.box2;
+      if (o.tr[0] != 1 || o.tr[1] != 2 || r.jmin < 1 - m.gh || r.jmax > m.jm + m.gh) return false;
+      const bool lowside = r.imin == 1 - m.gh && r.imax == 0 && d.imin == m.im - m.gh + 1 && d.imax == m.im;
+      const bool highside = r.imin == m.im + 1 && r.imax == m.im + m.gh && d.imin == 1 && d.imax == m.gh;
+      if (!(lowside || highside) || r.jmin != d.jmin || r.jmax != d.jmax) return false;
+      q.side = highside ? 1 : 0;
+    } else {
+      const Box& b = q.box;
+      const bool edge = q.loc == 0 ? b.imin == 1 && b.imax == 1 : q.loc == 1 ? b.imin == m.im && b.imax == m.im
+                      : q.loc == 2 ? b.jmin == 1 && b.jmax == 1 : b.jmin == m.jm && b.jmax == m.jm;
+      if (!edge) return false;
+      q.side = -1;
+    }
+    bool repeated = false;
+    for (int p = 0; p < seq.n; ++p) {
+      const BcSeqOp& e = seq.op[p];
+      const bool qi = q.kind == SEQ_JOIN || q.loc < 2, ei = e.kind == SEQ_JOIN || e.loc < 2;
+      const int qs = q.kind == SEQ_JOIN ? q.side : q.loc % 2, es = e.kind == SEQ_JOIN ? e.side : e.loc % 2;
+      if (qi == ei && qs == es) {
+        // the same side again: a repeated join with only joins since, or refused
+        repeated = q.kind == SEQ_JOIN && e.kind == SEQ_JOIN && q.box.jmin == e.box.jmin && q.box.jmax == e.box.jmax;
+        for (int x = p + 1; x < seq.n; ++x) repeated = repeated && seq.op[x].kind == SEQ_JOIN;
+        if (!repeated) return false;
+      } else if (qi != ei) {
+        // the earlier operation's lines into the ghosts this one fills
+        int lo, hi;
+        bc_seq_range(e, lo, hi);
+        const int n = ei ? m.jm : m.im;
+        if (qs == 0 ? lo < 1 : hi > n) return false;
+      }
+    }
+    if (repeated) continue;
+    if (seq.n == BC_SEQ) return false;
+    seq.op[seq.n++] = q;
+    if (q.kind == SEQ_JOIN) seq.donor[q.side] = 1;
+  }
+  for (int k = 0; k < seq.n; ++k) {
+    BcSeqOp& q = seq.op[k];
+    int lo, hi;
+    bc_seq_range(q, lo, hi);
+    const int n = (q.kind == SEQ_JOIN || q.loc < 2) ? m.jm : m.im;
+    q.lo = std::max(lo, m.gh + 2);
+    q.hi = std::min(hi, n - m.gh - 1);
+    q.first = seq.blocks;
+    if (q.hi >= q.lo) seq.blocks += (int)grid1((long)(q.hi - q.lo + 1) * bc_seq_width(q), BC_SEQ_THREADS);
+  }
+  return seq.n > 0;
+}
+
+}  // namespace
+
+extern "C" {
+
+int bca_bc_sequence(bca_ctx* c, double* w, double* wd, const bca_bc_op* ops, int nops, const double* nx,
+                    const double* ny) {
+  if (!c || !w) return fail(-1, "null argument");
+  if (nops < 0 || (nops > 0 && !ops)) return fail(-1, "bad boundary-condition list");
+  const Mesh& m = c->m;
+  int rc = 0;
+  for (int k = 0; k < nops; ++k)  // (a join out of the plan is checked by its own entry)
+    if (ops[k].kind != BCA_BC_JOIN && (rc = bc_check(m, ops[k], nx, ny))) return rc;
+  BcSeq seq;
+  if (bc_sequence_plan(m, ops, nops, seq)) {
+    Timed t(c, "k_bc_sequence");
+    const unsigned nb = (unsigned)seq.blocks + 4;
+    if (wd) k_bc_sequence<<<nb, BC_SEQ_THREADS, 0, c->stream>>>(PairView{m, w, wd}, seq, nx, ny);
+    else k_bc_sequence<<<nb, BC_SEQ_THREADS, 0, c->stream>>>(StateView<double>(m, w), seq, nx, ny);
+    BCA_LAUNCHED();
+    return 0;
+  }
+  for (int k = 0; k < nops; ++k) {
+    const bca_bc_op& o = ops[k];
+    if (o.kind == BCA_BC_JOIN) {
+      for (double* a : {wd, w})
+        if (a && (rc = bca_bc_join(c, a, o.box, o.box2, o.tr, 5, m.ni, m.nj))) return rc;
+    } else if ((rc = bc_entry(c, w, wd, o, nx, ny))) {
+      return rc;
+    }
+  }
+  return 0;
+}
+
 int bca_bc_inlet(bca_ctx* c, double* w, double* wd, int loc, const int box[4], const double* field,
                  int lm, const double* nx, const double* ny, double gam) {
   if (!box) return fail(-1, "null box");

@@ -126,26 +126,8 @@ class Flow:
 
     def apply_bcs(self, w, wd=None):
         """Ghost filling in place (w, and wd with the linearised BCs)."""
-        h = self.ctx.sync_stream()
-        L = self.L
-        for op in self.ops:
-            wp, wdp = _ptr(w), _ptr(wd)
-            box = (C.c_int * 4)(*op.box)
-            if op.kind == _lib.BC_INLET:
-                rc = L.bca_bc_inlet(h, wp, wdp, op.loc, box, op.data, op.lm, _ptr(self.nx), _ptr(self.ny), op.gam)
-            elif op.kind == _lib.BC_NOREF:
-                rc = L.bca_bc_noref(h, wp, wdp, op.data, op.lm, op.loc, box, _ptr(self.nx), _ptr(self.ny), op.gam)
-            elif op.kind == _lib.BC_EXTRAP2:
-                rc = L.bca_bc_extrap2(h, wp, wdp, op.loc, box, 5)
-            elif op.kind == _lib.BC_WALL_ADIA:
-                rc = L.bca_bc_wall_adia(h, wp, wdp, op.loc, box, op.gam)
-            else:
-                box2 = (C.c_int * 4)(*op.box2)
-                trc = (C.c_int * 2)(*op.tr)
-                rc = 0
-                for arr in ([wd] if wd is not None else []) + [w]:
-                    rc = rc or L.bca_bc_join(h, _ptr(arr), box, box2, trc, 5, self.ni, self.nj)
-            _lib.check(rc, "boundary condition")
+        _lib.check(self.L.bca_bc_sequence(self.ctx.sync_stream(), _ptr(w), _ptr(wd), self.ops, self.nops,
+                                          _ptr(self.nx), _ptr(self.ny)), "boundary condition")
 
     # ------------------------------------------------------------ operators
     def new_state(self):

@@ -210,6 +210,13 @@ int bca_bc_wall_adia(bca_ctx *ctx, double *w, double *wd, int loc, const int box
  * em planes. */
 int bca_bc_join(bca_ctx *ctx, double *a, const int prr[4], const int prd[4], const int tr[2],
                 int em, int ni_arr, int nj_arr);
+/* A whole sequence of them in order (w, and wd with the linearised BCs where it
+ * is not null), the driver's per-iteration ghost filling (BROADCAST_npz.py:
+ * 1018-1021, 1079-1082; cylinder.py:853-862): one launch where every operation
+ * lies on an edge of the block, else one after the other.  Joins are applied
+ * to w and to wd. */
+int bca_bc_sequence(bca_ctx *ctx, double *w, double *wd, const bca_bc_op *ops, int nops, const double *nx,
+                    const double *ny);
 
 /* ---- f_norm -------------------------------------------------------------- */
 /* compute_norml2inf(norm,ninf,rhs,im,jm,gh)  srcfv/norm.F90:34-77
