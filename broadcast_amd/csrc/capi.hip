@@ -19,6 +19,7 @@
 #include "vjp.h"
 #include "csr.h"
 #include "dz.h"
+#include "residual.h"
 #include "batch.h"
 #include "bcadj.h"
 #include "jaccsr.h"
@@ -48,14 +49,10 @@ int fail(int code, const std::string& msg) {
     if (e_ != hipSuccess) return fail(-3, std::string("kernel launch: ") + hipGetErrorString(e_)); \
   } while (0)
 
-// Per-scalar-type scratch planes of one pipeline pass.
-template <class T>
+// Primitives and velocity gradients of the Jacobian and adjoint passes.
 struct Work {
-  T* w = nullptr;
-  T* res = nullptr;
-  T* prim = nullptr;
-  T* grad = nullptr;
-  T* hn = nullptr;
+  double* prim = nullptr;
+  double* grad = nullptr;
 };
 
 }  // namespace
@@ -91,8 +88,9 @@ struct bca_ctx {
   hipEvent_t fork_ev = nullptr, join_ev[3] = {nullptr, nullptr, nullptr};
   long bytes = 0;
   KernelTimer timer;
-  Work<double> w0;
-  Work<Dual<1>> w1;
+  Work w0;
+  Dual<1>* wpair = nullptr;   // a state and its tangent packed for one boundary condition
+  double* res_tmp = nullptr;  // outputs of a residual or tangent that share memory with its inputs
   double* norm_part = nullptr;
   double* norm_out = nullptr;
   double* cellx = nullptr;  // 1 / rho and d mu / d T of every cell
@@ -116,7 +114,6 @@ struct bca_ctx {
   unsigned long long* jr_mask = nullptr;  // its kept masks (column order, 8 words per row)
   int* jr_cnt = nullptr;                  // its row lengths
   // launch shapes chosen by bca_autotune for this mesh (defaults until then)
-  dim3 tune_face{64, 4, 1};      // k_face<double>
   dim3 tune_blocks{64, 4, 1};    // interior face-block kernels of phase 1
   dim3 tune_assemble{256, 1, 1}; // k_assemble_colored
 };
@@ -127,11 +124,6 @@ constexpr int NORM_BLOCKS = 240;
 // csr_aux: SCAN_B * SCAN_B scan block sums, then the total, the error flag
 // and the changed-row flag of the refresh pass (every user allocates this size)
 constexpr long CSR_AUX_INTS = (long)SCAN_B * SCAN_B + 4;
-
-template <class T> const char* tname();
-template <> const char* tname<double>() { return "f64"; }
-template <> const char* tname<Dual<1>>() { return "dual1"; }
-template <> const char* tname<Dual<5>>() { return "dual5"; }
 
 // Records a start event before and a stop event after the launch it wraps.
 struct Timed {
@@ -174,25 +166,9 @@ int realloc_planes(bca_ctx* c, T** p, long count) {
   return alloc_planes(c, p, count);
 }
 
-template <class T>
-int ensure_work(bca_ctx* c, Work<T>& wk, bool with_state) {
-  const Mesh& m = c->m;
-  int rc = 0;
-  if ((rc = alloc_planes(c, &wk.prim, NPRIM * m.ncell))) return rc;
-  if ((rc = alloc_planes(c, &wk.grad, NGRAD * m.ncell))) return rc;
-  if ((rc = alloc_planes(c, &wk.hn, 10 * m.nnode))) return rc;
-  if (with_state) {
-    if ((rc = alloc_planes(c, &wk.w, 5 * m.ncell))) return rc;
-    if ((rc = alloc_planes(c, &wk.res, 5 * m.ncell))) return rc;
-  }
-  return 0;
-}
-
-template <class T>
-void free_work(Work<T>& wk) {
-  for (T* p : {wk.w, wk.res, wk.prim, wk.grad, wk.hn})
-    if (p) (void)hipFree(p);
-  wk = Work<T>();
+int ensure_work(bca_ctx* c) {
+  int rc = alloc_planes(c, &c->w0.prim, NPRIM * c->m.ncell);
+  return rc ? rc : alloc_planes(c, &c->w0.grad, NGRAD * c->m.ncell);
 }
 
 inline dim3 grid2(int ni, int nj, dim3 b) { return dim3((ni + b.x - 1) / b.x, (nj + b.y - 1) / b.y); }
@@ -216,57 +192,39 @@ int need_gh3(const bca_ctx* c) {
   return 0;
 }
 
-// The residual pipeline on scalar type T; residu == nullptr stops after the faces.
-// WP: the state as planes of T, or a SplitState (T = Dual<1>)
-template <class T, class WP = const T*>
-int run_pipeline(bca_ctx* c, Work<T>& wk, WP w, T* residu, const Metric& g, const Phys& ph,
-                 bool nowall = false, int ord = 5) {
-  const Mesh& m = c->m;
-  hipStream_t s = c->stream;
-  const std::string sfx = std::string("<") + tname<T>() + ">";
-  // the faces read the state by stencil from planes of T: a SplitState is
-  // copied to wk.w by k_prim on the way
-  const T* wf;
-  T* wcopy = nullptr;
-  if constexpr (std::is_same<WP, SplitState>::value) wf = wcopy = wk.w;
-  else wf = w;
-  {
-    Timed t(c, "k_prim" + sfx);
-    k_prim<T, WP><<<grid1(m.ncell, 256), 256, 0, s>>>(m, ph, w, wk.prim, wcopy);
-  }
+// Do the 5-plane arrays at a and b share memory?
+bool overlap(const Mesh& m, const double* a, const double* b) {
+  const long n = 5 * m.ncell;
+  return a && b && a < b + n && b < a + n;
+}
+
+// One launch of k_residual.  V: StateView<double> or PairView.
+template <class V>
+int launch_residual(const V& w, const bca_phys* p, const bca_metrics& g, const ResOut& out, bool nowall, int ord,
+                    hipStream_t s) {
+  const Mesh& m = w.m;
+  const ResPhys ph = res_phys(to_phys(p));
+  const Metric mg = to_metric(g);
+  const dim3 gr((m.im + TILE_CELLS - 1) / TILE_CELLS, (m.jm + TILE_CELLS - 1) / TILE_CELLS);
+#define BCA_RES(ORD, NW) k_residual<V, ORD, NW><<<gr, TILE_THREADS, 0, s>>>(w, ph, mg, out)
+  if (ord == 3 && nowall) BCA_RES(3, true);
+  else if (ord == 3) BCA_RES(3, false);
+  else if (ord == 7 && nowall) BCA_RES(7, true);
+  else if (ord == 7) BCA_RES(7, false);
+  else if (ord == 9 && nowall) BCA_RES(9, true);
+  else if (ord == 9) BCA_RES(9, false);
+  else if (nowall) BCA_RES(5, true);
+  else BCA_RES(5, false);
+#undef BCA_RES
   BCA_LAUNCHED();
+  return 0;
+}
+
+// Outputs that share memory with an input (w in place, say) go through tmp
+// (5 planes each): a tile's stencil reads cells that another tile writes.
+int launch_store(const Mesh& m, const double* from, double* to, hipStream_t s) {
   const dim3 b(64, 4);
-  {
-    Timed t(c, "k_grad" + sfx);
-    const dim3 gg = grid2(m.im, m.jm, b);
-    if (ord == 3) k_grad<T, 3><<<gg, b, 0, s>>>(m, g, wk.prim, wk.grad);
-    else if (ord == 7) k_grad<T, 7><<<gg, b, 0, s>>>(m, g, wk.prim, wk.grad);
-    else if (ord == 9) k_grad<T, 9><<<gg, b, 0, s>>>(m, g, wk.prim, wk.grad);
-    else k_grad<T><<<gg, b, 0, s>>>(m, g, wk.prim, wk.grad);
-  }
-  BCA_LAUNCHED();
-  k_grad_ghost<T><<<grid1(2 * m.im + m.jm, 256), 256, 0, s>>>(m, wk.grad);
-  BCA_LAUNCHED();
-  const dim3 bf = sizeof(T) > 8 ? dim3(64, 1) : c->tune_face;
-  {
-    Timed t(c, "k_face" + sfx);
-    const dim3 gf = grid2(m.im + 1, m.jm + 1, bf);
-#define BCA_FACE(NW, ORD) k_face<T, NW, ORD><<<gf, bf, 0, s>>>(m, ph, g, wf, wk.prim, wk.grad, wk.hn)
-    if (ord == 3 && nowall) BCA_FACE(true, 3);
-    else if (ord == 3) BCA_FACE(false, 3);
-    else if (ord == 7 && nowall) BCA_FACE(true, 7);
-    else if (ord == 7) BCA_FACE(false, 7);
-    else if (ord == 9 && nowall) BCA_FACE(true, 9);
-    else if (ord == 9) BCA_FACE(false, 9);
-    else if (nowall) BCA_FACE(true, 5);
-    else BCA_FACE(false, 5);
-#undef BCA_FACE
-  }
-  BCA_LAUNCHED();
-  if (residu) {
-    Timed t(c, "k_balance" + sfx);
-    k_balance<T><<<grid2(m.im, m.jm, b), b, 0, s>>>(m, wk.hn, residu);
-  }
+  k_store_interior<<<grid2(m.im, m.jm, b), b, 0, s>>>(m, from, to);
   BCA_LAUNCHED();
   return 0;
 }
@@ -479,8 +437,10 @@ int bca_ctx_destroy(bca_ctx* c) {
   }
   if (c->fork_ev) (void)hipEventDestroy(c->fork_ev);
   for (hipEvent_t e : c->timer.pool) (void)hipEventDestroy(e);
-  free_work(c->w0);
-  free_work(c->w1);
+  for (double* p : {c->w0.prim, c->w0.grad})
+    if (p) (void)hipFree(p);
+  if (c->wpair) (void)hipFree(c->wpair);
+  if (c->res_tmp) (void)hipFree(c->res_tmp);
   if (c->norm_part) (void)hipFree(c->norm_part);
   if (c->norm_out) (void)hipFree(c->norm_out);
   for (double* p : {c->cellx, c->blki, c->blkj, c->ghostT, c->vjpi, c->vjpj})
@@ -567,8 +527,16 @@ static int residual_impl(bca_ctx* c, double* residu, const double* w, bca_metric
   if (!c || !residu || !w || !p || !g.nx || !g.ny || !g.vol || !g.volf) return fail(-1, "null argument");
   int rc = order_ok(c, ord, nowall);
   if (rc) return rc;
-  if ((rc = ensure_work(c, c->w0, false))) return rc;
-  return run_pipeline<double>(c, c->w0, w, residu, to_metric(g), to_phys(p), nowall, ord);
+  const Mesh& m = c->m;
+  const bool through = overlap(m, residu, w);
+  if (through && (rc = alloc_planes(c, &c->res_tmp, 10 * m.ncell))) return rc;
+  {
+    Timed t(c, "k_residual<f64>");
+    if ((rc = launch_residual(StateView<double>(m, const_cast<double*>(w)), p, g,
+                              ResOut{through ? c->res_tmp : residu, nullptr}, nowall, ord, c->stream)))
+      return rc;
+  }
+  return through ? launch_store(m, c->res_tmp, residu, c->stream) : 0;
 }
 
 int bca_residual_dnc5(bca_ctx* c, double* residu, const double* w, bca_metrics g, const bca_phys* p) {
@@ -629,29 +597,14 @@ int bca_residual_dnc5_noalloc(double* residu, const double* w, bca_metrics g, co
     return fail(-4, "bca_residual_dnc5_noalloc: the mesh needs " + std::to_string(need) +
                         " bytes of scratch, the library's static scratch holds " +
                         std::to_string((long)BCA_NOALLOC_SCRATCH_BYTES));
-  double* base = nullptr;
-  if ((rc = noalloc_scratch(&base))) return rc;
-  double* prim = base;
-  double* grad = prim + NPRIM * m.ncell;
-  double* hn = grad + NGRAD * m.ncell;
+  // the kernel of bca_residual_dnc5, bit for bit; the scratch serves a residu
+  // that shares memory with w
   const hipStream_t s = (hipStream_t)stream;
-  const Metric mg = to_metric(g);
-  const Phys ph = to_phys(p);
-  // the kernels and launch shapes of bca_residual_dnc5 (every scratch value
-  // they read is written earlier in the same call, so nothing is cleared)
-  k_prim<double><<<grid1(m.ncell, 256), 256, 0, s>>>(m, ph, w, prim);
-  BCA_LAUNCHED();
-  const dim3 b(64, 4);
-  k_grad<double><<<grid2(m.im, m.jm, b), b, 0, s>>>(m, mg, prim, grad);
-  BCA_LAUNCHED();
-  k_grad_ghost<double><<<grid1(2 * m.im + m.jm, 256), 256, 0, s>>>(m, grad);
-  BCA_LAUNCHED();
-  const dim3 bf(64, 4);
-  k_face<double><<<grid2(m.im + 1, m.jm + 1, bf), bf, 0, s>>>(m, ph, mg, w, prim, grad, hn);
-  BCA_LAUNCHED();
-  k_balance<double><<<grid2(m.im, m.jm, b), b, 0, s>>>(m, hn, residu);
-  BCA_LAUNCHED();
-  return 0;
+  double* out = residu;
+  if (overlap(m, residu, w) && (rc = noalloc_scratch(&out))) return rc;
+  if ((rc = launch_residual(StateView<double>(m, const_cast<double*>(w)), p, g, ResOut{out, nullptr}, false, 5, s)))
+    return rc;
+  return out != residu ? launch_store(m, out, residu, s) : 0;
 }
 
 static int jvp_impl(bca_ctx* c, double* residu, double* residud, const double* w, const double* wd,
@@ -659,21 +612,19 @@ static int jvp_impl(bca_ctx* c, double* residu, double* residud, const double* w
   if (!c || !w || !wd || !p || !g.nx || !g.ny || !g.vol || !g.volf) return fail(-1, "null argument");
   int rc = order_ok(c, ord, nowall);
   if (rc) return rc;
-  if ((rc = ensure_work(c, c->w1, true))) return rc;
   const Mesh& m = c->m;
-  // the pipeline up to the face fluxes, reading (w, wd) as Dual<1> where it
-  // reads the state (no packed copy), then the balance straight into
-  // residu / residud
-  if ((rc = run_pipeline<Dual<1>, SplitState>(c, c->w1, SplitState{w, wd}, nullptr, to_metric(g), to_phys(p),
-                                               nowall, ord)))
-    return rc;
-  const dim3 b(64, 4);
+  const bool tr = overlap(m, residu, w) || overlap(m, residu, wd);
+  const bool td = overlap(m, residud, w) || overlap(m, residud, wd);
+  if ((tr || td) && (rc = alloc_planes(c, &c->res_tmp, 10 * m.ncell))) return rc;
+  double* const tmpd = c->res_tmp ? c->res_tmp + 5 * m.ncell : nullptr;
   {
-    Timed t(c, "k_balance<" + std::string(tname<Dual<1>>()) + ">");
-    k_balance_split<1><<<grid2(m.im, m.jm, b), b, 0, c->stream>>>(m, c->w1.hn, residu, residud);
+    Timed t(c, "k_residual<dual1>");
+    if ((rc = launch_residual(PairView{m, const_cast<double*>(w), const_cast<double*>(wd)}, p, g,
+                              ResOut{tr ? c->res_tmp : residu, td ? tmpd : residud}, nowall, ord, c->stream)))
+      return rc;
   }
-  BCA_LAUNCHED();
-  return 0;
+  if (tr && (rc = launch_store(m, c->res_tmp, residu, c->stream))) return rc;
+  return td ? launch_store(m, tmpd, residud, c->stream) : 0;
 }
 
 int bca_jvp_dnc5(bca_ctx* c, double* residu, double* residud, const double* w, const double* wd,
@@ -731,25 +682,25 @@ static int bc_entry(bca_ctx* c, double* w, double* wd, const bca_bc_op& op, cons
                     const double* ny) {
   if (!c || !w) return fail(-1, "null argument");
   if (!wd) return launch_bc<double>(c, w, op, nx, ny);
-  int rc = ensure_work(c, c->w1, true);
+  int rc = alloc_planes(c, &c->wpair, 5 * c->m.ncell);
   if (rc) return rc;
   if ((rc = bc_check(c->m, op, nx, ny))) return rc;
   // a BC on the block edge reads and writes the boundary frame only: pack
   // and unpack that (1/50 of the array at 2048 x 1024), else the whole array
   if (op_in_frame(c->m, op)) {
     const unsigned nb = grid1(frame_count(c->m, BC_FRAME), 256);
-    k_pack_frame<<<nb, 256, 0, c->stream>>>(c->m, w, wd, c->w1.w);
+    k_pack_frame<<<nb, 256, 0, c->stream>>>(c->m, w, wd, c->wpair);
     BCA_LAUNCHED();
-    if ((rc = launch_bc<Dual<1>>(c, c->w1.w, op, nx, ny))) return rc;
-    k_unpack_frame<<<nb, 256, 0, c->stream>>>(c->m, c->w1.w, w, wd);
+    if ((rc = launch_bc<Dual<1>>(c, c->wpair, op, nx, ny))) return rc;
+    k_unpack_frame<<<nb, 256, 0, c->stream>>>(c->m, c->wpair, w, wd);
     BCA_LAUNCHED();
     return 0;
   }
   const long n = 5 * c->m.ncell;
-  k_pack<1><<<grid1(n, 256), 256, 0, c->stream>>>(n, w, wd, c->w1.w);
+  k_pack<1><<<grid1(n, 256), 256, 0, c->stream>>>(n, w, wd, c->wpair);
   BCA_LAUNCHED();
-  if ((rc = launch_bc<Dual<1>>(c, c->w1.w, op, nx, ny))) return rc;
-  k_unpack<1><<<grid1(n, 256), 256, 0, c->stream>>>(n, c->w1.w, w, wd);
+  if ((rc = launch_bc<Dual<1>>(c, c->wpair, op, nx, ny))) return rc;
+  k_unpack<1><<<grid1(n, 256), 256, 0, c->stream>>>(n, c->wpair, w, wd);
   BCA_LAUNCHED();
   return 0;
 }
@@ -1086,7 +1037,7 @@ int jacobian_phase1(bca_ctx* c, const double* w, bca_metrics g, const bca_phys* 
   const Mesh& m = c->m;
   int rc = 0;
   if ((rc = check_ops_frame(m, ops, nops, g.nx, g.ny))) return rc;
-  if ((rc = ensure_work(c, c->w0, false))) return rc;
+  if ((rc = ensure_work(c))) return rc;
   const long nfi = (long)(m.im + 1) * m.jm, nfj = (long)m.im * (m.jm + 1);
   if ((rc = alloc_planes(c, &c->cellx, NCELLX * m.ncell))) return rc;
   if ((rc = alloc_planes(c, &c->blki, (long)NOFF * 25 * nfi))) return rc;
@@ -1211,7 +1162,7 @@ int bca_vjp_dnc5(bca_ctx* c, double* residub, double* wb, const double* w, bca_m
   if (int rc_gh = need_gh3(c)) return rc_gh;
   const Mesh& m = c->m;
   int rc = 0;
-  if ((rc = ensure_work(c, c->w0, false))) return rc;
+  if ((rc = ensure_work(c))) return rc;
   const long nfi = (long)(m.im + 1) * m.jm, nfj = (long)m.im * (m.jm + 1);
   if ((rc = alloc_planes(c, &c->vjpi, (long)NOFF * 5 * nfi))) return rc;
   if ((rc = alloc_planes(c, &c->vjpj, (long)NOFF * 5 * nfj))) return rc;
@@ -2262,18 +2213,6 @@ int bca_autotune(bca_ctx* c, const double* w, bca_metrics g, const bca_phys* p, 
                          dim3(64, 1)};
   std::string rep;
   float best = 0.f, ms = 0.f;
-  // residual faces
-  best = 1e30f;
-  for (const dim3& b : shapes) {
-    if ((rc = time_launch(c, reps, [&] {
-           k_face<double><<<grid2(m.im + 1, m.jm + 1, b), b, 0, s>>>(m, ph, gm, w, c->w0.prim, c->w0.grad, c->w0.hn);
-         }, ms)))
-      return rc;
-    BCA_LAUNCHED();
-    if (ms < best) { best = ms; c->tune_face = b; }
-  }
-  rep += "k_face " + std::to_string(c->tune_face.x) + "x" + std::to_string(c->tune_face.y) + " " +
-         std::to_string(best) + " ms; ";
   // interior face blocks (both families share the shape)
   best = 1e30f;
   for (const dim3& b : shapes) {
@@ -2287,7 +2226,7 @@ int bca_autotune(bca_ctx* c, const double* w, bca_metrics g, const bca_phys* p, 
     BCA_LAUNCHED();
     if (ms < best) { best = ms; c->tune_blocks = b; }
   }
-  rep += "face blocks " + std::to_string(c->tune_blocks.x) + "x" + std::to_string(c->tune_blocks.y) + " " +
+  rep += "k_face_blocks " + std::to_string(c->tune_blocks.x) + "x" + std::to_string(c->tune_blocks.y) + " " +
          std::to_string(best) + " ms; ";
   // colored assembly into the caller's COO (values only)
   best = 1e30f;

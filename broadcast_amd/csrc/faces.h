@@ -617,39 +617,4 @@ __device__ inline void jface_any(const A& a, typename A::Out hn[5]) {
   }
 }
 
-// One thread per (i, j) in [1, im+1] x [1, jm+1]: the i-face (i, j) when
-// j <= jm and the j-face (i, j) when i <= im (the faces the balance reads).
-// NOWALL: the variants without wall rows (srcfv/rhs/flux_num_dnc5_nowall.F90:
-// 140-154, flux_num_dnc3_nowall.F90): every face takes the interior formulas,
-// the centred Euler flux and the viscous flux of the order (compact 4th-order
-// for ORD 5, 7, 9, 2nd-order for ORD 3), the ghost layers supplying the stencil at
-// the block edges.  ORD: 3, 5, 7, 9 = flux_num_dnc3*, _dnc5*, _dnc7*, _dnc9*.
-template <class T, bool NOWALL = false, int ORD = 5>
-__global__ void __launch_bounds__(256) k_face(Mesh m, Phys ph, Metric g, const T* __restrict__ w,
-                                              const T* __restrict__ prim, const T* __restrict__ grad,
-                                              T* __restrict__ hn) {
-  int bx, by;
-  xcd_block(bx, by);
-  const int i = 1 + bx * blockDim.x + threadIdx.x;
-  const int j = 1 + by * blockDim.y + threadIdx.y;
-  if (i > m.im + 1 || j > m.jm + 1) return;
-  PlainAcc<T> a;
-  a.m = m; a.ph = ph; a.g = g; a.i = i; a.j = j;
-  a.w = w; a.prim = prim; a.grad = grad;
-  const long f = nidx(m, i, j);
-  T h[5];
-  if (j <= m.jm) {
-    if constexpr (NOWALL) iface<ORD != 3, ORD>(a, h);
-    else iface_any<ORD>(a, h);
-#pragma unroll
-    for (int e = 0; e < 5; ++e) hn[f + (long)e * m.nnode] = h[e];
-  }
-  if (i <= m.im) {
-    if constexpr (NOWALL) jface<0, ORD != 3, ORD>(a, h);
-    else jface_any<ORD>(a, h);
-#pragma unroll
-    for (int e = 0; e < 5; ++e) hn[f + (long)(5 + e) * m.nnode] = h[e];
-  }
-}
-
 }  // namespace bca

@@ -7,12 +7,11 @@
 // every multi-component field is a stack of such planes (SoA), so a wavefront
 // walking i reads 64 consecutive doubles per plane.
 //
-// The pipeline is four passes over HBM-resident planes:
-//   prim   : every cell (ghosts too)  w -> u, v, w, T, p, mu, H
+// The residual and its tangent are one kernel (residual.h).  The Jacobian and
+// adjoint passes read planes of
+//   prim   : every cell (ghosts too)  u, v, w, T, p, mu, H
 //   grad   : interior cells           4th-order velocity gradients (u, v)
 //   ghost  : one extrapolated layer of gradients where faces read it
-//   face   : every face               hn = Euler - dissipation - viscous
-//   balance: interior cells           residu = -(d_i hn_i + d_j hn_j)
 #pragma once
 #include <hip/hip_runtime.h>
 #include "dual.h"
@@ -139,14 +138,6 @@ struct Coef {
   static constexpr double twothird = 2.0 / 3.0;
 };
 
-template <class T>
-struct Planes {
-  const T* w;      // 5 cell planes
-  T* prim;         // NPRIM cell planes
-  T* grad;         // NGRAD cell planes
-  T* hn;           // 10 node planes: e + 5*dir
-};
-
 struct Metric {
   const double* nx;   // 2 node planes
   const double* ny;
@@ -154,22 +145,9 @@ struct Metric {
   const double* volf; // 2 cell planes
 };
 
-// The state (w, wd) of a tangent read straight from its two double arrays as
-// Dual<1> values, in place of a packed Dual<1> copy: w[k] = (w[k], wd[k]).
-struct SplitState {
-  const double* v;
-  const double* d;
-  __device__ Dual<1> operator[](long k) const {
-    Dual<1> x(v[k]);
-    x.d[0] = d[k];
-    return x;
-  }
-};
-
 // ---------------------------------------------------------------- primitives
-// WP: a pointer to planes of T, or a SplitState for T = Dual<1>
-template <class T, class WP = const T*>
-__device__ inline void primitives(const Mesh& m, const Phys& ph, WP w, T* prim, long c) {
+template <class T>
+__device__ inline void primitives(const Mesh& m, const Phys& ph, const T* w, T* prim, long c) {
   const double cvm1 = 1.0 / ph.cv;
   const double betas = ph.muref * (ph.tref + ph.cs) / (sqrt(ph.tref) * ph.tref);
   const long n = m.ncell;
@@ -191,16 +169,10 @@ __device__ inline void primitives(const Mesh& m, const Phys& ph, WP w, T* prim, 
   prim[c + P_MU * n] = betas / (t + ph.s_suth) * dsqrt(t) * t;
 }
 
-// wcopy (optional): the state as planes of T as well, for the kernels that
-// read it by stencil (one load per value there, where a SplitState takes two)
-template <class T, class WP = const T*>
-__global__ void k_prim(Mesh m, Phys ph, WP w, T* __restrict__ prim, T* __restrict__ wcopy = nullptr) {
+template <class T>
+__global__ void k_prim(Mesh m, Phys ph, const T* __restrict__ w, T* __restrict__ prim) {
   const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= m.ncell) return;
-  primitives<T, WP>(m, ph, w, prim, c);
-  if (wcopy)
-#pragma unroll
-    for (int e = 0; e < 5; ++e) wcopy[c + e * m.ncell] = w[c + e * m.ncell];
+  if (c < m.ncell) primitives(m, ph, w, prim, c);
 }
 
 // ---------------------------------------------------------------- gradients
@@ -305,33 +277,6 @@ __device__ inline T balance_at(const Mesh& m, const T* hn, int i, int j, int e) 
   const T* hi = hn + (long)e * nn;
   const T* hj = hn + (long)(5 + e) * nn;
   return -(hi[nidx(m, i + 1, j)] - hi[nidx(m, i, j)]) - (hj[nidx(m, i, j + 1)] - hj[nidx(m, i, j)]);
-}
-
-template <class T>
-__global__ void k_balance(Mesh m, const T* __restrict__ hn, T* __restrict__ residu) {
-  const int i = 1 + blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = 1 + blockIdx.y * blockDim.y + threadIdx.y;
-  if (i > m.im || j > m.jm) return;
-  const long c = cidx(m, i, j);
-#pragma unroll
-  for (int e = 0; e < 5; ++e) residu[c + (long)e * m.ncell] = balance_at(m, hn, i, j, e);
-}
-
-// The balance of Dual<N> fluxes written as residu (values) and residud (the
-// first tangent) on the interior (either may be null; ghosts untouched).
-template <int N>
-__global__ void k_balance_split(Mesh m, const Dual<N>* __restrict__ hn, double* __restrict__ residu,
-                                double* __restrict__ residud) {
-  const int i = 1 + blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = 1 + blockIdx.y * blockDim.y + threadIdx.y;
-  if (i > m.im || j > m.jm) return;
-  const long c = cidx(m, i, j);
-#pragma unroll
-  for (int e = 0; e < 5; ++e) {
-    const Dual<N> v = balance_at(m, hn, i, j, e);
-    if (residu) residu[c + (long)e * m.ncell] = v.v;
-    if (residud) residud[c + (long)e * m.ncell] = v.d[0];
-  }
 }
 
 }  // namespace bca
