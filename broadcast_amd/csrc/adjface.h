@@ -365,7 +365,7 @@ __device__ inline void face_reverse(const Mesh& m, const Phys& ph, const Metric&
 #pragma unroll
   for (int e = 0; e < 5; ++e) {
     const double jp = 0.5 * (a.template W<0, 0>(e) - a.template W<-DX, -DY>(e));
-    const double pr = predictor<5, DX, DY>(a, e);
+    const double pr = predictor<DX, DY>(a, e);
     rspb -= hb[e] * (ds.eps2 * jp + ds.eps4 * pr);
     e2b -= hb[e] * ds.rspec * jp;
     e4b -= hb[e] * ds.rspec * pr;
@@ -448,7 +448,7 @@ __device__ inline void face_reverse(const Mesh& m, const Phys& ph, const Metric&
 #pragma unroll
     for (int e = 0; e < 5; ++e) {
       const double cj = 0.5 * (ind.template W<0, 0>(e) - ind.template W<-DX, -DY>(e));
-      const double cp = predictor<5, DX, DY>(ind, e);
+      const double cp = predictor<DX, DY>(ind, e);
       wb[e] -= hb[e] * ds.rspec * (ds.eps2 * cj + ds.eps4 * cp);
     }
     // the dissipation scalars through the cell's state, T, p and gradients

@@ -452,25 +452,26 @@ __device__ inline void bc_seq_line(const V& w, const BcSeqOp& q, const double* n
     case SEQ_EXTRAP2: bc_extrap2_line(w, q.loc, q.box, 5, l); break;
     case SEQ_WALL: bc_wall_line(w, q.loc, q.box, q.gam, l); break;
     default:
-      for (int e = 0; e < 5; ++e) w.put(q.box.imin + col, t, e, w(q.box2.imin + col, t, e));
+      for (int e = 0; e < 5; ++e)
+        w.put(q.box.imin + col, t, e, w(q.box2.imin + col, t + q.box2.jmin - q.box.jmin, e));
   }
 }
 
+// workgroup `block` of seq.blocks + 4, BC_SEQ_THREADS threads
 template <class V>
-__global__ void __launch_bounds__(BC_SEQ_THREADS) k_bc_sequence(V w, BcSeq seq, const double* __restrict__ nx,
-                                                                const double* __restrict__ ny) {
+__device__ inline void bc_sequence(const V& w, const BcSeq& seq, const double* nx, const double* ny, int block) {
   const int tid = threadIdx.x;
   const Mesh& m = w.m;
-  if ((int)blockIdx.x < seq.blocks) {
+  if (block < seq.blocks) {
     int k = 0;
-    while (k + 1 < seq.n && (int)blockIdx.x >= seq.op[k + 1].first) ++k;
+    while (k + 1 < seq.n && block >= seq.op[k + 1].first) ++k;
     const BcSeqOp& q = seq.op[k];
-    const int x = ((int)blockIdx.x - q.first) * BC_SEQ_THREADS + tid, wd = bc_seq_width(q);
+    const int x = (block - q.first) * BC_SEQ_THREADS + tid, wd = bc_seq_width(q);
     const int t = q.lo + x / wd;
     if (t <= q.hi) bc_seq_line(w, q, nx, ny, t, x % wd);
     return;
   }
-  const int c = blockIdx.x - seq.blocks, is = c % 2, js = c / 2;
+  const int c = block - seq.blocks, is = c % 2, js = c / 2;
   for (int k = 0; k < seq.n; ++k) {
     const BcSeqOp& q = seq.op[k];
     const bool rows = q.kind == SEQ_JOIN || q.loc < 2;
@@ -488,6 +489,12 @@ __global__ void __launch_bounds__(BC_SEQ_THREADS) k_bc_sequence(V w, BcSeq seq, 
     __threadfence_block();
     __syncthreads();
   }
+}
+
+template <class V>
+__global__ void __launch_bounds__(BC_SEQ_THREADS) k_bc_sequence(V w, BcSeq seq, const double* __restrict__ nx,
+                                                                const double* __restrict__ ny) {
+  bc_sequence(w, seq, nx, ny, blockIdx.x);
 }
 
 }  // namespace bca

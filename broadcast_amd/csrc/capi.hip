@@ -716,20 +716,25 @@ namespace {
 // between writes but what it already copied); and where an operation's lines
 // run on into the ghosts of a side, nothing later in the sequence fills that
 // side.
+BcSeqOp to_seq_op(const bca_bc_op& o) {
+  BcSeqOp q{};
+  q.kind = o.kind == BCA_BC_INLET ? SEQ_INLET : o.kind == BCA_BC_NOREF ? SEQ_NOREF
+         : o.kind == BCA_BC_EXTRAP2 ? SEQ_EXTRAP2 : o.kind == BCA_BC_WALL_ADIA ? SEQ_WALL : SEQ_JOIN;
+  q.loc = o.loc;
+  q.box = Box{o.box[0], o.box[1], o.box[2], o.box[3]};
+  q.box2 = Box{o.box2[0], o.box2[1], o.box2[2], o.box2[3]};
+  q.data = o.data;
+  q.lm = o.lm;
+  q.gam = o.gam;
+  return q;
+}
+
 bool bc_sequence_plan(const Mesh& m, const bca_bc_op* ops, int nops, BcSeq& seq) {
   seq = BcSeq{};
   if (m.im < 2 * m.gh || m.jm < 2 * m.gh) return false;
   for (int k = 0; k < nops; ++k) {
     const bca_bc_op& o = ops[k];
-    BcSeqOp q{};
-    q.kind = o.kind == BCA_BC_INLET ? SEQ_INLET : o.kind == BCA_BC_NOREF ? SEQ_NOREF
-           : o.kind == BCA_BC_EXTRAP2 ? SEQ_EXTRAP2 : o.kind == BCA_BC_WALL_ADIA ? SEQ_WALL : SEQ_JOIN;
-    q.loc = o.loc;
-    q.box = Box{o.box[0], o.box[1], o.box[2], o.box[3]};
-    q.box2 = Box{o.box2[0], o.box2[1], o.box2[2], o.box2[3]};
-    q.data = o.data;
-    q.lm = o.lm;
-    q.gam = o.gam;
+    BcSeqOp q = to_seq_op(o);
     if (q.kind == SEQ_JOIN) {
       const Box &r = q.box, &d = q.box2;
       if (o.tr[0] != 1 || o.tr[1] != 2 || r.jmin < 1 - m.gh || r.jmax > m.jm + m.gh) return false;
@@ -1432,7 +1437,7 @@ int bca_jbeta_fill(bca_ctx* c, const double* jac, const double* jdz, const doubl
 // ------------------------------------------------------------------ batch
 struct bca_batch {
   hipStream_t stream = nullptr;
-  void* scratch = nullptr;  // per-mesh planes of the scalar type
+  void* scratch = nullptr;  // outputs that share memory with an input
   long scratch_bytes = 0;
   void* table = nullptr;    // device copy of the items and the plan
   void* host = nullptr;     // pinned staging of the table
@@ -1454,17 +1459,17 @@ int batch_grow(void** p, long* have, long want, bool pinned) {
   return 0;
 }
 
-template <class T>
+// V: StateView<double>, or PairView with tangents
+template <class V>
 int run_batch(bca_batch* b, const bca_batch_item* items, int n) {
+  constexpr bool tangent = std::is_same<V, PairView>::value;
   if (n < 1 || n > BATCH_MAX) return fail(-1, "batch size must be 1.." + std::to_string(BATCH_MAX));
-  // scratch layout and checks
-  long planes = 0;
   std::vector<Mesh> ms(n);
   for (int k = 0; k < n; ++k) {
     const bca_batch_item& it = items[k];
     if (!it.w || !it.residu || !it.g.nx || !it.g.ny || !it.g.vol || !it.g.volf)
       return fail(-1, "batch item " + std::to_string(k) + ": null argument");
-    if (std::is_same<T, double>::value != (it.wd == nullptr) || (it.wd && !it.residud))
+    if (tangent == (it.wd == nullptr) || (it.wd && !it.residud))
       return fail(-1, "batch items must all carry wd and residud, or none");
     if (it.nops < 0 || it.nops > BATCH_OPS || (it.nops && !it.ops))
       return fail(-1, "batch item " + std::to_string(k) + ": 0.." + std::to_string(BATCH_OPS) + " BC operations");
@@ -1473,11 +1478,27 @@ int run_batch(bca_batch* b, const bca_batch_item* items, int n) {
     if (rc) return rc;
     for (int o = 0; o < it.nops; ++o)
       if ((rc = bc_check(ms[k], it.ops[o], it.g.nx, it.g.ny))) return rc;
-    planes += (5 + NPRIM + NGRAD) * ms[k].ncell + 10 * ms[k].nnode;
   }
-  int rc = batch_grow(&b->scratch, &b->scratch_bytes, planes * (long)sizeof(T), false);
-  if (rc) return rc;
-  const long tbytes = (long)sizeof(BatchItem<T>) * BATCH_MAX + (long)sizeof(BatchPlan);
+  // Every input is read as the call found it: outputs that share memory with an
+  // input go through scratch, and meshes that share a state go one by one.
+  bool through = false, shared = false;
+  long planes = 0;
+  auto meet = [&](const double* a, const Mesh& ma, const double* c, const Mesh& mc) {
+    return a && c && a < c + 5 * mc.ncell && c < a + 5 * ma.ncell;
+  };
+  for (int k = 0; k < n; ++k) {
+    planes += 10 * ms[k].ncell;
+    for (int l = 0; l < n; ++l)
+      for (const double* in : {items[l].w, items[l].wd}) {
+        through = through || meet(items[k].residu, ms[k], in, ms[l]) || (tangent && meet(items[k].residud, ms[k], in, ms[l]));
+        shared = shared || (k < l && (meet(items[k].w, ms[k], in, ms[l]) || meet(items[k].wd, ms[k], in, ms[l])));
+      }
+  }
+  int rc = 0;
+  if (through && (rc = batch_grow(&b->scratch, &b->scratch_bytes, planes * (long)sizeof(double), false))) return rc;
+  // one plan, or one per mesh
+  const int groups = shared ? n : 1, per = shared ? 1 : n;
+  const long tbytes = (long)sizeof(BatchItem) * BATCH_MAX + (long)sizeof(BatchPlan) * BATCH_MAX;
   if (b->pending) {
     BCA_HIP(hipEventSynchronize(b->copied));
     b->pending = false;
@@ -1485,65 +1506,69 @@ int run_batch(bca_batch* b, const bca_batch_item* items, int n) {
   long have = b->table_bytes;
   if ((rc = batch_grow(&b->table, &b->table_bytes, tbytes, false))) return rc;
   if ((rc = batch_grow(&b->host, &have, tbytes, true))) return rc;
-  BatchItem<T>* hi = reinterpret_cast<BatchItem<T>*>(b->host);
-  BatchPlan* plan = reinterpret_cast<BatchPlan*>(hi + BATCH_MAX);
-  std::memset(b->host, 0, tbytes);
-  T* p = reinterpret_cast<T*>(b->scratch);
-  plan->n = n;
-  plan->maxops = 0;
-  for (int k = 0; k < n; ++k) {
-    const bca_batch_item& it = items[k];
-    const Mesh& m = ms[k];
-    BatchItem<T>& d = hi[k];
-    d.m = m;
-    d.ph = to_phys(&it.phys);
-    d.g = to_metric(it.g);
-    d.w = it.w; d.wd = it.wd; d.res = it.residu; d.resd = it.residud;
-    d.ws = p; p += 5 * m.ncell;
-    d.prim = p; p += NPRIM * m.ncell;
-    d.grad = p; p += NGRAD * m.ncell;
-    d.hn = p; p += 10 * m.nnode;
-    d.nops = it.nops;
-    plan->maxops = std::max(plan->maxops, it.nops);
-    for (int o = 0; o < it.nops; ++o) {
-      const bca_bc_op& op = it.ops[o];
-      d.ops[o] = BatchBc{op.kind, op.loc, Box{op.box[0], op.box[1], op.box[2], op.box[3]},
-                         Box{op.box2[0], op.box2[1], op.box2[2], op.box2[3]}, op.tr[0], op.tr[1], op.data, op.lm,
-                         op.gam};
+  BatchItem* hi = reinterpret_cast<BatchItem*>(b->host);
+  BatchPlan* plans = reinterpret_cast<BatchPlan*>(hi + BATCH_MAX);
+  double* p = reinterpret_cast<double*>(b->scratch);
+  std::vector<char> whole(groups, 1);  // every sequence of the group in one launch
+  for (int q = 0; q < groups; ++q) {
+    BatchPlan& plan = plans[q];
+    std::memset(&plan, 0, sizeof(plan));
+    plan.n = per;
+    for (int x = 0; x < per; ++x) {
+      const int k = q * per + x;
+      const bca_batch_item& it = items[k];
+      const Mesh& m = ms[k];
+      BatchItem& d = hi[k];
+      d = BatchItem{};
+      d.m = m;
+      d.ph = res_phys(to_phys(&it.phys));
+      d.g = to_metric(it.g);
+      d.w = it.w, d.wd = it.wd;
+      d.out = d.store = ResOut{it.residu, it.residud};
+      if (through) {
+        d.out = ResOut{p, p + 5 * m.ncell};
+        p += 10 * m.ncell;
+      }
+      d.nops = it.nops;
+      for (int o = 0; o < it.nops; ++o) d.ops[o] = to_seq_op(it.ops[o]);
+      const bool one = it.nops == 0 || bc_sequence_plan(m, it.ops, it.nops, d.seq);
+      whole[q] = whole[q] && one;
+      plan.seq[x + 1] = plan.seq[x] + (it.nops ? d.seq.blocks + 4 : 0);
+      plan.tiles[x + 1] =
+          plan.tiles[x] + ((m.im + TILE_CELLS - 1) / TILE_CELLS) * ((m.jm + TILE_CELLS - 1) / TILE_CELLS);
+      plan.cells[x + 1] = plan.cells[x] + m.im * m.jm;
+      for (int o = 0; o < BATCH_OPS; ++o)
+        plan.bc[o][x + 1] = plan.bc[o][x] + (o < it.nops ? (int)bc_items(it.ops[o]) : 0);
     }
-    plan->cells[k + 1] = plan->cells[k] + m.ncell;
-    plan->interior[k + 1] = plan->interior[k] + (long)m.im * m.jm;
-    plan->edges[k + 1] = plan->edges[k] + m.im + m.jm;
-    plan->faces[k + 1] = plan->faces[k] + (long)(m.im + 1) * (m.jm + 1);
   }
-  for (int o = 0; o < BATCH_OPS; ++o)
-    for (int k = 0; k < n; ++k)
-      plan->bc[o][k + 1] = plan->bc[o][k] + (o < items[k].nops ? bc_items(items[k].ops[o]) : 0);
   BCA_HIP(hipMemcpyAsync(b->table, b->host, tbytes, hipMemcpyHostToDevice, b->stream));
   if (!b->copied) BCA_HIP(hipEventCreateWithFlags(&b->copied, hipEventDisableTiming));
   BCA_HIP(hipEventRecord(b->copied, b->stream));
   b->pending = true;
-  // one launch per stage over all meshes' items
-  const BatchItem<T>* ditems = reinterpret_cast<const BatchItem<T>*>(b->table);
-  const BatchPlan* dplan = reinterpret_cast<const BatchPlan*>(ditems + BATCH_MAX);
+  const BatchItem* ditems = reinterpret_cast<const BatchItem*>(b->table);
+  const BatchPlan* dplans = reinterpret_cast<const BatchPlan*>(ditems + BATCH_MAX);
   hipStream_t s = b->stream;
-  k_batch_stage<T, BS_PACK><<<grid1(plan->cells[n], 256), 256, 0, s>>>(ditems, dplan, 0);
-  BCA_LAUNCHED();
-  for (int o = 0; o < plan->maxops; ++o) {
-    if (plan->bc[o][n] == 0) continue;
-    k_batch_stage<T, BS_BC><<<grid1(plan->bc[o][n], 256), 256, 0, s>>>(ditems, dplan, o);
+  for (int q = 0; q < groups; ++q) {
+    const BatchPlan& plan = plans[q];
+    const BatchItem* di = ditems + q * per;
+    if (whole[q]) {
+      if (plan.seq[per]) k_batch_bc_sequence<V><<<plan.seq[per], BC_SEQ_THREADS, 0, s>>>(di, dplans + q);
+      BCA_LAUNCHED();
+    } else {
+      for (int o = 0; o < BATCH_OPS; ++o) {
+        if (plan.bc[o][per] == 0) continue;
+        k_batch_bc<V><<<grid1(plan.bc[o][per], 256), 256, 0, s>>>(di, dplans + q, o);
+        BCA_LAUNCHED();
+      }
+    }
+    k_batch_residual<V><<<plan.tiles[per], TILE_THREADS, 0, s>>>(di, dplans + q);
     BCA_LAUNCHED();
   }
-  k_batch_stage<T, BS_PRIM><<<grid1(plan->cells[n], 256), 256, 0, s>>>(ditems, dplan, 0);
-  BCA_LAUNCHED();
-  k_batch_stage<T, BS_GRAD><<<grid1(plan->interior[n], 256), 256, 0, s>>>(ditems, dplan, 0);
-  BCA_LAUNCHED();
-  k_batch_stage<T, BS_GHOSTGRAD><<<grid1(plan->edges[n], 256), 256, 0, s>>>(ditems, dplan, 0);
-  BCA_LAUNCHED();
-  k_batch_stage<T, BS_FACE><<<grid1(plan->faces[n], 256), 256, 0, s>>>(ditems, dplan, 0);
-  BCA_LAUNCHED();
-  k_batch_stage<T, BS_BALANCE><<<grid1(plan->cells[n], 256), 256, 0, s>>>(ditems, dplan, 0);
-  BCA_LAUNCHED();
+  if (through)
+    for (int q = 0; q < groups; ++q) {
+      k_batch_store<<<grid1(plans[q].cells[per], 256), 256, 0, s>>>(ditems + q * per, dplans + q);
+      BCA_LAUNCHED();
+    }
   return 0;
 }
 
@@ -1577,8 +1602,8 @@ int bca_batch_destroy(bca_batch* b) {
 
 int bca_batch_residual_jvp(bca_batch* b, const bca_batch_item* items, int n) {
   if (!b || !items) return fail(-1, "null argument");
-  if (n >= 1 && items[0].wd) return run_batch<Dual<1>>(b, items, n);
-  return run_batch<double>(b, items, n);
+  if (n >= 1 && items[0].wd) return run_batch<PairView>(b, items, n);
+  return run_batch<StateView<double>>(b, items, n);
 }
 
 }  // extern "C"

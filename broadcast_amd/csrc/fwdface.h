@@ -53,7 +53,7 @@ __device__ inline void face_linearise(const PlainAcc<double>& a, FaceLin& f) {
 #pragma unroll
   for (int e = 0; e < 5; ++e) {
     const double jp = 0.5 * (a.template W<0, 0>(e) - a.template W<-DX, -DY>(e));
-    const double pr = predictor<5, DX, DY>(a, e);
+    const double pr = predictor<DX, DY>(a, e);
     f.A[e] = ds.eps2 * jp + ds.eps4 * pr;
     f.E[e] = ds.rspec * (jp - act * pr);
   }
@@ -163,7 +163,7 @@ __device__ inline void face_block(const PlainAcc<double>& a, const FaceLin& f, c
   // jump and predictor
   if constexpr (across == 0) {
     const double cj = 0.5 * (ind.template W<0, 0>(0) - ind.template W<-DX, -DY>(0));
-    const double cp = predictor<5, DX, DY>(ind, 0);
+    const double cp = predictor<DX, DY>(ind, 0);
     const double s = f.rspec * (f.eps2 * cj + f.eps4 * cp);
 #pragma unroll
     for (int e = 0; e < 5; ++e) B[e][e] -= s;

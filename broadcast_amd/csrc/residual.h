@@ -20,7 +20,7 @@
 // With the boundary conditions before it: residual 2048 x 1024 625 -> 192 us,
 // 96 x 64 38.6 -> 18.7 us, order 7 on a 383 x 255 O-mesh 80 -> 44 us; tangent on
 // a 509 x 381 O-mesh 93 -> 50 us.  The distance from an 80-bit evaluation is
-// 0.84 to 0.96 of the former kernels' (2-norm; flat plate 96 x 64 and 131 x 67,
+// 0.79 to 0.96 of the former kernels' (2-norm; flat plate 96 x 64 and 131 x 67,
 // O-mesh 28 x 12 and 128 x 90).
 #pragma once
 #include "bcs.h"

@@ -176,39 +176,20 @@ __global__ void k_prim(Mesh m, Phys ph, const T* __restrict__ w, T* __restrict__
 }
 
 // ---------------------------------------------------------------- gradients
-// gradop_5pi/j.F (ORD 5), gradop_3pi/j.F (ORD 3), gradop_7pi/j.F, gradop_9pi/j.F
-// + gradient.F + geom/dxdy.F
-template <int ORD = 5, class T>
+// gradop_5pi/j.F + gradient.F + geom/dxdy.F
+template <class T>
 __device__ inline void gradient_at(const Mesh& m, const Metric& g, const T* prim, int i, int j,
                                    T out[4]) {
   const long n = m.ncell;
   const T* U = prim + P_U * n;
   const T* V = prim + P_V * n;
-  auto di = [&](const T* f) -> T {
-    if constexpr (ORD == 3) return Coef3::b1 * (f[cidx(m, i + 1, j)] - f[cidx(m, i - 1, j)]);
-    else if constexpr (ORD == 5)
-      return Coef::b1 * (f[cidx(m, i + 1, j)] - f[cidx(m, i - 1, j)]) +
-             Coef::b2 * (f[cidx(m, i + 2, j)] - f[cidx(m, i - 2, j)]);
-    else {
-      T acc = CoefHi<ORD>::b(0) * (f[cidx(m, i + 1, j)] - f[cidx(m, i - 1, j)]);
-#pragma unroll
-      for (int n = 1; n < CoefHi<ORD>::NB; ++n)
-        acc = acc + CoefHi<ORD>::b(n) * (f[cidx(m, i + n + 1, j)] - f[cidx(m, i - n - 1, j)]);
-      return acc;
-    }
+  auto di = [&](const T* f) {
+    return Coef::b1 * (f[cidx(m, i + 1, j)] - f[cidx(m, i - 1, j)]) +
+           Coef::b2 * (f[cidx(m, i + 2, j)] - f[cidx(m, i - 2, j)]);
   };
-  auto dj = [&](const T* f) -> T {
-    if constexpr (ORD == 3) return Coef3::b1 * (f[cidx(m, i, j + 1)] - f[cidx(m, i, j - 1)]);
-    else if constexpr (ORD == 5)
-      return Coef::b1 * (f[cidx(m, i, j + 1)] - f[cidx(m, i, j - 1)]) +
-             Coef::b2 * (f[cidx(m, i, j + 2)] - f[cidx(m, i, j - 2)]);
-    else {
-      T acc = CoefHi<ORD>::b(0) * (f[cidx(m, i, j + 1)] - f[cidx(m, i, j - 1)]);
-#pragma unroll
-      for (int n = 1; n < CoefHi<ORD>::NB; ++n)
-        acc = acc + CoefHi<ORD>::b(n) * (f[cidx(m, i, j + n + 1)] - f[cidx(m, i, j - n - 1)]);
-      return acc;
-    }
+  auto dj = [&](const T* f) {
+    return Coef::b1 * (f[cidx(m, i, j + 1)] - f[cidx(m, i, j - 1)]) +
+           Coef::b2 * (f[cidx(m, i, j + 2)] - f[cidx(m, i, j - 2)]);
   };
   T gui = di(U), gvi = di(V), guj = dj(U), gvj = dj(V);
   const long nn = m.nnode;
@@ -223,13 +204,13 @@ __device__ inline void gradient_at(const Mesh& m, const Metric& g, const T* prim
   out[G_VY] = dym1 * gvi + dym2 * gvj;
 }
 
-template <class T, int ORD = 5>
+template <class T>
 __global__ void k_grad(Mesh m, Metric g, const T* __restrict__ prim, T* __restrict__ grad) {
   const int i = 1 + blockIdx.x * blockDim.x + threadIdx.x;
   const int j = 1 + blockIdx.y * blockDim.y + threadIdx.y;
   if (i > m.im || j > m.jm) return;
   T out[4];
-  gradient_at<ORD>(m, g, prim, i, j, out);
+  gradient_at(m, g, prim, i, j, out);
   const long c = cidx(m, i, j);
 #pragma unroll
   for (int k = 0; k < 4; ++k) grad[c + k * m.ncell] = out[k];
