@@ -214,25 +214,29 @@ struct RowPrefetch {
 // wrapped columns), in the edge launch: every slot from the tables, all
 // mask words in flight at once (this launch has a register budget of its
 // own).
+// mask words that a row's columns (7 per zone, 35 values each) can reach
+__host__ __device__ constexpr int jr_edge_words(int nz) { return (7 * nz * 35 + 63) / 64; }
+
 template <int NZ, int MODE, class PF>
 __device__ inline void jr_row_edge(const double* J, const JcTables<NZ, true>& T, const Zones& z, int r, int i,
                                    int jm, int row, long tr, long nt, int e, const PF& pf, int qr, bool has_cd,
                                    const double* G, long tn, double mini, unsigned long long* masks, int* cnt,
                                    int* indices, double* data, int* changed, int* bad) {
   constexpr int NA = 7 * NZ;
+  constexpr int W = jr_edge_words(NZ);
   const int lane = threadIdx.x % 64;
   const int rot = (i - 1) % 7;
-  double v[CSR_MASK_WORDS];
-  unsigned long long mk[CSR_MASK_WORDS];
+  double v[W];
+  unsigned long long mk[W];
   bool oob = false;
   const double cd = pf.cd(qr);
   // the lane's slots (word w, zone n): window indices first, then every
   // ghost-part load issued at once (from entry 0 where a slot has none, the
   // branch on tn being row-uniform), so that they are in flight together
-  int kks[CSR_MASK_WORDS], ls[CSR_MASK_WORDS][NZ];
-  double gv[CSR_MASK_WORDS][NZ];
+  int kks[W], ls[W][NZ];
+  double gv[W][NZ];
 #pragma unroll
-  for (int w = 0; w < CSR_MASK_WORDS; ++w) {
+  for (int w = 0; w < W; ++w) {
     const int t = w * 64 + lane;
     const int a = t / 35, b = (t / 5) % 7;
     kks[w] = t < NA * 35 ? (int)T.inv_k[b] : -1;
@@ -244,18 +248,18 @@ __device__ inline void jr_row_edge(const double* J, const JcTables<NZ, true>& T,
   }
   if (tn >= 0) {
 #pragma unroll
-    for (int w = 0; w < CSR_MASK_WORDS; ++w) {
+    for (int w = 0; w < W; ++w) {
       const int m5 = (w * 64 + lane) % 5;
 #pragma unroll
       for (int n = 0; n < NZ; ++n) {
         const int l = ls[w][n];
-        const long gi = l >= 0 ? (tn * (NZ * 49) + n * 49 + l * 7 + kks[w]) * 25 + e * 5 + m5 : 0;
+        const long gi = l >= 0 ? ((tn * 5 + e) * (NZ * 49) + n * 49 + l * 7 + kks[w]) * 5 + m5 : 0;
         gv[w][n] = G[gi];
       }
     }
   }
 #pragma unroll
-  for (int w = 0; w < CSR_MASK_WORDS; ++w) {
+  for (int w = 0; w < W; ++w) {
     const int m5 = (w * 64 + lane) % 5;
     const int kk = kks[w];
     double acc = 0.0;
@@ -287,12 +291,12 @@ __device__ inline void jr_row_edge(const double* J, const JcTables<NZ, true>& T,
   bool same = true;
   if constexpr (MODE == JR_REFRESH) {
 #pragma unroll
-    for (int w = 0; w < CSR_MASK_WORDS; ++w) same = (pf.mask(qr, e, w) == mk[w]) & same;
+    for (int w = 0; w < W; ++w) same = (pf.mask(qr, e, w) == mk[w]) & same;
   }
   if (MODE == JR_FILL || (MODE == JR_REFRESH && same)) {
     int pos = pf.start(qr, e);
 #pragma unroll
-    for (int w = 0; w < CSR_MASK_WORDS; ++w) {
+    for (int w = 0; w < W; ++w) {
       if ((mk[w] >> lane) & 1ull) {
         const int p = pos + __popcll(mk[w] & ((1ull << lane) - 1ull));
         if constexpr (MODE == JR_FILL) {
@@ -307,8 +311,9 @@ __device__ inline void jr_row_edge(const double* J, const JcTables<NZ, true>& T,
     int count = 0;
 #pragma unroll
     for (int w = 0; w < CSR_MASK_WORDS; ++w) {
-      count += __popcll(mk[w]);
-      if (lane == w) masks[w * nt + tr] = mk[w];
+      const unsigned long long word = w < W ? mk[w < W ? w : 0] : 0ull;
+      count += __popcll(word);
+      if (lane == w) masks[w * nt + tr] = word;
     }
     if (lane == 0) {
       cnt[row] = count;
@@ -529,7 +534,7 @@ __global__ void __launch_bounds__(EDGE ? JR_EDGE_THREADS : JR_THREADS) k_jac_csr
     if (!any) return;
   }
   const PlainLane pln = plain_lane(j);
-  RowPrefetch<MODE, EDGE ? CSR_MASK_WORDS : JR_PLAIN_WORDS, RPW> pf;
+  RowPrefetch<MODE, EDGE ? jr_edge_words(NZ) : JR_PLAIN_WORDS, RPW> pf;
   pf.load(m, i0, j, wave, NWAVE, masks, indptr, coefdiag);
 
 #pragma unroll 1
