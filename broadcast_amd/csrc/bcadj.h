@@ -8,13 +8,16 @@
 // its gh ghost layers (deeper layers may read the ones before, which the
 // forward-mode line function composes).  So the transpose is formed from the
 // tangent line functions: for each offset d, a unit Dual<5> tangent on the
-// offset-d cell of every line (lines are disjoint), the tangent BC applied,
-// and the ghost tangents contracted with wb(ghosts).  The four offsets are
-// four slots of one seeded array (slot d at ws + d cs, blockIdx.y = d), so a
-// BC takes one seed, one tangent BC and one accumulate launch.
+// offset-d cell of the line, the tangent BC applied, and the ghost tangents
+// contracted with wb(ghosts) as they are formed: a thread per line and offset,
+// nothing of the seeded states in memory.
+//
+// What bounds it: one thread's chain of Dual<5> operations (an inlet line ~10 us).
+// Seeding frames, the BC on them, the contraction and the clearing took four
+// launches per operation: adjoint 1024 x 256 662 -> 491 us, 127 x 93 O-mesh 191 ->
+// 157 us (the flux adjoint included).
 #pragma once
 #include "bcs.h"
-#include "jacobian.h"
 
 namespace bca {
 
@@ -28,69 +31,58 @@ __device__ inline void line_cell(int loc, Box b, int l, int& i, int& j, int& i0,
   j0 = s.j0;
 }
 
-// ws = w as Dual<5> with unit tangents d[e] on variable e of the offset-d
-// cell of every line of the interface, stored as the compact frame the
-// boundary conditions read or write (the ghost frame plus 4 interior layers,
-// StateView<T, true> layout; the offset-d cells, d <= 3, lie in it).
-__global__ void k_adj_seed(Mesh m, const double* __restrict__ w, Dual<5>* __restrict__ wsd, int loc, Box b,
-                           long cs) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const int d = blockIdx.y;
-  Dual<5>* __restrict__ ws = wsd + d * cs;
-  if (t >= frame_count(m, BC_FRAME)) return;
-  int a, bb;
-  frame_cell(m, BC_FRAME, t, a, bb);
-  const long c = a + (long)m.ni * bb, fc = frame_count(m, BC_FRAME);
-  const int i = a - m.gh + 1, j = bb - m.gh + 1;
-  const Side s = decode_side(loc, b.imin, b.jmin, b.imax, b.jmax);
-  const bool on = s.kdir == 1 ? (i == b.imin + d * s.i0 && j >= b.jmin && j <= b.jmax)
-                              : (j == b.jmin + d * s.j0 && i >= b.imin && i <= b.imax);
+// The state with a unit tangent d[e] on variable e of the cell (ci, cj); what a
+// line writes to a ghost is contracted with wb there: acc[q] += d ghost / d w_q wb.
+struct AdjView {
+  using Scalar = Dual<5>;
+  Mesh m;
+  const double* w;
+  const double* wb;
+  int ci, cj;
+  double* acc;
+  __device__ Dual<5> operator()(int i, int j, int e) const {
+    Dual<5> x(w[cidx(m, i, j) + (long)e * m.ncell]);
+    const double one = i == ci && j == cj ? 1.0 : 0.0;
 #pragma unroll
-  for (int e = 0; e < 5; ++e) {
-    Dual<5> x(w[c + e * m.ncell]);
-    if (on) x.d[e] = 1.0;
-    ws[t + e * fc] = x;
+    for (int q = 0; q < 5; ++q) x.d[q] = q == e ? one : 0.0;
+    return x;
   }
-}
+  __device__ void put(int i, int j, int e, const Dual<5>& x) const {
+    const double y = wb[cidx(m, i, j) + (long)e * m.ncell];
+#pragma unroll
+    for (int q = 0; q < 5; ++q) acc[q] += x.d[q] * y;
+  }
+};
 
-// wb(offset-d cell, q) += sum over the line's ghosts g and variables e of
-// d ws(g, e) / d w(offset-d cell, q) * wb(g, e)
-__global__ void k_adj_accumulate(Mesh m, const Dual<5>* __restrict__ wsd, double* __restrict__ wb, int loc, Box b,
-                                 long cs, int lmax) {
-  const int l = 1 + blockIdx.x * blockDim.x + threadIdx.x;
-  const int d = blockIdx.y;
-  const Dual<5>* __restrict__ ws = wsd + d * cs;
-  if (l > lmax) return;
-  int i, j, i0, j0;
-  line_cell(loc, b, l, i, j, i0, j0);
-  const long n = m.ncell, fc = frame_count(m, BC_FRAME);
-  double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  for (int de = 1; de <= m.gh; ++de) {
-    const int ig = i - de * i0, jg = j - de * j0;
-    const long g = cidx(m, ig, jg), gf = frame_index(m, BC_FRAME, ig + m.gh - 1, jg + m.gh - 1);
-#pragma unroll
-    for (int e = 0; e < 5; ++e) {
-      const Dual<5> x = ws[gf + e * fc];
-      const double y = wb[g + e * n];
-#pragma unroll
-      for (int q = 0; q < 5; ++q) acc[q] += x.d[q] * y;
-    }
-  }
-  const long s = cidx(m, i + d * i0, j + d * j0);
-#pragma unroll
-  for (int q = 0; q < 5; ++q) wb[s + q * n] += acc[q];
-}
+constexpr int ADJ_LINES = 64 / ADJ_REACH;  // lines per workgroup (one wave)
 
-__global__ void k_adj_clear_ghosts(Mesh m, double* __restrict__ wb, int loc, Box b, int lmax) {
-  const int l = 1 + blockIdx.x * blockDim.x + threadIdx.x;
-  if (l > lmax) return;
+// One BC operation: wb(offset-d cell, q) += sum over the line's ghosts g and
+// variables e of d ghost(g, e) / d w(offset-d cell, q) wb(g, e), then the line's
+// wb(g) = 0.  A line's offset-d cells and ghosts are its own, so only the lanes
+// of one line have to wait for each other before its ghosts are cleared.
+template <int KIND>
+__global__ void __launch_bounds__(64) k_bc_adjoint(Mesh m, const double* __restrict__ w, double* __restrict__ wb,
+                                                   BcSeqOp q, const double* __restrict__ nx,
+                                                   const double* __restrict__ ny, int lmax) {
+  const int l = 1 + blockIdx.x * ADJ_LINES + threadIdx.x % ADJ_LINES, d = threadIdx.x / ADJ_LINES;
   int i, j, i0, j0;
-  line_cell(loc, b, l, i, j, i0, j0);
-  for (int de = 1; de <= m.gh; ++de) {
-    const long g = cidx(m, i - de * i0, j - de * j0);
+  line_cell(q.loc, q.box, l, i, j, i0, j0);
+  if (l <= lmax) {
+    double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    const AdjView v{m, w, wb, i + d * i0, j + d * j0, acc};
+    if constexpr (KIND == SEQ_INLET) bc_inlet_line(v, q.loc, q.box, q.data, q.lm, nx, ny, q.gam, l);
+    else if constexpr (KIND == SEQ_NOREF) bc_noref_line(v, q.data, q.lm, q.loc, q.box, nx, ny, q.gam, l);
+    else if constexpr (KIND == SEQ_EXTRAP2) bc_extrap2_line(v, q.loc, q.box, 5, l);
+    else bc_wall_line(v, q.loc, q.box, q.gam, l);
+    const long s = cidx(m, i + d * i0, j + d * j0);
 #pragma unroll
-    for (int e = 0; e < 5; ++e) wb[g + e * m.ncell] = 0.0;
+    for (int e = 0; e < 5; ++e) wb[s + e * m.ncell] += acc[e];
   }
+  __syncthreads();
+  if (l <= lmax)
+    for (int de = d + 1; de <= m.gh; de += ADJ_REACH)
+#pragma unroll
+      for (int e = 0; e < 5; ++e) wb[cidx(m, i - de * i0, j - de * j0) + e * m.ncell] = 0.0;
 }
 
 // In-block join (identity transform, disjoint boxes): the copy wb(prr) <-

@@ -107,7 +107,6 @@ struct bca_ctx {
   double* vjpj = nullptr;   // j-faces
   double* jbeta_comp = nullptr;  // J(beta) components on the pattern
   long jbeta_cap = 0;
-  Dual<5>* wadj = nullptr;  // seeded states of the BC adjoints (compact BC frames)
   double* ghostG = nullptr; // ghost part of the fused CSR path, per near row and slot color
   long ghostG_cap = 0;
   CsrRecord csr_rec;        // the last pruned CSR written without the COO (refresh key)
@@ -453,7 +452,6 @@ int bca_ctx_destroy(bca_ctx* c) {
   if (c->jr_mask) (void)hipFree(c->jr_mask);
   if (c->jr_cnt) (void)hipFree(c->jr_cnt);
   if (c->jbeta_comp) (void)hipFree(c->jbeta_comp);
-  if (c->wadj) (void)hipFree(c->wadj);
   if (c->ghostG) (void)hipFree(c->ghostG);
   delete c;
   return 0;
@@ -1627,18 +1625,15 @@ int bca_bc_adjoint(bca_ctx* c, const double* w, double* wb, const bca_bc_op* op,
     return 0;
   }
   if ((rc = frame_check(m, *op))) return rc;
-  // the offsets d = 0..3 in ADJ_REACH slots of wadj, each the compact BC
-  // frame
-  const long cs = 5 * frame_count(m, BC_FRAME);
-  if ((rc = alloc_planes(c, &c->wadj, ADJ_REACH * cs))) return rc;
+  const BcSeqOp q = to_seq_op(*op);
   const int lmax = (int)bc_items(*op);
-  k_adj_seed<<<dim3(grid1(frame_count(m, BC_FRAME), 256), ADJ_REACH), 256, 0, c->stream>>>(m, w, c->wadj, op->loc,
-                                                                                          b, cs);
-  BCA_LAUNCHED();
-  if ((rc = launch_bc<Dual<5>, true>(c, c->wadj, *op, nx, ny, ADJ_REACH, cs))) return rc;
-  k_adj_accumulate<<<dim3(grid1(lmax, 64), ADJ_REACH), 64, 0, c->stream>>>(m, c->wadj, wb, op->loc, b, cs, lmax);
-  BCA_LAUNCHED();
-  k_adj_clear_ghosts<<<grid1(lmax, 64), 64, 0, c->stream>>>(m, wb, op->loc, b, lmax);
+  const unsigned nb = grid1(lmax, ADJ_LINES);
+  switch (q.kind) {
+    case SEQ_INLET: k_bc_adjoint<SEQ_INLET><<<nb, 64, 0, c->stream>>>(m, w, wb, q, nx, ny, lmax); break;
+    case SEQ_NOREF: k_bc_adjoint<SEQ_NOREF><<<nb, 64, 0, c->stream>>>(m, w, wb, q, nx, ny, lmax); break;
+    case SEQ_EXTRAP2: k_bc_adjoint<SEQ_EXTRAP2><<<nb, 64, 0, c->stream>>>(m, w, wb, q, nx, ny, lmax); break;
+    default: k_bc_adjoint<SEQ_WALL><<<nb, 64, 0, c->stream>>>(m, w, wb, q, nx, ny, lmax); break;
+  }
   BCA_LAUNCHED();
   return 0;
 }
