@@ -28,7 +28,8 @@
 //        viscous flux: the cell's coefficient in each linear stencil (found
 //          at compile time by evaluating ivals_o4 / jvals_o4 on an indicator
 //          accessor) times the face-level adjoints;
-//        then the primitives' adjoints through prim_of reversed by hand.
+//     the primitives' adjoints go back to the state through prim_of reversed by
+//     hand once per cell, in the gather.
 // The derivatives are those of the seeded passes (the same Dual
 // conventions at abs / max / sqrt / tanh), summed in another order.
 #pragma once
@@ -344,13 +345,13 @@ __host__ __device__ constexpr double euler_coef(int along) {
   }
 }
 
-// The face adjoint of one face: J = false an
-// i-face (compact viscous flux), true a centred j-face.  hb: the face's
-// adjoint hnb; out: out[(o * 5 + q) * nf + f].
-template <bool J, bool O4, int ROW>
+// The face adjoint of one face: J = false an i-face (O4: compact viscous flux),
+// true a j-face.  hb: the face's adjoint hnb; sink: takes what each stencil cell
+// receives, in the cell's state (wb) and its primitives (pb).
+template <bool J, bool O4, int ROW, class Sink>
 __device__ inline void face_reverse(const Mesh& m, const Phys& ph, const Metric& g, const double* w,
                                     const double* prim, const double* grad, int i, int j, const double hb[5],
-                                    double* out, long nf, long f) {
+                                    const Sink& sink) {
   constexpr int DX = J ? 0 : 1, DY = J ? 1 : 0, D = J ? 1 : 0;
   PlainAcc<double> a;
   a.m = m; a.ph = ph; a.g = g; a.i = i; a.j = j;
@@ -404,9 +405,6 @@ __device__ inline void face_reverse(const Mesh& m, const Phys& ph, const Metric&
     const bool used = k == 2 ? !ext0 || ext1 : k == 1 ? !ext1 || ext0 : k == 0 ? ext0 : ext1;
     gw[k] = used ? grad_weights<(k - 2) * DX, (k - 2) * DY>(a, gbp[k]) : GradW{0.0, 0.0, 0.0, 0.0};
   });
-  const double cvm1 = 1.0 / ph.cv;
-  const double betas = ph.muref * (ph.tref + ph.cs) / (sqrt(ph.tref) * ph.tref);
-
   sfor<0, NOFF>([&](auto O) {
     constexpr int o = decltype(O)::value;
     constexpr int SI = J ? joff_di(o) : ioff_di(o), SJ = J ? joff_dj(o) : ioff_dj(o);
@@ -415,12 +413,6 @@ __device__ inline void face_reverse(const Mesh& m, const Phys& ph, const Metric&
     if constexpr (o >= 22) {
       if (!(J ? joff_live(m, o, j) : ioff_live(m, o, i))) return;
     }
-    // the cell's state and primitives (plain FP64)
-    const long cc = cidx(m, i + SI, j + SJ);
-    double wc[5];
-#pragma unroll
-    for (int q = 0; q < 5; ++q) wc[q] = w[cc + (long)q * m.ncell];
-    const CellPrim pc = cell_prim(ph, cvm1, wc);
     double wb[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     double pb[NPRIM];
 #pragma unroll
@@ -432,8 +424,9 @@ __device__ inline void face_reverse(const Mesh& m, const Phys& ph, const Metric&
       double ae[5];
 #pragma unroll
       for (int e = 0; e < 5; ++e) ae[e] = c * hb[e];
-      const double sv = ae[0] + ae[1] * pc.u + ae[2] * pc.v + ae[3] * pc.ww + ae[4] * pc.h;
-      const double rn = nxf * wc[1] + nyf * wc[2];
+      const double sv = ae[0] + ae[1] * a.template P<SI, SJ>(P_U) + ae[2] * a.template P<SI, SJ>(P_V) +
+                        ae[3] * a.template P<SI, SJ>(P_W) + ae[4] * a.template P<SI, SJ>(P_H);
+      const double rn = nxf * a.template W<SI, SJ>(1) + nyf * a.template W<SI, SJ>(2);
       wb[1] += nxf * sv;
       wb[2] += nyf * sv;
       pb[P_U] += ae[1] * rn;
@@ -491,35 +484,111 @@ __device__ inline void face_reverse(const Mesh& m, const Phys& ph, const Metric&
       pb[P_W] += cm * va.mid[2];
       pb[P_MU] += cm * va.mid[3];
     }
-    prim_reverse(ph, cvm1, betas, wc, pc, pb, wb);
-    double* p = out + (long)o * 5 * nf + f;
-#pragma unroll
-    for (int q = 0; q < 5; ++q) p[q * nf] = wb[q];
+    sink.template put<SI, SJ>(wb, pb);
     // one offset at a time: the scheduler would otherwise hoist every
     // offset's loads to the top, far beyond the register file
     __builtin_amdgcn_sched_barrier(0);
   });
 }
 
-// One thread per face of rows [j0, j1]: J = false i-faces (O4: rows j >= 3, the
-// compact viscous flux; else rows 1, 2), J = true j-faces (ROW 0: rows j >= 4,
-// centred Euler flux; ROW 3, 2: the off-centred rows 3 (compact viscous flux)
-// and 2 (2nd-order)).
+// ---------------------------------------------------------------- tiles
+// A workgroup takes 16 x 16 faces of one family, a wave 16 x 4 of them.  What the
+// stencil cells receive is added up in LDS -- in arrays of the wave's own, where
+// one offset's 64 additions go to 64 cells and the next offset's come after
+// them: no barrier, and an order that does not depend on scheduling -- as the
+// adjoints of 5 state variables and 7 primitives; a cell off the faces' line only
+// receives u, v, w, T.  The waves' arrays are then added up and stored, one array
+// a tile; the gather adds the tiles' up and takes the primitives back to the
+// state, once per cell.
+constexpr int REV = 16, REV_ROWS = 4, REV_WAVES = REV / REV_ROWS;
+template <bool J>
+struct RevTile {
+  // U, V, W, T: all stencil cells; the other 8 (state, P, MU, H): those along the
+  // normal.  Cells (-4 .. 3) along, -2 .. 2 across.
+  static constexpr int W4 = J ? REV + 4 : REV + 7, H4 = J ? REV + 7 : REV + 4;
+  static constexpr int W8 = J ? REV : REV + 7, H8 = J ? REV + 7 : REV;
+  static constexpr int C4 = J ? 2 : 4, R4 = J ? 4 : 2, C8 = J ? 0 : 4, R8 = J ? 4 : 0;  // of the tile's first face
+  static constexpr int N4 = 4 * W4 * H4, N8 = 8 * W8 * H8, N = N4 + N8;
+  // of one wave
+  static constexpr int h4 = J ? REV_ROWS + 7 : REV_ROWS + 4, h8 = J ? REV_ROWS + 7 : REV_ROWS;
+  static constexpr int n4 = 4 * W4 * h4, n8 = 8 * W8 * h8, n = n4 + n8;
+};
+static_assert(RevTile<false>::N == RevTile<true>::N, "one size of tile");
+constexpr int REV_N = RevTile<false>::N;
+
+template <bool J>
+struct RevSink {
+  using R = RevTile<J>;
+  double* a;   // the wave's arrays
+  int tx, ty;  // the face in them
+  __device__ static void add(double* p, double x) { __hip_atomic_fetch_add(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+  template <int SI, int SJ>
+  __device__ void put(const double wb[5], const double pb[NPRIM]) const {
+    double* p = a + (ty + SJ + R::R4) * R::W4 + tx + SI + R::C4;
+    constexpr int s4 = R::W4 * R::h4, s8 = R::W8 * R::h8;
+    add(p, pb[P_U]);
+    add(p + s4, pb[P_V]);
+    add(p + 2 * s4, pb[P_W]);
+    add(p + 3 * s4, pb[P_T]);
+    if constexpr ((J ? SI : SJ) == 0) {
+      double* q = a + R::n4 + (ty + SJ + R::R8) * R::W8 + tx + SI + R::C8;
+#pragma unroll
+      for (int e = 0; e < 5; ++e) add(q + e * s8, wb[e]);
+      add(q + 5 * s8, pb[P_P]);
+      add(q + 6 * s8, pb[P_MU]);
+      add(q + 7 * s8, pb[P_H]);
+    }
+  }
+};
+
+// The faces of rows [j0, j1]: J = false i-faces (O4: rows j >= 3, the compact
+// viscous flux; else rows 1, 2), J = true j-faces (ROW 0: rows j >= 4, centred
+// Euler flux; ROW 3, 2: the off-centred rows 3 (compact viscous flux) and 2
+// (2nd-order)).  out: REV_N values per tile.
+//
+// What bounds it: one wave a SIMD (256 VGPRs and 170 AGPRs; held to 256 in all it
+// spills 0.7 KB and the adjoint takes 432 us in the place of 330).  1024 x 256:
+// i- and j-faces 98 + 93 us, gather 30 us, where 24 x 5 values per face in
+// planes, each taken back to the state (a division and a square root), took
+// 132 + 108 + 131 us.
 template <bool J, bool O4, int ROW>
 __global__ void __launch_bounds__(256) k_face_reverse(Mesh m, Phys ph, Metric g, const double* __restrict__ w,
                                                       const double* __restrict__ prim,
                                                       const double* __restrict__ grad, double* __restrict__ out,
                                                       const double* __restrict__ resb, int j0, int j1) {
+  using R = RevTile<J>;
+  __shared__ double lds[REV_WAVES * R::n];
   int bx, by;
   xcd_block(bx, by);
-  const int i = 1 + bx * (int)blockDim.x + (int)threadIdx.x;
-  const int j = j0 + by * blockDim.y + threadIdx.y;
-  if (i > (J ? m.im : m.im + 1) || j > j1) return;
-  const long nf = J ? (long)m.im * (m.jm + 1) : (long)(m.im + 1) * m.jm;
-  const long f = J ? (i - 1) + (long)m.im * (j - 1) : (i - 1) + (long)(m.im + 1) * (j - 1);
-  double hb[5];
-  face_adjoint(m, resb, i, j, J ? 0 : 1, J ? 1 : 0, hb);
-  face_reverse<J, O4, ROW>(m, ph, g, w, prim, grad, i, j, hb, out, nf, f);
+  const int tid = threadIdx.x, wave = tid / 64, tx = tid % REV, ty = tid / REV % REV_ROWS;
+  const int i = 1 + bx * REV + tx, j = j0 + by * REV + wave * REV_ROWS + ty;
+  double* a = lds + wave * R::n;
+  for (int x = tid % 64; x < R::n; x += 64) a[x] = 0.0;
+  if (i <= (J ? m.im : m.im + 1) && j <= j1) {
+    double hb[5];
+    face_adjoint(m, resb, i, j, J ? 0 : 1, J ? 1 : 0, hb);
+    face_reverse<J, O4, ROW>(m, ph, g, w, prim, grad, i, j, hb, RevSink<J>{a, tx, ty});
+  }
+  __syncthreads();
+  double* o = out + (long)(bx + by * (int)gridDim.x) * REV_N;
+  // the waves' rows of a tile row, in wave order
+  auto sum = [&](int row, int h, int at, int pitch) {
+    double v = 0.0;
+#pragma unroll
+    for (int k = 0; k < REV_WAVES; ++k) {
+      const int r = row - k * REV_ROWS;
+      if (r >= 0 && r < h) v += lds[k * R::n + at + r * pitch];
+    }
+    return v;
+  };
+  for (int x = tid; x < R::N4; x += 256) {
+    const int c = x % R::W4, row = x / R::W4 % R::H4, k = x / (R::W4 * R::H4);
+    o[x] = sum(row, R::h4, k * R::W4 * R::h4 + c, R::W4);
+  }
+  for (int x = tid; x < R::N8; x += 256) {
+    const int c = x % R::W8, row = x / R::W8 % R::H8, k = x / (R::W8 * R::H8);
+    o[R::N4 + x] = sum(row, R::h8, R::n4 + k * R::W8 * R::h8 + c, R::W8);
+  }
 }
 
 }  // namespace bca

@@ -103,8 +103,8 @@ struct bca_ctx {
   int* csr_cnt = nullptr;   // row lengths of the pruned CSR
   int* csr_aux = nullptr;   // scan block sums, then total, error flag, changed flag (CSR_AUX_INTS)
   unsigned long long* csr_mask = nullptr;  // kept masks of the rows in column order
-  double* vjpi = nullptr;   // VJP contributions per face and offset, i-faces
-  double* vjpj = nullptr;   // j-faces
+  double* vjpj = nullptr;   // VJP contributions of the wall faces, per offset
+  double* vjpt = nullptr;   // those of the others, per tile (RevTile)
   double* jbeta_comp = nullptr;  // J(beta) components on the pattern
   long jbeta_cap = 0;
   double* ghostG = nullptr; // ghost part of the fused CSR path, per near row and slot color
@@ -442,7 +442,7 @@ int bca_ctx_destroy(bca_ctx* c) {
   if (c->res_tmp) (void)hipFree(c->res_tmp);
   if (c->norm_part) (void)hipFree(c->norm_part);
   if (c->norm_out) (void)hipFree(c->norm_out);
-  for (double* p : {c->cellx, c->blki, c->blkj, c->ghostT, c->vjpi, c->vjpj})
+  for (double* p : {c->cellx, c->blki, c->blkj, c->ghostT, c->vjpj, c->vjpt})
     if (p) (void)hipFree(p);
   if (c->wcol) (void)hipFree(c->wcol);
   if (c->ghostnz) (void)hipFree(c->ghostnz);
@@ -1166,9 +1166,19 @@ int bca_vjp_dnc5(bca_ctx* c, double* residub, double* wb, const double* w, bca_m
   const Mesh& m = c->m;
   int rc = 0;
   if ((rc = ensure_work(c))) return rc;
-  const long nfi = (long)(m.im + 1) * m.jm, nfj = (long)m.im * (m.jm + 1);
-  if ((rc = alloc_planes(c, &c->vjpi, (long)NOFF * 5 * nfi))) return rc;
-  if ((rc = alloc_planes(c, &c->vjpj, (long)NOFF * 5 * nfj))) return rc;
+  if ((rc = alloc_planes(c, &c->vjpj, (long)NOFF * 5 * m.im * (m.jm + 1)))) return rc;
+  // the tiles of the five launches, one after the other
+  auto tiles = [](int n) { return (n + REV - 1) / REV; };
+  RevSets sets{{{nullptr, 3, tiles(m.im + 1), tiles(m.jm - 2)}, {nullptr, 1, tiles(m.im + 1), 1}},
+               {{nullptr, 4, tiles(m.im), tiles(m.jm - 2)}, {nullptr, 3, tiles(m.im), 1}, {nullptr, 2, tiles(m.im), 1}}};
+  long total = 0;
+  for (const RevSet* q : {&sets.i[0], &sets.i[1], &sets.j[0], &sets.j[1], &sets.j[2]}) total += rev_doubles(*q);
+  if ((rc = alloc_planes(c, &c->vjpt, total))) return rc;
+  double* part = c->vjpt;
+  for (RevSet* q : {&sets.i[0], &sets.i[1], &sets.j[0], &sets.j[1], &sets.j[2]}) {
+    q->part = part;
+    part += rev_doubles(*q);
+  }
   const Metric gm = to_metric(g);
   const Phys ph = to_phys(p);
   hipStream_t s = c->stream;
@@ -1180,37 +1190,35 @@ int bca_vjp_dnc5(bca_ctx* c, double* residub, double* wb, const double* w, bca_m
   BCA_LAUNCHED();
   k_grad_ghost<double><<<grid1(2 * m.im + m.jm, 256), 256, 0, s>>>(m, c->w0.grad);
   BCA_LAUNCHED();
-  // edge rows on the side streams while the interior runs (disjoint face
-  // rows of vjpi / vjpj; residub is only read until the join); the interior
-  // kernels are queued first, so that a side stream sharing a hardware
-  // queue with c->stream does not hold them back
+  // edge rows on the side streams while the interior runs (tiles of their
+  // own; residub is only read until the join); the interior kernels are queued
+  // first, so that a side stream sharing a hardware queue with c->stream does
+  // not hold them back
   hipStream_t es[3];
   if ((rc = edge_fork(c, es))) return rc;
-  BlockArgs ai{m, ph, gm, w, c->w0.prim, c->w0.grad, c->vjpi, residub, 3, m.jm, nullptr};
+  auto args = [&](const RevSet& q, int j1) {
+    return BlockArgs{m, ph, gm, w, c->w0.prim, c->w0.grad, const_cast<double*>(q.part), residub, q.j0, j1, nullptr};
+  };
+  auto grid = [](const RevSet& q) { return dim3(q.nbx, q.nby); };
   {
     Timed t(c, "k_iface_vjp");
-    launch_iface_vjp_rev(grid2(m.im + 1, m.jm - 2, b), b, s, ai);
+    launch_iface_vjp_rev(grid(sets.i[0]), 256, s, args(sets.i[0], m.jm));
   }
-  BlockArgs aj{m, ph, gm, w, c->w0.prim, c->w0.grad, c->vjpj, residub, 4, m.jm + 1, nullptr};
   {
     Timed t(c, "k_jface_vjp");
-    launch_jface_vjp_rev(grid2(m.im, m.jm - 2, b), b, s, aj);
+    launch_jface_vjp_rev(grid(sets.j[0]), 256, s, args(sets.j[0], m.jm + 1));
   }
   BCA_LAUNCHED();
-  BlockArgs ae{m, ph, gm, w, c->w0.prim, c->w0.grad, c->vjpi, residub, 1, 2, nullptr};
-  launch_iface_vjp_rev_o2(grid2(m.im + 1, 2, b), b, es[0], ae);
-  ae.out = c->vjpj;
-  ae.j0 = ae.j1 = 3;
-  launch_jface_vjp_rev_r3(grid2(m.im, 1, b), b, es[1], ae);
-  ae.j0 = ae.j1 = 2;
-  launch_jface_vjp_rev_r2(grid2(m.im, 1, b), b, es[2], ae);
-  ae.j0 = ae.j1 = 1;
+  launch_iface_vjp_rev_o2(grid(sets.i[1]), 256, es[0], args(sets.i[1], 2));
+  launch_jface_vjp_rev_r3(grid(sets.j[1]), 256, es[1], args(sets.j[1], 3));
+  launch_jface_vjp_rev_r2(grid(sets.j[2]), 256, es[2], args(sets.j[2], 2));
+  BlockArgs ae{m, ph, gm, w, c->w0.prim, c->w0.grad, c->vjpj, residub, 1, 1, nullptr};
   launch_jface_vjp_wall(grid2(m.im, 1, b), b, es[0], ae);
   BCA_LAUNCHED();
   if ((rc = edge_join(c, es))) return rc;
   {
     Timed t(c, "k_vjp_gather");
-    k_vjp_gather<<<grid2(m.ni, m.nj, b), b, 0, s>>>(m, c->vjpi, c->vjpj, wb);
+    k_vjp_gather<<<grid2(m.ni, m.nj, b), b, 0, s>>>(m, ph, w, sets, c->vjpj, wb);
   }
   BCA_LAUNCHED();
   k_zero_interior<<<grid2(m.im, m.jm, b), b, 0, s>>>(m, residub);
