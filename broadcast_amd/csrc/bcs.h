@@ -457,9 +457,14 @@ __device__ inline void bc_seq_line(const V& w, const BcSeqOp& q, const double* n
   }
 }
 
-// workgroup `block` of seq.blocks + 4, BC_SEQ_THREADS threads
-template <class V>
-__device__ inline void bc_sequence(const V& w, const BcSeq& seq, const double* nx, const double* ny, int block) {
+// Workgroup `block` of seq.blocks + 4, BC_SEQ_THREADS threads.  live(q, t, col):
+// does the line away from the corners have to be done (k_ghost_sequence)?
+struct EveryLine {
+  __device__ bool operator()(const BcSeqOp&, int, int) const { return true; }
+};
+template <class V, class Live = EveryLine>
+__device__ inline void bc_sequence(const V& w, const BcSeq& seq, const double* nx, const double* ny, int block,
+                                   const Live& live = Live()) {
   const int tid = threadIdx.x;
   const Mesh& m = w.m;
   if (block < seq.blocks) {
@@ -468,7 +473,7 @@ __device__ inline void bc_sequence(const V& w, const BcSeq& seq, const double* n
     const BcSeqOp& q = seq.op[k];
     const int x = (block - q.first) * BC_SEQ_THREADS + tid, wd = bc_seq_width(q);
     const int t = q.lo + x / wd;
-    if (t <= q.hi) bc_seq_line(w, q, nx, ny, t, x % wd);
+    if (t <= q.hi && live(q, t, x % wd)) bc_seq_line(w, q, nx, ny, t, x % wd);
     return;
   }
   const int c = block - seq.blocks, is = c % 2, js = c / 2;

@@ -99,7 +99,9 @@ struct bca_ctx {
   double* ghostT = nullptr; // ghost tangents per zone and color
   Dual<5>* wcol = nullptr;  // seeded states of the zones x 49 colors (compact BC frames)
   unsigned char* ghostnz = nullptr;  // nonzero flags of the ghost tangents
-  int zone_cap = 0;         // number of zones the three arrays above hold
+  double* ghostv = nullptr; // values of the ghosts under the BC sequence
+  int zone_cap = 0;         // number of zones ghostT and ghostnz hold
+  int wcol_cap = 0;         // and wcol
   int* csr_cnt = nullptr;   // row lengths of the pruned CSR
   int* csr_aux = nullptr;   // scan block sums, then total, error flag, changed flag (CSR_AUX_INTS)
   unsigned long long* csr_mask = nullptr;  // kept masks of the rows in column order
@@ -442,7 +444,7 @@ int bca_ctx_destroy(bca_ctx* c) {
   if (c->res_tmp) (void)hipFree(c->res_tmp);
   if (c->norm_part) (void)hipFree(c->norm_part);
   if (c->norm_out) (void)hipFree(c->norm_out);
-  for (double* p : {c->cellx, c->blki, c->blkj, c->ghostT, c->vjpj, c->vjpt})
+  for (double* p : {c->cellx, c->blki, c->blkj, c->ghostT, c->ghostv, c->vjpj, c->vjpt})
     if (p) (void)hipFree(p);
   if (c->wcol) (void)hipFree(c->wcol);
   if (c->ghostnz) (void)hipFree(c->ghostnz);
@@ -963,16 +965,29 @@ int ghost_tangents(bca_ctx* c, const double* w, const bca_metrics& g, const bca_
   const long ng = ghost_count(m);
   int rc = 0;
   if (c->zone_cap < z.n) {
-    c->bytes -= (long)c->zone_cap * ncol *
-                (ng * 25 * (long)sizeof(double) + 5 * frame_count(m, BC_FRAME) * (long)sizeof(Dual<5>) + ng);
+    c->bytes -= (long)c->zone_cap * ncol * (ng * 25 * (long)sizeof(double) + ng);
     if ((rc = realloc_planes(c, &c->ghostT, (long)nslot * ng * 25))) return rc;
-    if ((rc = realloc_planes(c, &c->wcol, (long)nslot * 5 * frame_count(m, BC_FRAME)))) return rc;
     if ((rc = realloc_planes(c, &c->ghostnz, (long)nslot * ng))) return rc;
     c->zone_cap = z.n;
   }
   hipStream_t s = c->stream;
   Timed t(c, "ghost_tangents");
+  BcSeq seq;
+  if (bc_sequence_plan(m, ops, nops, seq)) {
+    if ((rc = alloc_planes(c, &c->ghostv, 5 * ng))) return rc;
+    k_ghost_reset<<<grid1(5 * ng, 256), 256, 0, s>>>(m, w, nslot, c->ghostv, c->ghostnz);
+    BCA_LAUNCHED();
+    k_ghost_sequence<<<dim3(seq.blocks + 4, nslot), BC_SEQ_THREADS, 0, s>>>(m, z, w, seq, g.nx, g.ny, c->ghostv,
+                                                                         c->ghostT, c->ghostnz);
+    BCA_LAUNCHED();
+    return 0;
+  }
   const long cs = 5 * frame_count(m, BC_FRAME);
+  if (c->wcol_cap < z.n) {
+    c->bytes -= (long)c->wcol_cap * ncol * cs * (long)sizeof(Dual<5>);
+    if ((rc = realloc_planes(c, &c->wcol, nslot * cs))) return rc;
+    c->wcol_cap = z.n;
+  }
   k_seed_frames<<<dim3(grid1(frame_count(m, BC_FRAME), 256), nslot), 256, 0, s>>>(m, z, w, c->wcol, cs);
   BCA_LAUNCHED();
   for (int q = 0; q < nops; ++q)

@@ -119,6 +119,93 @@ __global__ void k_ghost_tangents(Mesh m, const Dual<5>* __restrict__ ws, long cs
   nz[(long)color * ng + g] = any ? 1 : 0;
 }
 
+// The seeded state of one zone and color as the BC lines read it (interior cells
+// from w, the seed as they are read) and what they write to the ghosts, straight
+// in T and nz; the ghosts' values, the same for every seed, in gv (ghost_index
+// order, 5 planes).
+struct SeedView {
+  using Scalar = Dual<5>;
+  Mesh m;
+  const double* w;
+  int l, k, lo, hi;  // color, the zone's columns
+  double* gv;
+  double* T;
+  unsigned char* nz;
+  long ng;
+  __device__ bool on(int i, int j) const {
+    const int step = 2 * m.gh + 1;
+    return i >= lo + l && i <= hi && j >= k + 1 && j <= m.jm && (i - lo - l) % step == 0 && (j - k - 1) % step == 0;
+  }
+  __device__ bool inside(int i, int j) const { return i >= 1 && i <= m.im && j >= 1 && j <= m.jm; }
+  __device__ Dual<5> operator()(int i, int j, int e) const {
+    if (inside(i, j)) {
+      Dual<5> x(w[cidx(m, i, j) + (long)e * m.ncell]);
+      const double one = on(i, j) ? 1.0 : 0.0;
+#pragma unroll
+      for (int q = 0; q < 5; ++q) x.d[q] = q == e ? one : 0.0;
+      return x;
+    }
+    const long g = ghost_index(m, i + m.gh - 1, j + m.gh - 1);
+    Dual<5> x(gv[g + e * ng]);
+    if (nz[g])
+#pragma unroll
+      for (int q = 0; q < 5; ++q) x.d[q] = T[g * 25 + e * 5 + q];
+    return x;
+  }
+  __device__ void put(int i, int j, int e, const Dual<5>& x) const {
+    const long g = ghost_index(m, i + m.gh - 1, j + m.gh - 1);
+    gv[g + e * ng] = x.v;
+    bool any = false;
+#pragma unroll
+    for (int q = 0; q < 5; ++q) {
+      T[g * 25 + e * 5 + q] = x.d[q];
+      any = any || x.d[q] != 0.0;
+    }
+    if (any) nz[g] = 1;
+  }
+  // does a line away from the corners read a seeded cell?
+  __device__ bool operator()(const BcSeqOp& q, int t, int col) const {
+    if (q.kind == SEQ_JOIN) return on(q.box2.imin + col, t + q.box2.jmin - q.box.jmin);
+    bool any = false;
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+      any = any || (q.loc < 2 ? on(q.box.imin + (q.loc == 0 ? d : -d), t) : on(t, q.box.jmin + (q.loc == 2 ? d : -d)));
+    return any;
+  }
+};
+
+// nz = 0 for every slot, and the ghosts' values as w holds them (a ghost that no
+// operation fills keeps its own)
+__global__ void k_ghost_reset(Mesh m, const double* __restrict__ w, int nslot, double* __restrict__ gv,
+                              unsigned char* __restrict__ nz) {
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x, ng = ghost_count(m);
+  if (t < 5 * ng) {
+    int a, b;
+    frame_cell(m, m.gh, t % ng, a, b);
+    gv[t] = w[a + (long)m.ni * b + t / ng * m.ncell];
+  }
+  for (long x = t; x < nslot * ng; x += (long)gridDim.x * blockDim.x) nz[x] = 0;
+}
+
+// The ghost tangents of a sequence that goes in one launch (bc_sequence_plan):
+// T and nz of every zone and color (blockIdx.y).  Only 4 of 49 colors seed a cell
+// that a line reads: the others' lines end at once, their nz stays 0 (T is read
+// where nz is set).  What bounds it: the chain of a corner's lines.  All seeds'
+// frames seeded, conditioned and copied, in a launch per operation and two more:
+// 640 us beside the face blocks of 512 x 384 in two zones, now 112 + 52 us (three
+// Newton Jacobians 11.85 -> 10.9 ms); 131 x 67 97 -> 39 us.
+__global__ void __launch_bounds__(BC_SEQ_THREADS) k_ghost_sequence(Mesh m, Zones z, const double* __restrict__ w,
+                                                                   BcSeq seq, const double* __restrict__ nx,
+                                                                   const double* __restrict__ ny, double* gv,
+                                                                   double* T, unsigned char* nz) {
+  const int step = 2 * m.gh + 1, ncol = step * step;
+  const int color = blockIdx.y % ncol, zn = blockIdx.y / ncol;
+  const long ng = ghost_count(m);
+  const SeedView v{m, w, color / step, color % step, z.lo[zn], z.hi[zn],
+                   gv, T + (long)blockIdx.y * ng * 25, nz + (long)blockIdx.y * ng, ng};
+  bc_sequence(v, seq, nx, ny, blockIdx.x, v);
+}
+
 // ------------------------------------------------------------------ phase 2
 __device__ inline bool interior(const Mesh& m, int i, int j) {
   return i >= 1 && i <= m.im && j >= 1 && j <= m.jm;
