@@ -1374,12 +1374,13 @@ int bca_dz_colored(bca_ctx* c, const double* w, bca_metrics g, const bca_phys* p
   rc = ghost_tangents(c, w, g, ops, nops, z);
   if (rc) return rc;
   const dim3 b(64, 4);
-  dim3 gr = grid2(m.im, m.jm, b);
-  gr.z = step * step;
   {
     Timed t(c, "k_dz_colored");
-    k_dz_colored<<<gr, b, 0, c->stream>>>(m, to_phys(p), to_metric(g), w, c->ghostT, c->ghostnz, jdz, jdz2, ia, ja,
-                                          write_index);
+    k_dz_colored_edge<<<dim3(grid1(dz_edge_count(m), 256), step * step), 256, 0, c->stream>>>(
+        m, to_phys(p), to_metric(g), w, c->ghostT, c->ghostnz, jdz, jdz2, ia, ja, write_index);
+    dim3 gr = grid2(m.im - 2 * DZ_EDGE, m.jm - 2 * DZ_EDGE, b);
+    gr.z = step;
+    k_dz_colored<<<gr, b, 0, c->stream>>>(m, to_phys(p), to_metric(g), w, jdz, jdz2, ia, ja, write_index);
   }
   BCA_LAUNCHED();
   return 0;

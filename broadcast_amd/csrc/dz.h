@@ -316,16 +316,33 @@ struct ColorTangent {
   }
 };
 
-// Grid (x: i, y: j, z: color).  ia/ja are those of both operators.
-__global__ void __launch_bounds__(256) k_dz_colored(Mesh m, Phys ph, Metric g, const double* __restrict__ w,
+// The cells whose cross reaches a ghost: DZ_EDGE from an edge (im, jm >= 5).
+constexpr int DZ_EDGE = 2;
+__host__ __device__ inline long dz_edge_count(const Mesh& m) {
+  return (long)m.im * m.jm - (long)(m.im - 2 * DZ_EDGE) * (m.jm - 2 * DZ_EDGE);
+}
+__device__ inline void dz_edge_cell(const Mesh& m, long t, int& i, int& j) {
+  const long rows = (long)DZ_EDGE * m.im;
+  if (t < rows) { i = 1 + (int)(t % m.im), j = 1 + (int)(t / m.im); return; }
+  t -= rows;
+  if (t < rows) { i = 1 + (int)(t % m.im), j = m.jm - DZ_EDGE + 1 + (int)(t / m.im); return; }
+  t -= rows;
+  j = DZ_EDGE + 1 + (int)(t / (2 * DZ_EDGE));
+  const int q = (int)(t % (2 * DZ_EDGE));
+  i = q < DZ_EDGE ? 1 + q : m.im - 2 * DZ_EDGE + 1 + q;
+}
+
+// Those cells, grid (x: cells, y: color).  ia/ja are those of both operators.
+__global__ void __launch_bounds__(256) k_dz_colored_edge(Mesh m, Phys ph, Metric g, const double* __restrict__ w,
                                                     const double* __restrict__ T,
                                                     const unsigned char* __restrict__ nz,
                                                     double* __restrict__ jdz, double* __restrict__ jdz2,
                                                     int* __restrict__ ia, int* __restrict__ ja, int write_index) {
-  const int i = 1 + blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = 1 + blockIdx.y * blockDim.y + threadIdx.y;
-  const int color = blockIdx.z;
-  if (i > m.im || j > m.jm) return;
+  const long cell = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int color = blockIdx.y;
+  if (cell >= dz_edge_count(m)) return;
+  int i, j;
+  dz_edge_cell(m, cell, i, j);
   const int im = m.im, jm = m.jm, gh = m.gh, step = 2 * gh + 1;
   const int l = color / step, k = color % step;
   const long ng = ghost_count(m);
@@ -367,6 +384,129 @@ __global__ void __launch_bounds__(256) k_dz_colored(Mesh m, Phys ph, Metric g, c
       if (write_index) {
         ia[cur] = ok ? row : 5 * im * jm - 1;
         ja[cur] = ok ? mm + valj * 5 + vali * jm * 5 : 0;
+      }
+    }
+  }
+}
+
+// The other cells: their cross is interior, so a color's 5 columns are one cell's
+// block of the cross or zero.  Grid (x, y: the inner cells, z: k): k decides the
+// row dj of the color's cell for a whole wave, the colors l = 0 .. 6 follow in the
+// thread.  A neighbour's block is its velocity tangents (3 numbers) times the
+// gradient's weight; the row cell's own is the pointwise terms of dz_cell.
+//
+// What bounds it: the stores (49 x 25 slots of both operators and the indices a
+// cell).  256 x 96: 236 us, and 86 us for the edge cells, where every cell and color
+// ran dz_cell (992 B of scratch; 35 of 49 colors have one in a wave): 755 us.
+__global__ void __launch_bounds__(256) k_dz_colored(Mesh m, Phys ph, Metric g, const double* __restrict__ w,
+                                                    double* __restrict__ jdz, double* __restrict__ jdz2,
+                                                    int* __restrict__ ia, int* __restrict__ ja, int write_index) {
+  const int i = 1 + DZ_EDGE + blockIdx.x * blockDim.x + threadIdx.x;
+  const int j = 1 + DZ_EDGE + blockIdx.y * blockDim.y + threadIdx.y;
+  const int k = blockIdx.z;
+  if (i > m.im - DZ_EDGE || j > m.jm - DZ_EDGE) return;
+  const int im = m.im, jm = m.jm, gh = m.gh, step = 2 * gh + 1;
+  int dj = ((k - (j - 1)) % step + step) % step;
+  if (dj > gh) dj -= step;
+  const long n = m.ncell, c = cidx(m, i, j);
+  const double betas = ph.muref * (ph.tref + ph.cs) / (sqrt(ph.tref) * ph.tref);
+  const double b1 = Coef::b1, b2 = Coef::b2, twothird = 2.0 / 3.0;
+  const DzPrim q0 = dz_prim(m, ph, w, c, betas);
+  const double mu = q0.mu, u = q0.u, v = q0.v, wz = q0.w;
+  const double fmu = betas * (sqrt(q0.t) * q0.t / (ph.s_suth + q0.t));
+  const double volm1 = 1.0 / g.vol[c];
+  const long f0 = nidx(m, i, j);
+  const double dxm1 = 0.5 * (g.nx[f0] + g.nx[f0 + 1]) * volm1;
+  const double dxm2 = 0.5 * (g.nx[f0 + m.nnode] + g.nx[f0 + m.ni + 1 + m.nnode]) * volm1;
+  const double dym1 = 0.5 * (g.ny[f0] + g.ny[f0 + 1]) * volm1;
+  const double dym2 = 0.5 * (g.ny[f0 + m.nnode] + g.ny[f0 + m.ni + 1 + m.nnode]) * volm1;
+  // the row cell's own block: dz_cell with the tangents of its neighbours zero
+  Lin<5> a[5], b[5];
+#pragma unroll
+  for (int e = 0; e < 5; ++e) a[e] = b[e] = td_zero<Lin<5>>();
+  if (dj == 0) {
+    Lin<5> one[5];
+#pragma unroll
+    for (int q = 0; q < 5; ++q)
+#pragma unroll
+      for (int x = 0; x < 5; ++x) one[q].d[x] = q == x ? 1.0 : 0.0;
+    const DzTan<Lin<5>> t0 = dz_tan<Lin<5>>(ph, q0, w, c, n, one, true, betas);
+    double pi[4][4], pj[4][4];  // u, v, w, mu of the cross
+    const int off[4] = {-1, 1, -2, 2};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const DzPrim x = dz_prim(m, ph, w, c + off[s], betas), y = dz_prim(m, ph, w, c + (long)off[s] * m.ni, betas);
+      pi[0][s] = x.u, pi[1][s] = x.v, pi[2][s] = x.w, pi[3][s] = x.mu;
+      pj[0][s] = y.u, pj[1][s] = y.v, pj[2][s] = y.w, pj[3][s] = y.mu;
+    }
+    auto g4 = [&](const double* p) { return b1 * (p[1] - p[0]) + b2 * (p[3] - p[2]); };
+    double g1[4], g2[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const double gi = g4(pi[q]), gj = g4(pj[q]);
+      g1[q] = dxm1 * gi + dxm2 * gj;
+      g2[q] = dym1 * gi + dym2 * gj;
+    }
+    const double gu1 = g1[0], gw1 = g1[2], gm1 = g1[3], gv2 = g2[1], gw2 = g2[2], gm2 = g2[3];
+    const double s12 = gu1 + gv2, cpprandtl = ph.cp / ph.prandtl;
+    b[1] = -mu * t0.ud;
+    b[2] = -mu * t0.vd;
+    b[3] = -(2.0 * twothird * mu) * t0.wd;
+    b[4] = (-mu * cpprandtl) * t0.td + (-mu * u) * t0.ud + (-mu * v) * t0.vd + (-(2.0 * twothird * mu * wz)) * t0.wd;
+    a[0] = one[3];
+    a[1] = wz * one[1] + w[c + n] * t0.wd - gw1 * t0.mud + (twothird * gm1) * t0.wd;
+    a[2] = wz * one[2] + w[c + 2 * n] * t0.wd - gw2 * t0.mud + (twothird * gm2) * t0.wd;
+    a[3] = wz * one[3] + w[c + 3 * n] * t0.wd + t0.pd + (twothird * s12) * t0.mud + (-gm1) * t0.ud + (-gm2) * t0.vd;
+    a[4] = wz * (one[4] + t0.pd) + (w[c + 4 * n] + q0.p) * t0.wd + (twothird * (gm1 * u + mu * gu1)) * t0.wd +
+           (-(gm1 * wz + mu * gw1)) * t0.ud + (twothird * (gm2 * v + mu * gv2)) * t0.wd +
+           (-(gm2 * wz + mu * gw2)) * t0.vd + (-mu * gw1) * t0.ud + (-u * gw1) * t0.mud + (-mu * gw2) * t0.vd +
+           (-v * gw2) * t0.mud + (twothird * mu * s12) * t0.wd + (twothird * wz * s12) * t0.mud;
+  }
+  const long plane = (long)im * jm;
+#pragma unroll 1
+  for (int l = 0; l < step; ++l) {
+    int di = ((l - (i - 1)) % step + step) % step;
+    if (di > gh) di -= step;
+    const bool own = di == 0 && dj == 0;
+    const bool near = (dj == 0 && di != 0 && di >= -2 && di <= 2) || (di == 0 && dj != 0 && dj >= -2 && dj <= 2);
+    // block of the neighbour (columns 0 .. 3; column 4 is zero)
+    double x1[4], x2[4], x3[4], x4[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) x1[q] = x2[q] = x3[q] = x4[q] = 0.0;
+    if (near) {
+      const int d = dj == 0 ? di : dj;
+      const double gw = d == 1 ? b1 : d == -1 ? -b1 : d == 2 ? b2 : -b2;
+      const double cx = (dj == 0 ? dxm1 : dxm2) * gw, cy = (dj == 0 ? dym1 : dym2) * gw;
+      const long cc = c + di + (long)dj * m.ni;
+      const double ro = w[cc], r1 = 1.0 / ro, r2 = -(1.0 / (ro * ro));
+      const double ud0 = w[cc + n] * r2, vd0 = w[cc + 2 * n] * r2, wd0 = w[cc + 3 * n] * r2;
+      // gud1 = cx ud, gvd2 = cy vd, ...
+      const double k1 = (twothird * mu - fmu) * cx, k2 = (twothird * mu - fmu) * cy;  // of wd in rows 1, 2
+      const double k3 = twothird * fmu - mu;                                            // of ud cx + vd cy in row 3
+      const double k4 = twothird * mu * wz - mu * wz;                                   // and in row 4
+      const double kw = u * k1 + v * k2;                                                // of wd in row 4
+      x1[0] = k1 * wd0, x1[3] = k1 * r1;
+      x2[0] = k2 * wd0, x2[3] = k2 * r1;
+      const double e0 = cx * ud0 + cy * vd0, e1 = cx * r1, e2 = cy * r1;
+      x3[0] = k3 * e0, x3[1] = k3 * e1, x3[2] = k3 * e2;
+      x4[0] = k4 * e0 + kw * wd0, x4[1] = k4 * e1, x4[2] = k4 * e2, x4[3] = kw * r1;
+    }
+    int vali, valj;
+    const bool ok = seed_column_dz(i, j, l, k, gh, im, jm, vali, valj);
+    const long base = (long)(i - 1) + (long)(j - 1) * im + (long)k * plane * 5 + (long)l * plane * 5 * step;
+#pragma unroll
+    for (int e = 0; e < 5; ++e) {
+      const int row = e + (j - 1) * 5 + (i - 1) * jm * 5;
+#pragma unroll
+      for (int mm = 0; mm < 5; ++mm) {
+        const long cur = base + (long)e * plane + (long)mm * plane * 5 * step * step;
+        const double x = mm == 4 || e == 0 ? 0.0 : e == 1 ? x1[mm & 3] : e == 2 ? x2[mm & 3] : e == 3 ? x3[mm & 3] : x4[mm & 3];
+        if (jdz) jdz[cur] = ok ? (own ? a[e].d[mm] : x) : 0.0;
+        if (jdz2) jdz2[cur] = ok && own ? b[e].d[mm] : 0.0;
+        if (write_index) {
+          ia[cur] = ok ? row : 5 * im * jm - 1;
+          ja[cur] = ok ? mm + valj * 5 + vali * jm * 5 : 0;
+        }
       }
     }
   }
