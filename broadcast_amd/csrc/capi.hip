@@ -1667,6 +1667,13 @@ int bca_bc_adjoint(bca_ctx* c, const double* w, double* wb, const bca_bc_op* op,
 // ------------------------------------------------------------------ fused colored Jacobian -> CSR
 namespace {
 
+// Edge tiles up to which a workgroup takes one variable row of its tile in the
+// place of five: a small mesh's tiles are all resident at once, so the pass takes
+// as long as one workgroup's chain; above, each row forming the tables again
+// costs more.  A full CSR with 32 tiles 438 -> 378 us, 276 (two zones) 576 -> 526,
+// 318 495 -> 474; with 632 848 -> 890 (two zones 1115 -> 1097), 960 1478 -> 1631.
+constexpr unsigned EDGE_SPLIT = 400;
+
 // The pruned CSR of the colored Jacobian without the COO (k_jac_csr_rows).
 // refresh: when the context's record says indptr / indices hold the CSR of an
 // earlier call with the same zones and mini, one row pass checks every row's
@@ -1723,6 +1730,8 @@ int jac_csr(bca_ctx* c, const double* w, bca_metrics g, const bca_phys* p, const
   k_fill_int<<<1, 64, 0, s>>>(bad, 2, 0);
   BCA_LAUNCHED();
   const dim3 gr((m.im + JC_TI - 1) / JC_TI, m.jm);
+  const unsigned nedge = (unsigned)jr_edge_tiles(gr.x, m.jm);
+  const dim3 ge(nedge, nedge <= EDGE_SPLIT ? 5 : 1);
   auto rows_pass = [&](int mode, const char* name) -> int {
     Timed t(c, name);
 #define BCA_ROWS(NZ, MODE)                                                                                     \
@@ -1730,7 +1739,7 @@ int jac_csr(bca_ctx* c, const double* w, bca_metrics g, const bca_phys* p, const
     k_jac_csr_rows<NZ, MODE, false><<<gr, JR_THREADS, 0, s>>>(m, z, c->blki, c->blkj, coefdiag, c->ghostG,    \
                                                               mini, c->jr_mask, c->jr_cnt, indptr, indices,   \
                                                               data, changed, bad);                            \
-    k_jac_csr_rows<NZ, MODE, true><<<(unsigned)jr_edge_tiles(gr.x, m.jm), JR_EDGE_THREADS, 0, s>>>(            \
+    k_jac_csr_rows<NZ, MODE, true><<<ge, JR_EDGE_THREADS, 0, s>>>(                                             \
         m, z, c->blki, c->blkj, coefdiag, c->ghostG, mini, c->jr_mask, c->jr_cnt, indptr, indices, data, changed, \
         bad);                                                                                                  \
   } while (0)

@@ -537,8 +537,10 @@ __global__ void __launch_bounds__(EDGE ? JR_EDGE_THREADS : JR_THREADS) k_jac_csr
   RowPrefetch<MODE, EDGE ? jr_edge_words(NZ) : JR_PLAIN_WORDS, RPW> pf;
   pf.load(m, i0, j, wave, NWAVE, masks, indptr, coefdiag);
 
+  // an edge launch of 5 rows of workgroups takes one variable in each
+  const int e0 = EDGE && gridDim.y == 5 ? blockIdx.y : 0, e1 = EDGE && gridDim.y == 5 ? e0 + 1 : 5;
 #pragma unroll 1
-  for (int e = 0; e < 5; ++e) {
+  for (int e = e0; e < e1; ++e) {
     // J(il, cell, m) of variable row e, each summed in registers in the face
     // order of the COO path; loads from a stand-in offset 0 where a face has
     // no block keep them all in flight, selects keep the sums exact
