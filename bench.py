@@ -233,7 +233,7 @@ def main():
 
     nzones = 1 if f.two_zone_split is None else 2
     nseeds = 245 * nzones
-    # launch shapes of the residual faces, face blocks and assembly for this mesh
+    # launch shapes of the face blocks and the assembly for this mesh
     f.apply_bcs(w)
     tuned = f.autotune(w, jac=bufs[0])
     print(f"bench: autotuned {tuned}", file=sys.stderr, flush=True)
@@ -613,7 +613,7 @@ def vjp_figure(im=1024, jm=256, reps=10):
           file=sys.stderr, flush=True)
     return {"cells": cells, "vjp_ms": ms_v, "mcells_per_s": cells / (ms_v * 1e-3) / 1e6, "achieved_gbs": gbs,
             "frac": gbs / HBM_PEAK_GBS, "vjp_with_bc_adjoints_ms": ms_vb,
-            "workload": "flux adjoint (a reverse sweep per face, the wall row by 24 seeded passes contracted "
+            "workload": "flux adjoint (a reverse sweep per face, the wall row by seeded passes contracted "
                         "with the face adjoint, fixed-order gather); then the BC adjoints in reverse order"}
 
 

@@ -4,7 +4,7 @@ Per mesh the work is the reference's per-iteration sequence -- the BC calls in
 order, then flux_num_dnc5_2d (BROADCAST_npz.py:1018-1031) or, with a tangent,
 the linearised BCs and flux_num_dnc5_2d_d (:1079-1085) -- as ``Flow.residual``
 / ``Flow.jvp`` do one mesh at a time; ``UnevenBatch`` runs all meshes
-together, one launch per stage over the concatenated work of every mesh
+together, two launches over the workgroups of every mesh
 (bca_batch_residual_jvp), so small meshes do not each pay a chain of
 launches on a mostly idle chip.
 """

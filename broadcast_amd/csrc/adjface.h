@@ -1,8 +1,7 @@
 // Reverse-mode face adjoints (the VJP of the DNC5 residual): for every i-face
 // and every j-face above the wall row, hnb(face)^T d hn(face) / d w(cell) for the 24
-// stencil cells, the same 5 values per offset that the seeded passes of
-// k_iface_blocks / k_jface_blocks (MODE_VJP) store, in the same planes, so
-// that k_vjp_gather reads either.  The reference's adjoint is TAPENADE's
+// stencil cells, as adjoints of each cell's state and primitives, added up per
+// tile for k_vjp_gather.  The reference's adjoint is TAPENADE's
 // reverse sweep of the face loop with recomputation
 // (srcfv/adjoint/flux_num_dnc5_b.f90:15-6676); here one thread takes one
 // face:
@@ -12,7 +11,7 @@
 //      gradients and face values;
 //   2. the face-level adjoints: of the Roe spectral radius and eps2 / eps4
 //      (rspec_b = -sum_e hnb_e (eps2 jump_e + eps4 pred_e), ...), and of the
-//      viscous flux by the transposed stress (stress_of reversed by hand,
+//      viscous flux by the transposed stress (reversed by hand,
 //      down to the four staggered values N, S, O, E of u, v, w, T and the
 //      face values of mu, u, v, w);
 //   3. per stencil cell (compile-time offsets), the cell's 5 values, all
@@ -30,7 +29,7 @@
 //          accessor) times the face-level adjoints;
 //     the primitives' adjoints go back to the state through prim_of reversed by
 //     hand once per cell, in the gather.
-// The derivatives are those of the seeded passes (the same Dual
+// The derivatives are those of forward mode (the same Dual
 // conventions at abs / max / sqrt / tanh), summed in another order.
 #pragma once
 #include "blockskern.h"
@@ -107,14 +106,14 @@ __device__ inline ViscPrimal visc_primal(const A& a) {
 
 // Face-level adjoints of the viscous flux: of the staggered values (N, S, O,
 // E) of u, v, w, T and of the face values of u, v, w, mu, from the adjoints
-// fb[e], gb[e] (e = 1..4) of the stress components vis_f<e>, vis_g<e>.
+// fb[e], gb[e] (e = 1..4) of the x- and y-stress components.
 struct ViscAdj {
   double N[4], S[4], O[4], E[4];  // k = P_U, P_V, P_W, P_T
   double mid[4];                  // u, v, w, mu
 };
 __device__ inline ViscAdj visc_reverse(const ViscPrimal& v, const double fb[5], const double gb[5], double cpp) {
   constexpr double tt = Coef::twothird;
-  // stress_of forward, for the products the reverse needs
+  // the stresses, for the products the reverse needs
   const double fv1 = tt * v.mmu * (2.0 * v.ux - v.vy), fv2 = v.mmu * (v.uy + v.vx), fv3 = v.mmu * v.wx;
   const double gv1 = v.mmu * (v.uy + v.vx), gv2 = tt * v.mmu * (-v.ux + 2.0 * v.vy), gv3 = v.mmu * v.wy;
   const double f1b = fb[1] + fb[4] * v.uu, f2b = fb[2] + fb[4] * v.vv, f3b = fb[3] + fb[4] * v.ww;
@@ -143,8 +142,9 @@ __device__ inline ViscAdj visc_reverse(const ViscPrimal& v, const double fb[5], 
   return r;
 }
 
-// The quantities of diss_scalars<DX, DY> (the face between cell 0 and cell
-// -1 = (-DX, -DY)) that its reverse needs, computed as diss_scalars does.
+// The dissipation scalars of a face between cell 0 and cell -1 = (-DX, -DY): the
+// Roe-weighted spectral radius, eps2 and eps4 of the sensor, with what their
+// reverse needs.
 struct DissPrim {
   double rr, rl, ur, vr, ul, vl, c2r, c2l, q, rt, wl, wr, nxf, nyf, n2, un, c2n;
   double rspec, eps2, eps4;
@@ -192,7 +192,7 @@ __device__ inline DissPrim diss_primal(const A& a, int d) {
   return P;
 }
 
-// Adjoints of the inputs of diss_scalars: of W(0..2) and T of cells 0 and
+// Adjoints of the inputs of diss_primal: of W(0..2) and T of cells 0 and
 // -1, of the pressure of cells -2, -1, 0, 1 along the face normal, and of
 // the gradients G of cells 0 and -1; from the adjoints of rspec, eps2 and
 // eps4.  The derivative conventions are Dual's: abs takes + at 0, sqrt has
@@ -371,7 +371,7 @@ __device__ inline void face_reverse(const Mesh& m, const Phys& ph, const Metric&
     e2b -= hb[e] * ds.rspec * jp;
     e4b -= hb[e] * ds.rspec * pr;
   }
-  // viscous: hn_e -= (vis_f<e> nxl + vis_g<e> nyl) sn, e = 1..4
+  // viscous: hn_e -= (f_e nxl + g_e nyl) sn, e = 1..4
   const ViscPrimal vp = visc_primal<J, O4>(a);
   double fb[5], gb[5];
 #pragma unroll
@@ -408,8 +408,7 @@ __device__ inline void face_reverse(const Mesh& m, const Phys& ph, const Metric&
   sfor<0, NOFF>([&](auto O) {
     constexpr int o = decltype(O)::value;
     constexpr int SI = J ? joff_di(o) : ioff_di(o), SJ = J ? joff_dj(o) : ioff_dj(o);
-    // the two extra offsets exist only on the faces the seeded passes store
-    // them for (reached through the extrapolated gradients)
+    // the two extra offsets exist only on the faces that reach them (through the extrapolated gradients)
     if constexpr (o >= 22) {
       if (!(J ? joff_live(m, o, j) : ioff_live(m, o, i))) return;
     }

@@ -7,7 +7,6 @@
 //   abs(x)   : x >= 0 takes the + branch                      (:945-951)
 //   sqrt(x)  : derivative 0 where x == 0                       (:953-957)
 //   max(a,b) : a < b ? b : a                                   (:1054-1074)
-//   tanh     : 1 - tanh^2                                      (:1025-1026)
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -66,12 +65,6 @@ template <int N> __device__ inline Dual<N> dsqrt(const Dual<N>& a) {
   const double s = sqrt(a.v);
   const double g = (a.v == 0.0) ? 0.0 : 0.5 / s;
   BCA_D2(s, a.d[k] * g)
-}
-__device__ inline double dtanh(double a) { return tanh(a); }
-template <int N> __device__ inline Dual<N> dtanh(const Dual<N>& a) {
-  const double t = tanh(a.v);
-  const double g = 1.0 - t * t;
-  BCA_D2(t, a.d[k] * g)
 }
 // x ** e with a real constant exponent
 __device__ inline double dpow(double a, double e) { return pow(a, e); }

@@ -5,7 +5,7 @@
 // hn = Euler - dissipation - viscous depends on a stencil cell through its own
 // Euler flux (a fixed coefficient), through the jump and predictor (fixed
 // coefficients), through the dissipation scalars rspec and eps2 (two gradients
-// of the face, formed once by the reverse of diss_scalars) and through the
+// of the face, formed once by the reverse of diss_primal) and through the
 // linear stencils of the viscous flux (a face gradient weight per direction
 // and a face-value weight).  So after one primal pass of the face a block is a
 // few products of face-level numbers with the cell's d prim / d w:

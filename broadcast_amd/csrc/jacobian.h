@@ -6,12 +6,13 @@
 // misc/ComputeJacobian.f90:357-374, 503-570).  Here the same numbers come from
 // two passes that never evaluate a dense tangent:
 //
-//  phase 1  (k_iface_blocks / k_jface_blocks) every face computes
+//  phase 1  (k_face_blocks) every face computes
 //           B(face, o) = d hn(face) / d w(face + o) for the 24 stencil offsets
-//           o of its family by compile-time sparse forward mode (SeededAcc),
+//           o of its family by hand-derived forward differentiation,
 //           ghost cells included as independent inputs, one plane per offset;
-//  ghosts   (k_seed_frames + linearised BCs + k_ghost_tangents, all 49 colors
-//           per launch) the tangent the BC sequence gives every ghost cell,
+//  ghosts   (k_ghost_sequence, all 49 colors in one launch; a sequence that is
+//           not of its kind by k_seed_frames + linearised BCs +
+//           k_ghost_tangents) the tangent the BC sequence gives every ghost cell,
 //           T(color, g), computed on the boundary frame only;
 //  phase 2  (k_assemble_colored, then k_assemble_ghosts on the rows near the
 //           mesh edge) for every row cell and color, the tangent residual of

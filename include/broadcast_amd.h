@@ -70,9 +70,9 @@ long bca_ctx_scratch_bytes(const bca_ctx *ctx);
 /* Kernel timing with HIP events recorded on the context stream around each
  * pipeline launch (no reference counterpart; the reference times with wall
  * clocks, BROADCAST_npz.py:1003-1007).  enable resets the record; read sums
- * the launches of one kernel, named "k_face<f64>", "k_face<dual1>",
- * "k_face<dual5>", "k_prim<..>", "k_grad<..>", "k_balance<..>",
- * "k_balance_scatter<dual5>". */
+ * the launches of one kernel or stage, named "k_residual<f64>",
+ * "k_residual<dual1>", "k_bc_sequence", "k_iface_blocks", "k_jface_blocks",
+ * "ghost_tangents", "k_ghost_part", "k_jac_csr_refresh", ... */
 int bca_profile_enable(bca_ctx *ctx, int on);
 int bca_profile_read(bca_ctx *ctx, const char *kernel, double *total_ms, long *launches);
 
@@ -96,14 +96,13 @@ int bca_residual_dnc5(bca_ctx *ctx, double *residu, const double *w, bca_metrics
 
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc): the residual of bca_residual_dnc5, same kernels and
- * results, without a context, enqueued on `hip_stream`.  Its scratch planes
- * (prim, grad, hn) live in one static device array of
- * BCA_NOALLOC_SCRATCH_BYTES that each GPU holds until the process ends; the
- * call allocates and frees nothing.  A mesh needing more scratch
- * (bca_residual_noalloc_bytes) is refused with -4 before any launch.  Every
- * call on one GPU shares that GPU's array: calls that overlap on one GPU
- * (two streams, two host threads) race and must be ordered by the caller. */
+ * forbid hipMalloc): the residual of bca_residual_dnc5, same kernel and
+ * results, without a context, enqueued on `hip_stream`; the call allocates and
+ * frees nothing.  A mesh of more than BCA_NOALLOC_SCRATCH_BYTES by
+ * bca_residual_noalloc_bytes is refused with -4 before any launch.  A residu
+ * that shares memory with w goes through one static device array of that size
+ * that each GPU holds until the process ends: such calls must not overlap on one
+ * GPU (two streams, two host threads); others may. */
 #define BCA_NOALLOC_SCRATCH_BYTES (64L * 1024L * 1024L)
 long bca_residual_noalloc_bytes(int im, int jm, int gh);
 int bca_residual_dnc5_noalloc(double *residu, const double *w, bca_metrics g, const bca_phys *phys,
@@ -292,8 +291,7 @@ int bca_jbeta_fill(bca_ctx *ctx, const double *jac, const double *jdz, const dou
  * face-local Jacobian blocks are computed once and summed per row and seed.
  * write_index = 0 skips ia/ja (they depend on the mesh only).  Every BC box
  * of `ops` must lie on the block edge and every join box in the 7-layer
- * boundary frame; the seeded states are stored for that frame only, and any
- * other box returns an error. */
+ * boundary frame; any other box returns an error. */
 int bca_jacobian_colored(bca_ctx *ctx, const double *w, bca_metrics g, const bca_phys *phys,
                          const bca_bc_op *ops, int nops, const double *coefdiag, int withjn,
                          double *jac, int *ia, int *ja, long nbentry, int write_index);
@@ -311,7 +309,8 @@ int bca_jacobian_colored_2zones(bca_ctx *ctx, const double *w, bca_metrics g, co
  * (BROADCAST_npz.py:1018-1021, tangent :1079-1082) then flux_num_dnc5_2d
  * (srcfv/rhs/flux_num_dnc5.F90:7-226) or flux_num_dnc5_2d_d
  * (srcfv/tangent/flux_num_dnc5_d.f90:15) -- for up to 16 meshes of different
- * sizes (gh = 3), one launch per stage over all meshes.  Per item: the ghost
+ * sizes (gh = 3): one launch for all ghost fillings, one for all residuals
+ * (meshes that share a state go one by one).  Per item: the ghost
  * frames of w (and wd) are filled in place by the BC sequence, residu (and
  * residud = dR/dw . wd) are written on the interior.  Items carry wd and
  * residud all or none (residual only).  No reference counterpart as a batch:
@@ -344,8 +343,7 @@ int bca_batch_residual_jvp(bca_batch *batch, const bca_batch_item *items, int n)
  * (the reference routine takes two arrays and zeroes the donor adjoint
  * first, which in one block would clear wb).  nx, ny: the metrics (inlet and
  * no-reflexion read them).  Except for the join, the box must lie on the
- * block edge (the seeded states cover the 7-layer boundary frame only);
- * other boxes return an error. */
+ * block edge; other boxes return an error. */
 int bca_bc_adjoint(bca_ctx *ctx, const double *w, double *wb, const bca_bc_op *op, const double *nx,
                    const double *ny);
 
@@ -430,8 +428,8 @@ int bca_gemm_bf16(void *hip_stream, int M, int N, int K, const unsigned short *A
                   int ksplit);
 
 /* ---- launch-shape autotuner ------------------------------------------------ */
-/* No reference counterpart.  Times candidate block shapes of the residual face
- * kernel, the interior face-block kernels and the colored assembly on this
+/* No reference counterpart.  Times candidate block shapes of the interior
+ * face-block kernels and the colored assembly on this
  * context's mesh and state (median of reps launches each; nzones and zparam as
  * for bca_jacobian_colored_csr; jac: a COO buffer of nbentry values used as
  * scratch) and keeps the fastest for the context's later launches.  Results
