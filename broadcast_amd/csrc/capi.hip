@@ -1067,9 +1067,7 @@ int jacobian_phase1(bca_ctx* c, const double* w, bca_metrics g, const bca_phys* 
   // primal primitives and gradients of the state (ghost frame as given)
   k_prim<double><<<grid1(m.ncell, 256), 256, 0, s>>>(m, ph, w, c->w0.prim);
   BCA_LAUNCHED();
-  k_grad<double><<<grid2(m.im, m.jm, b), b, 0, s>>>(m, gm, c->w0.prim, c->w0.grad);
-  BCA_LAUNCHED();
-  k_grad_ghost<double><<<grid1(2 * m.im + m.jm, 256), 256, 0, s>>>(m, c->w0.grad);
+  k_grad<double><<<grid2(m.im + 2, m.jm + 2, b), b, 0, s>>>(m, gm, c->w0.prim, c->w0.grad);
   BCA_LAUNCHED();
   k_cellx<<<grid1(m.ncell, 256), 256, 0, s>>>(m, ph, w, c->w0.prim, c->cellx);
   BCA_LAUNCHED();
@@ -1201,9 +1199,7 @@ int bca_vjp_dnc5(bca_ctx* c, double* residub, double* wb, const double* w, bca_m
   // recomputed primal primitives and gradients (no tape)
   k_prim<double><<<grid1(m.ncell, 256), 256, 0, s>>>(m, ph, w, c->w0.prim);
   BCA_LAUNCHED();
-  k_grad<double><<<grid2(m.im, m.jm, b), b, 0, s>>>(m, gm, c->w0.prim, c->w0.grad);
-  BCA_LAUNCHED();
-  k_grad_ghost<double><<<grid1(2 * m.im + m.jm, 256), 256, 0, s>>>(m, c->w0.grad);
+  k_grad<double><<<grid2(m.im + 2, m.jm + 2, b), b, 0, s>>>(m, gm, c->w0.prim, c->w0.grad);
   BCA_LAUNCHED();
   // edge rows on the side streams while the interior runs (tiles of their
   // own; residub is only read until the join); the interior kernels are queued

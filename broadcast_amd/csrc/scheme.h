@@ -10,8 +10,8 @@
 // The residual and its tangent are one kernel (residual.h).  The Jacobian and
 // adjoint passes read planes of
 //   prim   : every cell (ghosts too)  u, v, w, T, p, mu, H
-//   grad   : interior cells           4th-order velocity gradients (u, v)
-//   ghost  : one extrapolated layer of gradients where faces read it
+//   grad   : interior cells           4th-order velocity gradients (u, v), and
+//            one extrapolated layer where faces read it
 #pragma once
 #include <hip/hip_runtime.h>
 #include "dual.h"
@@ -204,60 +204,29 @@ __device__ inline void gradient_at(const Mesh& m, const Metric& g, const T* prim
   out[G_VY] = dym1 * gvi + dym2 * gvj;
 }
 
+// The gradients of the interior, and (gradveloingh.F) of the ghost cells that the
+// faces read: columns 0 and im+1 (rows 1..jm) and rows 0 and jm+1 (columns 1..im),
+// where the reference's two-pass linear extrapolation reduces to 2 g(1) - g(2),
+// formed here from the two cells' own gradients (a launch after this one, for the
+// edges alone, took 5-8 us).
 template <class T>
 __global__ void k_grad(Mesh m, Metric g, const T* __restrict__ prim, T* __restrict__ grad) {
-  const int i = 1 + blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = 1 + blockIdx.y * blockDim.y + threadIdx.y;
-  if (i > m.im || j > m.jm) return;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int j = blockIdx.y * blockDim.y + threadIdx.y;
+  if (i > m.im + 1 || j > m.jm + 1) return;
+  const int di = i < 1 ? 1 : i > m.im ? -1 : 0, dj = j < 1 ? 1 : j > m.jm ? -1 : 0;
+  if (di && dj) return;
   T out[4];
-  gradient_at(m, g, prim, i, j, out);
+  gradient_at(m, g, prim, i + di, j + dj, out);
+  if (di || dj) {
+    T far[4];
+    gradient_at(m, g, prim, i + 2 * di, j + 2 * dj, far);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) out[k] = 2.0 * out[k] - far[k];
+  }
   const long c = cidx(m, i, j);
 #pragma unroll
   for (int k = 0; k < 4; ++k) grad[c + k * m.ncell] = out[k];
-}
-
-// gradveloingh.F: the faces that reach the residual read ghost gradients only
-// in columns 0 and im+1 (rows 1..jm), in row jm+1 and -- the variant without
-// wall rows, whose first j-faces are centred -- row 0 (columns 1..im); there
-// the reference's two-pass linear extrapolation reduces to 2 g(1) - g(2).
-template <class T>
-__global__ void k_grad_ghost(Mesh m, T* __restrict__ grad) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const long n = m.ncell;
-  if (t >= m.jm + m.im && t < m.jm + 2 * m.im) {
-    const int i = 1 + t - m.jm - m.im;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      T* G = grad + k * n;
-      G[cidx(m, i, 0)] = 2.0 * G[cidx(m, i, 1)] - G[cidx(m, i, 2)];
-    }
-    return;
-  }
-  if (t < m.jm) {
-    const int j = 1 + t;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      T* G = grad + k * n;
-      G[cidx(m, 0, j)] = 2.0 * G[cidx(m, 1, j)] - G[cidx(m, 2, j)];
-      G[cidx(m, m.im + 1, j)] = 2.0 * G[cidx(m, m.im, j)] - G[cidx(m, m.im - 1, j)];
-    }
-  } else if (t < m.jm + m.im) {
-    const int i = 1 + t - m.jm;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      T* G = grad + k * n;
-      G[cidx(m, i, m.jm + 1)] = 2.0 * G[cidx(m, i, m.jm)] - G[cidx(m, i, m.jm - 1)];
-    }
-  }
-}
-
-// balanceloop.F
-template <class T>
-__device__ inline T balance_at(const Mesh& m, const T* hn, int i, int j, int e) {
-  const long nn = m.nnode;
-  const T* hi = hn + (long)e * nn;
-  const T* hj = hn + (long)(5 + e) * nn;
-  return -(hi[nidx(m, i + 1, j)] - hi[nidx(m, i, j)]) - (hj[nidx(m, i, j + 1)] - hj[nidx(m, i, j)]);
 }
 
 }  // namespace bca
