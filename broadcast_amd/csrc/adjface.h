@@ -384,7 +384,7 @@ __device__ inline void face_reverse(const Mesh& m, const Phys& ph, const Metric&
   // The gradients' adjoints as weights of u and v along i and j, on the four
   // cells P_k = (k DX, k DY), k = -2..1, whose 4th-order gradients they
   // reach: cell 0's and cell -1's own gradients, or where one of them is on
-  // the extrapolated ghost layer of SeededAcc::G (i = 0, i = im+1, j = jm+1;
+  // the extrapolated ghost layer of gradients (i = 0, i = im+1, j = jm+1;
   // faces i = 1, i = im+1, j = jm+1) the two gradients 2 g(a) - g(b) it is
   // extrapolated from.
   const bool ext0 = J ? j == m.jm + 1 : i == m.im + 1;  // cell 0 at i = im+1 or j = jm+1

@@ -76,7 +76,7 @@ __device__ inline void face_linearise(const PlainAcc<double>& a, FaceLin& f) {
     f.et0 = r.t0, f.et1 = r.t1;
     // the gradients' adjoints on the four cells along the normal whose
     // 4th-order gradients they reach (an extrapolated ghost gradient is
-    // 2 g(a) - g(b), SeededAcc::G)
+    // 2 g(a) - g(b))
     const bool ext0 = J ? a.j == a.m.jm + 1 : a.i == a.m.im + 1;  // cell 0 a ghost layer
     const bool ext1 = !J && a.i == 1;                             // cell -1 a ghost layer
     double gbp[4][NGRAD];
