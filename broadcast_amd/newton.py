@@ -311,12 +311,13 @@ class BlockBandLU:
 
     def solve(self, b):
         """x with A x = b, b in the reference's unknown order."""
+        b = b.reshape(-1).contiguous()
         if self.np_lu and self.diag == "inv":
             # one correction with the matrix itself belongs to the solve: the
             # upward half of the elimination runs against the flow on a
             # boundary layer, where (weakly relaxed) it loses some digits
             x = self._apply(b)
-            r = csr_residual(self.csr, x, b.reshape(-1))
+            r = csr_residual(self.csr, x, b)
             if self.shift is not None:
                 r += self.shift * x
             return x + self._apply(r)
@@ -374,6 +375,8 @@ def csr_residual(csr, x, b):
 
     t = dev.torch()
     indptr, indices, data = csr
+    # the kernel reads both as consecutive values
+    x, b = x.contiguous(), b.contiguous()
     r = t.empty_like(b)
     _lib.check(_lib.lib().bca_csr_residual(dev.current_stream_ptr(), b.numel(), C.c_void_p(indptr.data_ptr()),
                                            C.c_void_p(indices.data_ptr()), C.c_void_p(data.data_ptr()),

@@ -1,0 +1,39 @@
+"""BlockBandLU.solve and csr_residual take what torch takes: right-hand sides of
+any stride.  The same kernels on the same values, so the same bits as for
+contiguous arrays."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def system(kind="bl"):
+    """Small relaxed Newton matrix: (case, outer, csr, right-hand side)."""
+    import torch as t
+    from broadcast_amd.cases import bl_case, cylinder_case
+    from broadcast_amd.flow import Flow, to_device
+
+    case = bl_case(24, 16, seed=5) if kind == "bl" else cylinder_case(21, 16, seed=5)
+    f = Flow(case)
+    w = to_device(case.w)
+    f.apply_bcs(w)
+    n = 5 * case.im * case.jm
+    cd = t.full((case.im * case.jm,), 1e-3, dtype=t.float64, device="cuda")
+    b = t.randn(n, dtype=t.float64, device="cuda", generator=t.Generator("cuda").manual_seed(1))
+    return case, "i" if kind == "bl" else "j", tuple(a.clone() for a in f.jacobian_csr(w, coefdiag=cd)), b
+
+
+@pytest.mark.parametrize("kind", ["bl", "cyl"])
+def test_solve_right_hand_side_of_any_stride(kind):
+    import torch as t
+    from broadcast_amd.newton import BlockBandLU, csr_residual
+
+    case, outer, csr, b = system(kind)
+    lu = BlockBandLU(case.im, case.jm, outer=outer).factor(*csr)
+    x = lu.solve(b)
+    column = t.stack((b, b + 1.0), 1)[:, 0]
+    assert not column.is_contiguous()
+    assert t.equal(lu.solve(column), x)
+    assert t.equal(csr_residual(csr, t.stack((x, b), 1)[:, 0], column), csr_residual(csr, x, b))
+    one = t.ones(1, dtype=t.float64, device="cuda").expand(b.numel())
+    assert t.equal(lu.solve(one), lu.solve(one.clone()))
+    assert t.equal(lu.solve(b.reshape(-1, 1)), x)
