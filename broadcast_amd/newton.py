@@ -92,7 +92,8 @@ class BlockBandLU:
         return e + 5 * (i + self.im * j)
 
     def factor(self, indptr, indices, data, shift=None):
-        """Factor the CSR matrix (minus shift * I when shift is given)."""
+        """Factor the CSR matrix (minus shift * I when shift is given): indptr
+        of any integer type, its first entry that of indices and data."""
         t = self.t
         dv = data.device
         n, B = self.n, self.B
@@ -137,7 +138,7 @@ class BlockBandLU:
                 # solve() corrects with the matrix: a copy, the caller's
                 # arrays may hold another one by then
                 if self.diag == "inv":
-                    self.csr, self.shift = (indptr.clone(), indices.clone(), data.clone()), shift
+                    self.csr, self.shift = csr_int32(indptr - indptr[:1], indices, data, copy=True), shift
                 return self
             # a pivot came out too small: refactor with partial pivoting
             self.np_lu = False
@@ -368,13 +369,21 @@ class BlockBandLU:
         return y.reshape(self.jm, self.im, 5).permute(1, 0, 2).reshape(-1)
 
 
+def csr_int32(indptr, indices, data, copy=False):
+    """The CSR as the kernels read it: int32 row starts and columns (torch's
+    own CSR holds int64), each array consecutive."""
+    t = dev.torch()
+    indptr, indices = (a.to(t.int32, copy=copy).contiguous() for a in (indptr, indices))
+    return indptr, indices, (data.clone() if copy else data).contiguous()
+
+
 def csr_residual(csr, x, b):
     """b - A x for the CSR (indptr, indices, data) on the device."""
     import ctypes as C
     from . import _lib
 
     t = dev.torch()
-    indptr, indices, data = csr
+    indptr, indices, data = csr_int32(*csr)
     # the kernel reads both as consecutive values
     x, b = x.contiguous(), b.contiguous()
     r = t.empty_like(b)

@@ -1,6 +1,6 @@
 """BlockBandLU.solve and csr_residual take what torch takes: right-hand sides of
-any stride.  The same kernels on the same values, so the same bits as for
-contiguous arrays."""
+any stride, any integer index type.  The same kernels on the same values, so the same bits as for
+contiguous int32 arrays."""
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -37,3 +37,24 @@ def test_solve_right_hand_side_of_any_stride(kind):
     one = t.ones(1, dtype=t.float64, device="cuda").expand(b.numel())
     assert t.equal(lu.solve(one), lu.solve(one.clone()))
     assert t.equal(lu.solve(b.reshape(-1, 1)), x)
+
+
+def test_solve_index_types():
+    import torch as t
+    from broadcast_amd.newton import BlockBandLU, csr_residual
+
+    case, outer, csr, b = system()
+    x = BlockBandLU(case.im, case.jm, outer=outer).factor(*csr).solve(b)
+    indptr, indices, data = csr
+    forms = {"int64": (indptr.long(), indices.long(), data),
+             "strided": tuple(t.stack((a, a), 1)[:, 0] for a in (indptr, indices, data))}
+    for name, form in forms.items():
+        print(name, flush=True)
+        assert t.equal(BlockBandLU(case.im, case.jm, outer=outer).factor(*form).solve(b), x)
+        assert t.equal(csr_residual(form, x, b), csr_residual(csr, x, b))
+    # the rows of a larger matrix: factor counts from the first row start, the
+    # product reads at the row starts
+    part = (indptr + 7, indices, data)
+    assert t.equal(BlockBandLU(case.im, case.jm, outer=outer).factor(*part).solve(b), x)
+    whole = (indptr + 7, t.cat((indices[:7], indices)), t.cat((data[:7], data)))
+    assert t.equal(csr_residual(whole, x, b), csr_residual(csr, x, b))
