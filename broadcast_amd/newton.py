@@ -314,6 +314,7 @@ class BlockBandLU:
         """x with A x = b, b in the reference's unknown order."""
         b = b.reshape(-1).contiguous()
         if self.np_lu and self.diag == "inv":
+            check_vector(b, self.R)
             # one correction with the matrix itself belongs to the solve: the
             # upward half of the elimination runs against the flow on a
             # boundary layer, where (weakly relaxed) it loses some digits
@@ -377,6 +378,12 @@ def csr_int32(indptr, indices, data, copy=False):
     return indptr, indices, (data.clone() if copy else data).contiguous()
 
 
+def check_vector(v, a):
+    """The kernels read v as float64 values on the HIP device of the matrix a."""
+    if v.dtype != dev.torch().float64 or v.device != a.device or not v.is_cuda:
+        raise RuntimeError(f"expected float64 values on {a.device}, got {v.dtype} on {v.device}")
+
+
 def csr_residual(csr, x, b):
     """b - A x for the CSR (indptr, indices, data) on the device."""
     import ctypes as C
@@ -384,6 +391,8 @@ def csr_residual(csr, x, b):
 
     t = dev.torch()
     indptr, indices, data = csr_int32(*csr)
+    for a in (x, b, data):
+        check_vector(a, indptr)
     # the kernel reads both as consecutive values
     x, b = x.contiguous(), b.contiguous()
     r = t.empty_like(b)

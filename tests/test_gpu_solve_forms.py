@@ -58,3 +58,21 @@ def test_solve_index_types():
     assert t.equal(BlockBandLU(case.im, case.jm, outer=outer).factor(*part).solve(b), x)
     whole = (indptr + 7, t.cat((indices[:7], indices)), t.cat((data[:7], data)))
     assert t.equal(csr_residual(whole, x, b), csr_residual(csr, x, b))
+
+
+def test_solve_refuses_other_types_and_devices():
+    """Raised on the host, before any kernel is given an address."""
+    import torch as t
+    from broadcast_amd.newton import BlockBandLU, csr_residual
+
+    case, outer, csr, b = system()
+    lu = BlockBandLU(case.im, case.jm, outer=outer).factor(*csr)
+    for wrong in (b.cpu(), b.float(), b.to(t.complex128)):
+        with pytest.raises(RuntimeError):
+            lu.solve(wrong)
+        with pytest.raises(RuntimeError):
+            csr_residual(csr, b, wrong)
+        with pytest.raises(RuntimeError):
+            csr_residual(csr, wrong, b)
+    with pytest.raises(RuntimeError):
+        csr_residual(tuple(a.cpu() for a in csr), b.cpu(), b.cpu())
