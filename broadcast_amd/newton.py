@@ -134,14 +134,15 @@ class BlockBandLU:
         self.np_lu = self.pivot is not True and dv.type == "cuda" and data.dtype == t.float64
         if self.np_lu:
             self._bad = t.zeros(1, dtype=t.int32, device=dv)
+            # solve() corrects with the matrix: a copy, the caller's arrays may
+            # hold another one by then; queued before np_factor waits for its
+            # result, so that a solve on any stream finds it complete
+            if self.diag == "inv":
+                self.csr, self.shift = csr_int32(indptr - indptr[:1], indices, data, copy=True), shift
             if self.np_factor(R, F):
-                # solve() corrects with the matrix: a copy, the caller's
-                # arrays may hold another one by then
-                if self.diag == "inv":
-                    self.csr, self.shift = csr_int32(indptr - indptr[:1], indices, data, copy=True), shift
                 return self
             # a pivot came out too small: refactor with partial pivoting
-            self.np_lu = False
+            self.np_lu, self.csr = False, None
             self.pivot, self.kb = True, None
             return self.factor(indptr, indices, data, shift)
         side = t.cuda.Stream() if (self.lookahead and dv.type == "cuda") else None

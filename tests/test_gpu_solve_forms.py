@@ -76,3 +76,22 @@ def test_solve_refuses_other_types_and_devices():
             csr_residual(csr, wrong, b)
     with pytest.raises(RuntimeError):
         csr_residual(tuple(a.cpu() for a in csr), b.cpu(), b.cpu())
+
+
+def test_factor_is_complete_when_it_returns():
+    """Nothing of factor is left on its stream when it returns, so a solve on
+    another stream, which waits for nothing, finds the factors and the matrix."""
+    import torch as t
+    from broadcast_amd.newton import BlockBandLU
+
+    case, outer, csr, b = system()
+    x = BlockBandLU(case.im, case.jm, outer=outer).factor(*csr).solve(b)
+    t.cuda.synchronize()
+    first, second = t.cuda.Stream(), t.cuda.Stream()
+    with t.cuda.stream(first):
+        lu = BlockBandLU(case.im, case.jm, outer=outer).factor(*csr)
+        assert first.query()
+    with t.cuda.stream(second):
+        y = lu.solve(b)
+    t.cuda.synchronize()
+    assert t.equal(x, y)
