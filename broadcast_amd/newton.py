@@ -322,7 +322,7 @@ class BlockBandLU:
             x = self._apply(b)
             r = csr_residual(self.csr, x, b)
             if self.shift is not None:
-                r += self.shift * x
+                r = r + self.shift * x
             return x + self._apply(r)
         return self._apply(b)
 
@@ -337,7 +337,7 @@ class BlockBandLU:
         y = t.cat((y, y.new_zeros(self.np - self.n))).reshape(nb, B)
         R = self.R
         if self.np_lu and self.diag == "inv":
-            y = self._solve_band(y)
+            y = self._solve_band_torch(y) if differentiated(y) else self._solve_band(y)
             return self._unpermute(y)
         for I in range(nb):
             y[I] = self._solve_diag(I, y[I])
@@ -364,6 +364,30 @@ class BlockBandLU:
             C.c_void_p(y.data_ptr()), C.c_void_p(z.data_ptr())), "bca_band_solve")
         return z
 
+    def _solve_band_torch(self, y):
+        """bca_band_solve's products by torch, for derivatives through the solve."""
+        nb, B, kb, mid, R = self.nb, self.B, self.kb, self.mid, self.R
+        steps = [(I, range(I + 1, min(I + kb, nb - 1) + 1)) for I in range(mid)]
+        if mid < nb:
+            steps += [(I, range(I - kb, I)) for I in range(nb - 1, mid + kb - 1, -1)]
+            steps += [(I, range(I + 1, mid + kb)) for I in range(mid, mid + kb)]
+
+        def block(K, J):
+            return R[K, :, (J - K + kb) * B:(J - K + kb + 1) * B]
+
+        y, z = list(y.unbind(0)), [None] * nb
+        for I, reach in steps:
+            z[I] = block(I, I) @ y[I]
+            for K in reach:
+                y[K] = y[K] - block(K, I) @ z[I]
+        for I, reach in reversed(steps):
+            for K in reach:
+                z[I] = z[I] - block(I, K) @ z[K]
+            if I == 0:
+                for f in range(1, min(self.nfar, nb - 1 - kb) + 1):
+                    z[0] = z[0] - self.F[:, (f - 1) * B:f * B] @ z[kb + f]
+        return self.t.stack(z)
+
     def _unpermute(self, y):
         y = y.reshape(-1)[:self.n]
         if self.outer == "i":
@@ -385,6 +409,19 @@ def check_vector(v, a):
         raise RuntimeError(f"expected float64 values on {a.device}, got {v.dtype} on {v.device}")
 
 
+def differentiated(v):
+    """Does torch take derivatives through v (or map over it)?  The kernels,
+    which are given v's address, would leave it out."""
+    t = dev.torch()
+    if (v.requires_grad and t.is_grad_enabled()) or t.autograd.forward_ad.unpack_dual(v).tangent is not None:
+        return True
+    try:
+        v.data_ptr()
+    except RuntimeError:  # a transform's wrapper has no storage
+        return True
+    return False
+
+
 def csr_residual(csr, x, b):
     """b - A x for the CSR (indptr, indices, data) on the device."""
     import ctypes as C
@@ -394,6 +431,11 @@ def csr_residual(csr, x, b):
     indptr, indices, data = csr_int32(*csr)
     for a in (x, b, data):
         check_vector(a, indptr)
+    if differentiated(x) or differentiated(b):
+        counts = (indptr[1:] - indptr[:-1]).long()
+        rows = t.repeat_interleave(t.arange(counts.numel(), device=data.device), counts)
+        part = slice(int(indptr[0]), int(indptr[-1]))
+        return b.index_add(0, rows, data[part] * x[indices[part].long()], alpha=-1)
     # the kernel reads both as consecutive values
     x, b = x.contiguous(), b.contiguous()
     r = t.empty_like(b)
