@@ -15,11 +15,15 @@
 //                     panels, 64 x 64 output tiles on the FP64 matrix cores
 //                     (v_mfma_f64_16x16x4f64), panels staged in LDS.
 //
-// No pivoting: the relaxed (or pure) Newton Jacobians of these flows factor
-// stably without it (element growth below 5 on the oracle's Jacobians, solves
-// as accurate as the pivoted ones); a pivot below tiny * the tile's largest
-// entry is reported so the caller can fall back, and the Newton driver
-// refines every solve with the CSR residual.
+// No pivoting: downwards, as the flow runs, the relaxed (or pure) Newton
+// Jacobians of these flows factor stably without it (element growth below 5 on
+// the oracle's Jacobians, solves as accurate as the pivoted ones).  The
+// two-ended elimination's upward half runs against the flow and loses some
+// digits on a weakly relaxed boundary layer.  A pivot below tiny * its tile's
+// largest entry is reported, which does not show growth across the blocks: the
+// Newton driver's solves are corrected once with the CSR residual, and where
+// the residual then says that entries grew, the driver factors again downwards
+// only, then with pivoting.
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -31,16 +31,24 @@ R[K] = [A(K, K-kb) ... A(K, K+kb)], (nblocks, B, (2 kb + 1) B) doubles.
 An i-periodic mesh (the O-mesh) couples the first and last i-lines; it is
 solved with j outermost instead (blocks of one j-line), where the band is
 that of the radial stencil.  Complex matrices, small pivots and CPU tensors
-take torch's pivoted LU of the diagonal blocks.
+take torch's pivoted LU of the diagonal blocks.  solve() looks at its residual
+(SOLVE_TOL): entries that grew in the elimination make it factor again,
+downwards only, then with the pivoted LU.
 """
 from __future__ import annotations
 
+import math
 import time
 from dataclasses import dataclass, field
 
 import numpy as np
 
 from . import device as dev
+
+# residual of a solve, relative to the right-hand side, above which the matrix
+# is factored again a safer way: the solves of the Newton matrices end at 1e-12
+# to 1e-15, and 1e-8 still gives Newton its full step
+SOLVE_TOL = 1e-8
 
 
 class BlockBandLU:
@@ -81,6 +89,8 @@ class BlockBandLU:
         self.np = self.nb * self.B                 # padded with identity rows past n
         self.kb = kb
         self.lookahead = lookahead
+        self.ends = 2                              # ends of the band the elimination may work from
+        self.mid = self.nb                         # block rows eliminated downwards (nb: all)
 
     def _perm(self, u):
         """Block-major index of the reference's unknown u."""
@@ -97,6 +107,7 @@ class BlockBandLU:
         t = self.t
         dv = data.device
         n, B = self.n, self.B
+        self.csr = None
         counts = (indptr[1:] - indptr[:-1]).long()
         rows = self._perm(t.repeat_interleave(t.arange(n, device=dv), counts))
         cols = self._perm(indices.long())
@@ -141,9 +152,8 @@ class BlockBandLU:
                 self.csr, self.shift = csr_int32(indptr - indptr[:1], indices, data, copy=True), shift
             if self.np_factor(R, F):
                 return self
-            # a pivot came out too small: refactor with partial pivoting
-            self.np_lu, self.csr = False, None
-            self.pivot, self.kb = True, None
+            # a pivot came out too small
+            self._safer()
             return self.factor(indptr, indices, data, shift)
         side = t.cuda.Stream() if (self.lookahead and dv.type == "cuda") else None
         cur = t.cuda.current_stream() if side is not None else None
@@ -217,7 +227,7 @@ class BlockBandLU:
         # (they meet with the downward end kb steps behind: the upward end's
         # last kb steps come after it)
         self.mid = nb // 2 - kb
-        if not self.lookahead or self.mid < kb + self.nfar + 1:
+        if not self.lookahead or self.ends == 1 or self.mid < kb + self.nfar + 1:
             self.mid = nb
         scratch = t.empty(2 * (1 + kb + self.nfar) * B * B, dtype=t.float64, device=R.device)
         cur = t.cuda.current_stream()
@@ -316,15 +326,45 @@ class BlockBandLU:
         b = b.reshape(-1).contiguous()
         if self.np_lu and self.diag == "inv":
             check_vector(b, self.R)
-            # one correction with the matrix itself belongs to the solve: the
-            # upward half of the elimination runs against the flow on a
-            # boundary layer, where (weakly relaxed) it loses some digits
-            x = self._apply(b)
-            r = csr_residual(self.csr, x, b)
-            if self.shift is not None:
-                r = r + self.shift * x
-            return x + self._apply(r)
+            if differentiated(b):
+                return self._corrected(b)
+            while self.np_lu:
+                x = self._corrected(b)
+                if self._accurate(x, b):
+                    return x
+                self._safer()
+                self.factor(*self.csr, shift=self.shift)
         return self._apply(b)
+
+    def _corrected(self, b):
+        """The factors applied, and one correction with the matrix itself: the
+        upward half of the elimination runs against the flow on a boundary
+        layer, where (weakly relaxed) it loses some digits."""
+        x = self._apply(b)
+        return x + self._apply(self._residual(x, b))
+
+    def _residual(self, x, b):
+        r = csr_residual(self.csr, x, b)
+        return r if self.shift is None else r + self.shift * x
+
+    def _accurate(self, x, b):
+        """||b - A x|| <= SOLVE_TOL ||b||.  No pivot is chosen across the
+        blocks, so the entries may grow in the elimination, which the pivots
+        of the tiles do not show; the residual does."""
+        t = self.t
+        if t.cuda.is_current_stream_capturing():
+            return True  # (a captured solve cannot ask)
+        rn, bn = t.stack((self._residual(x, b).norm(), b.norm())).tolist()
+        return rn <= SOLVE_TOL * bn or not math.isfinite(bn)
+
+    def _safer(self):
+        """The next factorization's way: downwards only, as the flow runs, then
+        with pivoting inside the diagonal blocks.  The present factors go."""
+        if self.mid < self.nb:
+            self.ends = 1
+        else:
+            self.pivot, self.kb = True, None
+        self.R = self.F = None
 
     def _apply(self, b):
         """The factors applied to b once."""

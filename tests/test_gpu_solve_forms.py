@@ -110,9 +110,8 @@ def band(outer, lines, line, kb):
     if outer == "j":
         # from j-line blocks to the reference's order
         A = A.reshape(lines, line, 5, lines, line, 5).permute(1, 0, 2, 4, 3, 5).reshape(n, n)
-    c = A.to_sparse_csr()
     im, jm = (lines, line) if outer == "i" else (line, lines)
-    return im, jm, A, (c.crow_indices(), c.col_indices(), c.values())
+    return im, jm, A, to_csr(A)
 
 
 @pytest.mark.parametrize("outer", ["i", "j"])
@@ -146,3 +145,65 @@ def test_derivatives_through_the_solve(outer, lines):
     bt = b.clone().requires_grad_()
     csr_residual(csr, g, bt).backward(g)
     assert t.equal(bt.grad, g)
+
+
+def weak_schur(A, B, at, to, eps):
+    """A(at, at) such that eliminating block `to` leaves it one singular value of
+    eps in place of 1: rows of the elimination in that direction grow by 1 / eps,
+    though no pivot is below 1e-14 of its tile; the matrix stays well conditioned."""
+    import torch as t
+
+    r, c = slice(at * B, (at + 1) * B), slice(to * B, (to + 1) * B)
+    g = t.Generator("cuda").manual_seed(7)
+    U, V = (t.linalg.qr(t.randn(B, B, dtype=t.float64, device="cuda", generator=g))[0] for _ in range(2))
+    s = t.ones(B, dtype=t.float64, device="cuda")
+    s[0] = eps
+    A[r, r] = A[r, c] @ t.linalg.solve(A[c, c], A[c, r]) + (U * s) @ V
+
+
+def to_csr(A):
+    c = A.to_sparse_csr()
+    return c.crow_indices(), c.col_indices(), c.values()
+
+
+def test_growth_in_the_upward_elimination_is_noticed():
+    """A matrix (condition about 1e3) that only the upward elimination is unstable
+    for: the solve is downwards then and accurate.  Tolerance: 40 n cond 2^-53."""
+    import torch as t
+    from broadcast_amd.newton import BlockBandLU
+
+    im, jm, A, _ = band("i", 12, 4, 1)
+    B, n = 5 * jm, A.shape[0]
+    weak_schur(A, B, im - 2, im - 1, 1e-11)
+    b = t.randn(n, dtype=t.float64, device="cuda", generator=t.Generator("cuda").manual_seed(2))
+    lu = BlockBandLU(im, jm).factor(*to_csr(A))
+    assert lu.np_lu and lu.mid < lu.nb
+    ref, cond = t.linalg.solve(A, b), float(t.linalg.cond(A))
+    for _ in range(2):
+        x = lu.solve(b)
+        assert float((x - ref).norm()) <= 40 * n * cond * 2.0 ** -53 * float(ref.norm())
+        assert lu.np_lu and lu.mid == lu.nb
+
+
+@pytest.mark.parametrize("pivot", [2e-14, 0.0])
+def test_growth_inside_a_block_is_pivoted(pivot):
+    """A second pivot just above the reported size, or a first one of zero, in
+    the first and the last block row: the pivoted LU of the diagonal blocks in
+    the end."""
+    import torch as t
+    from broadcast_amd.newton import BlockBandLU
+
+    im, jm, A, _ = band("i", 12, 4, 1)
+    B, n = 5 * jm, A.shape[0]
+    for k in (0, n - B):
+        m = float(A[k:k + B, k:k + B].abs().max())
+        A[k:k + 2, k:k + 2] = m
+        A[k + 1, k + 1] += m * pivot
+        if pivot == 0.0:
+            A[k, k] = 0.0
+    b = t.randn(n, dtype=t.float64, device="cuda", generator=t.Generator("cuda").manual_seed(2))
+    lu = BlockBandLU(im, jm).factor(*to_csr(A))
+    ref, cond = t.linalg.solve(A, b), float(t.linalg.cond(A))
+    x = lu.solve(b)
+    assert float((x - ref).norm()) <= 40 * n * cond * 2.0 ** -53 * float(ref.norm())
+    assert not lu.np_lu
