@@ -362,7 +362,7 @@ struct GjSmem {
   double U[GJ_NB][GJ_T + 16];
 };
 
-// The inverse of the nb x nb tile S(r, c) = get(in, r, c) (identity where in is
+// The inverse of the nb x nb tile S(r, c) = get(in, r, c) (a diagonal where in is
 // false), read by one wave in both layouts, stored through put(in, r, c, value); a pivot
 // below tiny times the tile's largest |entry| sets *bad.
 template <class Get, class Put>
@@ -378,15 +378,27 @@ __device__ inline void gj_invert_tile(int nb, double tiny, int* bad, const Get& 
       for (int t = 0; t < 4; ++t) {
         const int r = 16 * a + lk + 4 * t, c = 16 * b + lr;
         const bool in = r < nb && c < nb;
-        const double x = get(in, r, c), y = get(in, c, r);
-        X[a][b][t] = in ? x : (r == c ? 1.0 : 0.0);
-        Y[a][b][t] = in ? y : (r == c ? 1.0 : 0.0);
-        amax = fmax(amax, in ? fabs(x) : 0.0);
+        X[a][b][t] = get(in, r, c);
+        Y[a][b][t] = get(in, c, r);
+        amax = fmax(amax, in ? fabs(X[a][b][t]) : 0.0);
+      }
+  // the diagonal past nb: the power of two above the first pivot, |S(0, 0)|, so
+  // that the padded pivots are never the smallest and no rounding depends on them
+  const double pad = __builtin_ldexp(1.0, __builtin_amdgcn_frexp_exp(readlane_f64(X[0][0][0], 0)));
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int r = 16 * a + lk + 4 * t, c = 16 * b + lr;
+        const bool in = r < nb && c < nb;
+        X[a][b][t] = in ? X[a][b][t] : (r == c ? pad : 0.0);
+        Y[a][b][t] = in ? Y[a][b][t] : (r == c ? pad : 0.0);
       }
   const double pmin = gj_inv32(X, Y);
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) amax = fmax(amax, __shfl_xor(amax, off));
-  // padded pivots are 1: only a tile of tiny entries could be judged by them
   if (lane == 0 && !(pmin > tiny * amax)) *bad = 1;
 #pragma unroll
   for (int a = 0; a < 2; ++a)
