@@ -193,6 +193,7 @@ __global__ void __launch_bounds__(256) k_gemm_f64_sub(int M, int N, int K, const
 // inverse 0.22 against 0.73 ms (480: 0.18 / 0.57, 1920: 1.33 / 2.29 ms).
 constexpr int GJ_NB = 32;
 constexpr int GJ_T = 64;
+constexpr int GJ_RANGE = 300;  // binary exponents up to which a tile is inverted as it is
 
 // Doubles of a row-major tile through a buffer descriptor of its rows: an
 // index of NOWHERE is out of the descriptor's range, so such a load gives 0
@@ -384,7 +385,20 @@ __device__ inline void gj_invert_tile(int nb, double tiny, int* bad, const Get& 
       }
   // the diagonal past nb: the power of two above the first pivot, |S(0, 0)|, so
   // that the padded pivots are never the smallest and no rounding depends on them
-  const double pad = __builtin_ldexp(1.0, __builtin_amdgcn_frexp_exp(readlane_f64(X[0][0][0], 0)));
+  int e = __builtin_amdgcn_frexp_exp(readlane_f64(X[0][0][0], 0));
+  // the 2 x 2 determinants are of the order of its square: a tile where that
+  // would leave the range of a double is inverted scaled (exactly) by it
+  const int shift = e > GJ_RANGE || e < -GJ_RANGE ? e : 0;
+  if (shift != 0) {
+    amax = ldexp(amax, -shift);
+#pragma unroll
+    for (int x = 0; x < 16; ++x) {
+      X[x / 8][x / 4 % 2][x % 4] = ldexp(X[x / 8][x / 4 % 2][x % 4], -shift);
+      Y[x / 8][x / 4 % 2][x % 4] = ldexp(Y[x / 8][x / 4 % 2][x % 4], -shift);
+    }
+    e = 0;
+  }
+  const double pad = ldexp(1.0, e);
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -400,6 +414,9 @@ __device__ inline void gj_invert_tile(int nb, double tiny, int* bad, const Get& 
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) amax = fmax(amax, __shfl_xor(amax, off));
   if (lane == 0 && !(pmin > tiny * amax)) *bad = 1;
+  if (shift != 0)
+#pragma unroll
+    for (int x = 0; x < 16; ++x) X[x / 8][x / 4 % 2][x % 4] = ldexp(X[x / 8][x / 4 % 2][x % 4], -shift);
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll

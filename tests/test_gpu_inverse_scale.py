@@ -23,7 +23,7 @@ def inverse(A):
 
 
 @pytest.mark.parametrize("n", [1, 2, 3, 31, 33, 40, 65, 97, 130])
-@pytest.mark.parametrize("power", [53, -53])
+@pytest.mark.parametrize("power", [53, -53, 310, -310, 700, -700])
 def test_inverse_of_a_scaled_block(n, power):
     import torch as t
 
