@@ -201,6 +201,7 @@ constexpr int GJ_RANGE = 300;  // binary exponents up to which a tile is inverte
 // guarded load serialises the loads of a tile).
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 constexpr unsigned NOWHERE = ~0u;
+template <bool WIDE = false>
 struct TileBuf {
   __amdgpu_buffer_rsrc_t r;
   // rows rows of pitch ld from p, n columns (at least one row)
@@ -218,6 +219,18 @@ struct TileBuf {
   }
   __device__ void store(bool in, int row, long ld, int col, double v) const {
     store(in ? (unsigned)(row * (int)ld + col) * 8u : NOWHERE, v);
+  }
+};
+
+// The same by 64-bit addresses, for rows too far apart for the 32-bit offsets of a
+// descriptor.
+template <>
+struct TileBuf<true> {
+  double* p;
+  __device__ TileBuf(const double* q, int, long, int) : p(const_cast<double*>(q)) {}
+  __device__ double load(bool in, int row, long ld, int col) const { return in ? p[row * ld + col] : 0.0; }
+  __device__ void store(bool in, int row, long ld, int col, double v) const {
+    if (in) p[row * ld + col] = v;
   }
 };
 
@@ -437,10 +450,11 @@ struct GjPair {
 };
 
 // The first panel's pivot tile, inverted in place (one wave).
+template <bool WIDE>
 __global__ void __launch_bounds__(64) k_gj_first(GjPair m, long lda, int nb, double tiny, int* __restrict__ bad) {
   __builtin_amdgcn_s_setprio(3);
   double* A = m.in[blockIdx.y];
-  const TileBuf t(A, nb, lda, nb);
+  const TileBuf<WIDE> t(A, nb, lda, nb);
   gj_invert_tile(nb, tiny, bad, [&](bool in, int r, int c) { return t.load(in, r, lda, c); },
                  [&](bool in, int r, int c, double v) { t.store(in, r, lda, c, v); });
 }
@@ -448,6 +462,7 @@ __global__ void __launch_bounds__(64) k_gj_first(GjPair m, long lda, int nb, dou
 // One step, panel k0 .. k0 + nb - 1 (its pivot tile in Ain already inverted);
 // nb2 columns in the panel after it (0: none), whose pivot tile the last
 // workgroup updates and inverts.
+template <bool WIDE>
 __global__ void __launch_bounds__(256) k_gj_step(GjPair m, long lda, long ldo, int n, int k0, int nb, int nb2,
                                                  double tiny, int* __restrict__ bad) {
   __shared__ GjSmem sm;
@@ -463,7 +478,7 @@ __global__ void __launch_bounds__(256) k_gj_step(GjPair m, long lda, long ldo, i
   const int ni = ahead ? nb2 : n - i0, nj = ahead ? nb2 : n - j0;  // rows and columns present
   auto in_panel = [&](int g) { return g >= k0 && g < kn; };
   // the tile's rows and the panel's rows
-  const TileBuf rows(Ain + (long)i0 * lda, ni < GJ_T ? ni : GJ_T, lda, n), kk(Ain + (long)k0 * lda, nb, lda, n);
+  const TileBuf<WIDE> rows(Ain + (long)i0 * lda, ni < GJ_T ? ni : GJ_T, lda, n), kk(Ain + (long)k0 * lda, nb, lda, n);
 #pragma unroll
   for (int x = 0; x < GJ_T * GJ_NB / 256; ++x) {
     const int r = x * 8 + tid / GJ_NB, c = tid % GJ_NB;
@@ -517,7 +532,7 @@ __global__ void __launch_bounds__(256) k_gj_step(GjPair m, long lda, long ldo, i
       }
   }
   __syncthreads();
-  const TileBuf out(Aout + (long)i0 * ldo, ni < GJ_T ? ni : GJ_T, ldo, n);
+  const TileBuf<WIDE> out(Aout + (long)i0 * ldo, ni < GJ_T ? ni : GJ_T, ldo, n);
   if (ahead) {
     // S = A(next, next) - T U, through LDS to wave 0, which inverts it
     double av[GJ_NB / 4], bv[GJ_NB / 4];
@@ -632,7 +647,7 @@ __global__ void __launch_bounds__(256) k_block_products(BlockProducts list, int 
   double ra[NA], rb[NB];
   auto fetch = [&](int k0) {
     const int kr = min(KS, n - k0);
-    const TileBuf ta(q.A + (long)m0 * q.lda + k0, mr, q.lda, kr), tb(q.B + (long)k0 * q.ldb, kr, q.ldb, n);
+    const TileBuf<> ta(q.A + (long)m0 * q.lda + k0, mr, q.lda, kr), tb(q.B + (long)k0 * q.ldb, kr, q.ldb, n);
     if (kr == KS) {
 #pragma unroll
       for (int x = 0; x < NA; ++x) ra[x] = ta.load(oa[x]);
@@ -652,7 +667,7 @@ __global__ void __launch_bounds__(256) k_block_products(BlockProducts list, int 
 #pragma unroll
     for (int x = 0; x < NB; ++x) Bs[s][x * (256 / TN) + tid / TN][tid % TN] = rb[x];
   };
-  const TileBuf tc(q.C + (long)m0 * q.ldc, mr, q.ldc, n);
+  const TileBuf<> tc(q.C + (long)m0 * q.ldc, mr, q.ldc, n);
   f64x4 acc[MT][NT], cv[MT][NT];
 #pragma unroll
   for (int a = 0; a < MT; ++a)

@@ -1850,7 +1850,10 @@ int invert_blocks(hipStream_t s, int batch, double* const A[], int n, long ld, d
     m.in[q] = A[q];
     m.out[q] = work[q];
   }
-  k_gj_first<<<dim3(1, batch), 64, 0, s>>>(m, ld, std::min(GJ_NB, n), tiny, bad);
+  // 32-bit byte offsets within a tile's rows, or 64-bit addresses
+  const bool wide = GJ_T * ld * (long)sizeof(double) > 4294967295L;
+  if (wide) k_gj_first<true><<<dim3(1, batch), 64, 0, s>>>(m, ld, std::min(GJ_NB, n), tiny, bad);
+  else k_gj_first<false><<<dim3(1, batch), 64, 0, s>>>(m, ld, std::min(GJ_NB, n), tiny, bad);
   BCA_LAUNCHED();
   if (n <= GJ_NB) return 0;  // one panel: its pivot tile is the block
   // Panels of GJ_NB columns; the steps alternate between A and work, so an
@@ -1872,7 +1875,9 @@ int invert_blocks(hipStream_t s, int batch, double* const A[], int n, long ld, d
   int k0 = 0;
   for (size_t q = 0; q < widths.size(); ++q) {
     const int nb = widths[q], nb2 = q + 1 < widths.size() ? widths[q + 1] : 0;
-    k_gj_step<<<dim3(nt * nt + (nb2 ? 1 : 0), batch), 256, 0, s>>>(m, ldi, ldo, n, k0, nb, nb2, tiny, bad);
+    const dim3 gr(nt * nt + (nb2 ? 1 : 0), batch);
+    if (wide) k_gj_step<true><<<gr, 256, 0, s>>>(m, ldi, ldo, n, k0, nb, nb2, tiny, bad);
+    else k_gj_step<false><<<gr, 256, 0, s>>>(m, ldi, ldo, n, k0, nb, nb2, tiny, bad);
     BCA_LAUNCHED();
     std::swap(ldi, ldo);
     for (int x = 0; x < batch; ++x) std::swap(m.in[x], m.out[x]);
