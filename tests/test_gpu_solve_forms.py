@@ -207,3 +207,19 @@ def test_growth_inside_a_block_is_pivoted(pivot):
     x = lu.solve(b)
     assert float((x - ref).norm()) <= 40 * n * cond * 2.0 ** -53 * float(ref.norm())
     assert not lu.np_lu
+
+
+@pytest.mark.parametrize("lines,kb", [(1, 1), (1, 3), (2, 3), (3, 7)])
+def test_half_width_beyond_the_matrix(lines, kb):
+    """A half-width of the band given by the caller may exceed the block rows.
+    Tolerance: 40 n 2^-53, as above."""
+    import torch as t
+    from broadcast_amd.newton import BlockBandLU
+
+    im, jm, A, csr = band("i", lines, 3, min(kb, lines - 1))
+    n = A.shape[0]
+    b = t.randn(n, dtype=t.float64, device="cuda", generator=t.Generator("cuda").manual_seed(2))
+    lu = BlockBandLU(im, jm, kb=kb).factor(*csr)
+    ref = t.linalg.solve(A, b)
+    assert lu.np_lu and lu.kb == kb
+    assert float((lu.solve(b) - ref).norm()) <= 40 * n * 2.0 ** -53 * float(ref.norm())
