@@ -2017,6 +2017,8 @@ int band_step(const BandMatrix& a, const BandStreams& c, const std::vector<BandS
 
 int band_check(const BandMatrix& a, int mid) {
   if (a.nb < 1 || a.B < 1 || a.kb < 0 || a.nfar < 0) return fail(-1, "band: bad block counts");
+  // (its elimination fills block row 1 up to column kb + nfar)
+  if (a.nfar > 1) return fail(-1, "band: block row 0 may reach one block beyond the band");
   if (mid != a.nb && (mid < 1 || mid + a.kb >= a.nb)) return fail(-1, "band: mid must be nb or leave rows on both ends");
   if (a.W() * 8L * 128 > 2147483647L) return fail(-1, "band: block row too wide");
   return 0;

@@ -58,8 +58,8 @@ class BlockBandLU:
     The band half-width kb (in blocks) is the widest coupling of every block
     row but the first: on the O-mesh (j-line blocks) the wall row j = 1 also
     reaches j = 5 (the off-centred Euler flux of the face j = 2), one block
-    beyond the radial stencil's 3.  Such far blocks of block row 0 are kept
-    outside the band (eliminating block 0 turns them into in-band updates of
+    beyond the radial stencil's 3.  Such a far block of block row 0 is kept
+    outside the band (eliminating block 0 turns it into in-band updates of
     block rows 1..kb), so the band stays 2 kb + 1 blocks wide: with kb = 3
     instead of 4, 9 instead of 16 Schur products per block step.
 
@@ -118,7 +118,10 @@ class BlockBandLU:
             kb = int(d[rest].abs().max()) if bool(rest.any()) else 0
             kb = max(kb, int((-d).max()), 1 if self.nb > 1 else 0)
             self.kb = min(kb, self.nb - 1)
-        kb = self.kb
+        # a far block two beyond the band would leave fill in block row 1 that
+        # the band does not hold
+        first = d[K == 0]
+        self.kb = kb = max(self.kb, int(first.max()) - 1 if first.numel() else 0)
         W = (2 * kb + 1) * B
         far = d > kb
         if bool((far & (K > 0)).any()) or bool((d < -kb).any()):

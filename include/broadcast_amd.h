@@ -397,8 +397,8 @@ int bca_lu_np(void *hip_stream, double *A, int n, long ld, double tiny, int *bad
 int bca_inv_np(void *hip_stream, double *A, int n, long ld, double *work, double tiny, int *bad);
 /* Block-banded elimination of nb block rows of B unknowns, kb blocks to either
  * side: R holds row K as [A(K, K-kb) ... A(K, K+kb)] (B x (2 kb + 1) B,
- * row-major, rows back to back), F (B x nfar B) the blocks kb+1 .. kb+nfar of
- * block row 0.  Rows 0 .. mid-1 are eliminated downwards, nb-1 .. mid+kb
+ * row-major, rows back to back), F (B x nfar B) the block kb+1 of block row 0
+ * (nfar 0 or 1).  Rows 0 .. mid-1 are eliminated downwards, nb-1 .. mid+kb
  * upwards beside them, then the kb rows between (mid = nb: all downwards).
  * In place: D_I^-1 on the diagonal, D_I^-1 A(I, J) for the blocks J a row
  * still reaches, the others as given.  streams: the caller's (ordered before
