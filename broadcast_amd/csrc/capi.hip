@@ -1462,6 +1462,8 @@ struct bca_batch {
   long table_bytes = 0;
   hipEvent_t copied = nullptr;  // the last table copy (the staging is reused after it)
   bool pending = false;
+  hipEvent_t done = nullptr;    // the last call's kernels (table and scratch are reused after them)
+  bool ran = false;
 };
 
 namespace {
@@ -1474,6 +1476,19 @@ int batch_grow(void** p, long* have, long want, bool pinned) {
   if (pinned) BCA_HIP(hipHostMalloc(p, want, hipHostMallocDefault));
   else BCA_HIP(hipMalloc(p, want));
   *have = want;
+  return 0;
+}
+
+bool batch_capturing(const bca_batch* b) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(b->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
+// The batch's stream waits for the last call's kernels; a stream under capture
+// cannot wait for work outside it, so there the host does.
+int batch_wait(bca_batch* b) {
+  if (batch_capturing(b)) BCA_HIP(hipEventSynchronize(b->done));
+  else BCA_HIP(hipStreamWaitEvent(b->stream, b->done, 0));
   return 0;
 }
 
@@ -1513,6 +1528,8 @@ int run_batch(bca_batch* b, const bca_batch_item* items, int n) {
       }
   }
   int rc = 0;
+  // the last call may run on another stream: this one starts after it
+  if (b->ran && (rc = batch_wait(b))) return rc;
   if (through && (rc = batch_grow(&b->scratch, &b->scratch_bytes, planes * (long)sizeof(double), false))) return rc;
   // one plan, or one per mesh
   const int groups = shared ? n : 1, per = shared ? 1 : n;
@@ -1566,28 +1583,37 @@ int run_batch(bca_batch* b, const bca_batch_item* items, int n) {
   const BatchItem* ditems = reinterpret_cast<const BatchItem*>(b->table);
   const BatchPlan* dplans = reinterpret_cast<const BatchPlan*>(ditems + BATCH_MAX);
   hipStream_t s = b->stream;
-  for (int q = 0; q < groups; ++q) {
-    const BatchPlan& plan = plans[q];
-    const BatchItem* di = ditems + q * per;
-    if (whole[q]) {
-      if (plan.seq[per]) k_batch_bc_sequence<V><<<plan.seq[per], BC_SEQ_THREADS, 0, s>>>(di, dplans + q);
+  auto launches = [&]() -> int {
+    for (int q = 0; q < groups; ++q) {
+      const BatchPlan& plan = plans[q];
+      const BatchItem* di = ditems + q * per;
+      if (whole[q]) {
+        if (plan.seq[per]) k_batch_bc_sequence<V><<<plan.seq[per], BC_SEQ_THREADS, 0, s>>>(di, dplans + q);
+        BCA_LAUNCHED();
+      } else {
+        for (int o = 0; o < BATCH_OPS; ++o) {
+          if (plan.bc[o][per] == 0) continue;
+          k_batch_bc<V><<<grid1(plan.bc[o][per], 256), 256, 0, s>>>(di, dplans + q, o);
+          BCA_LAUNCHED();
+        }
+      }
+      k_batch_residual<V><<<plan.tiles[per], TILE_THREADS, 0, s>>>(di, dplans + q);
       BCA_LAUNCHED();
-    } else {
-      for (int o = 0; o < BATCH_OPS; ++o) {
-        if (plan.bc[o][per] == 0) continue;
-        k_batch_bc<V><<<grid1(plan.bc[o][per], 256), 256, 0, s>>>(di, dplans + q, o);
+    }
+    if (through)
+      for (int q = 0; q < groups; ++q) {
+        k_batch_store<<<grid1(plans[q].cells[per], 256), 256, 0, s>>>(ditems + q * per, dplans + q);
         BCA_LAUNCHED();
       }
-    }
-    k_batch_residual<V><<<plan.tiles[per], TILE_THREADS, 0, s>>>(di, dplans + q);
-    BCA_LAUNCHED();
+    return 0;
+  };
+  rc = launches();
+  if (!batch_capturing(b)) {
+    if (!b->done) BCA_HIP(hipEventCreateWithFlags(&b->done, hipEventDisableTiming));
+    BCA_HIP(hipEventRecord(b->done, s));
+    b->ran = true;
   }
-  if (through)
-    for (int q = 0; q < groups; ++q) {
-      k_batch_store<<<grid1(plans[q].cells[per], 256), 256, 0, s>>>(ditems + q * per, dplans + q);
-      BCA_LAUNCHED();
-    }
-  return 0;
+  return rc;
 }
 
 }  // namespace
@@ -1611,6 +1637,7 @@ int bca_batch_destroy(bca_batch* b) {
   if (!b) return 0;
   if (b->pending) (void)hipEventSynchronize(b->copied);
   if (b->copied) (void)hipEventDestroy(b->copied);
+  if (b->done) (void)hipEventDestroy(b->done);
   if (b->scratch) (void)hipFree(b->scratch);
   if (b->table) (void)hipFree(b->table);
   if (b->host) (void)hipHostFree(b->host);

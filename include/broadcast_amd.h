@@ -313,8 +313,10 @@ int bca_jacobian_colored_2zones(bca_ctx *ctx, const double *w, bca_metrics g, co
  * (meshes that share a state go one by one).  Per item: the ghost
  * frames of w (and wd) are filled in place by the BC sequence, residu (and
  * residud = dR/dw . wd) are written on the interior.  Items carry wd and
- * residud all or none (residual only).  No reference counterpart as a batch:
- * the reference calls the per-mesh routines once per mesh. */
+ * residud all or none (residual only).  A call on another stream than the last
+ * one's starts after it (they share the batch's table and scratch).  No
+ * reference counterpart as a batch: the reference calls the per-mesh routines
+ * once per mesh. */
 typedef struct bca_batch bca_batch;
 typedef struct {
   int im, jm;
