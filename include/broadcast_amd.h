@@ -72,7 +72,9 @@ long bca_ctx_scratch_bytes(const bca_ctx *ctx);
  * clocks, BROADCAST_npz.py:1003-1007).  enable resets the record; read sums
  * the launches of one kernel or stage, named "k_residual<f64>",
  * "k_residual<dual1>", "k_bc_sequence", "k_iface_blocks", "k_jface_blocks",
- * "ghost_tangents", "k_ghost_part", "k_jac_csr_refresh", ... */
+ * "ghost_tangents", "k_ghost_part", "k_jac_csr_refresh", ...; "k_face<f64>" and
+ * "k_face<dual1>" read the residual's and the tangent's kernel, which hold what
+ * "k_prim<..>", "k_grad<..>" and "k_balance<..>" were beside it. */
 int bca_profile_enable(bca_ctx *ctx, int on);
 int bca_profile_read(bca_ctx *ctx, const char *kernel, double *total_ms, long *launches);
 
