@@ -563,6 +563,10 @@ __global__ void __launch_bounds__(256) k_face_reverse(Mesh m, Phys ph, Metric g,
   const int i = 1 + bx * REV + tx, j = j0 + by * REV + wave * REV_ROWS + ty;
   double* a = lds + wave * R::n;
   for (int x = tid % 64; x < R::n; x += 64) a[x] = 0.0;
+  // other lanes of the wave add to these zeros (the LDS takes a wave's operations
+  // in order: no wait, but none may be moved over)
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
   if (i <= (J ? m.im : m.im + 1) && j <= j1) {
     double hb[5];
     face_adjoint(m, resb, i, j, J ? 0 : 1, J ? 1 : 0, hb);
