@@ -290,6 +290,12 @@ int bc_check(const Mesh& m, const bca_bc_op& op, const double* nx, const double*
   }
 }
 
+// The inlet's profile is as long as the interface reaches (its own entry and the
+// sequence).
+int inlet_check(const bca_bc_op& op) {
+  return op.lm < (op.loc <= 1 ? op.box[3] : op.box[2]) ? fail(-1, "field shorter than the interface") : 0;
+}
+
 // Does the index box [i0, i1] x [j0, j1] lie wholly in the frame of width W
 // around the array (storage coordinates a < W or a >= ni - W, likewise b)?
 bool box_in_frame(const Mesh& m, int i0, int j0, int i1, int j1, int W) {
@@ -798,8 +804,10 @@ int bca_bc_sequence(bca_ctx* c, double* w, double* wd, const bca_bc_op* ops, int
   if (nops < 0 || (nops > 0 && !ops)) return fail(-1, "bad boundary-condition list");
   const Mesh& m = c->m;
   int rc = 0;
-  for (int k = 0; k < nops; ++k)  // (a join out of the plan is checked by its own entry)
+  for (int k = 0; k < nops; ++k) {  // (a join out of the plan is checked by its own entry)
+    if (ops[k].kind == BCA_BC_INLET && (rc = inlet_check(ops[k]))) return rc;
     if (ops[k].kind != BCA_BC_JOIN && (rc = bc_check(m, ops[k], nx, ny))) return rc;
+  }
   BcSeq seq;
   if (bc_sequence_plan(m, ops, nops, seq)) {
     Timed t(c, "k_bc_sequence");
@@ -827,7 +835,9 @@ int bca_bc_inlet(bca_ctx* c, double* w, double* wd, int loc, const int box[4], c
   bca_bc_op op{};
   op.kind = BCA_BC_INLET; op.loc = loc; std::memcpy(op.box, box, sizeof(op.box));
   op.data = field; op.lm = lm; op.gam = gam;
-  if (c && lm < (loc <= 1 ? box[3] : box[2])) return fail(-1, "field shorter than the interface");
+  if (c) {
+    if (int rc = inlet_check(op)) return rc;
+  }
   return bc_entry(c, w, wd, op, nx, ny);
 }
 
