@@ -383,7 +383,6 @@ template <class Get, class Put>
 __device__ inline void gj_invert_tile(int nb, double tiny, int* bad, const Get& get, const Put& put) {
   const int lane = threadIdx.x % 64, lr = lane % 16, lk = lane / 16;
   f64x4 X[2][2], Y[2][2];
-  double amax = 0.0;
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -394,16 +393,14 @@ __device__ inline void gj_invert_tile(int nb, double tiny, int* bad, const Get& 
         const bool in = r < nb && c < nb;
         X[a][b][t] = get(in, r, c);
         Y[a][b][t] = get(in, c, r);
-        amax = fmax(amax, in ? fabs(X[a][b][t]) : 0.0);
       }
   // the diagonal past nb: the power of two above the first pivot, |S(0, 0)|, so
   // that the padded pivots are never the smallest and no rounding depends on them
-  int e = __builtin_amdgcn_frexp_exp(readlane_f64(X[0][0][0], 0));
+  int e = __builtin_amdgcn_readfirstlane(__builtin_amdgcn_frexp_exp(readlane_f64(X[0][0][0], 0)));
   // the 2 x 2 determinants are of the order of its square: a tile where that
   // would leave the range of a double is inverted scaled (exactly) by it
   const int shift = e > GJ_RANGE || e < -GJ_RANGE ? e : 0;
-  if (shift != 0) {
-    amax = ldexp(amax, -shift);
+  if (__builtin_expect(shift != 0, 0)) {
 #pragma unroll
     for (int x = 0; x < 16; ++x) {
       X[x / 8][x / 4 % 2][x % 4] = ldexp(X[x / 8][x / 4 % 2][x % 4], -shift);
@@ -412,6 +409,7 @@ __device__ inline void gj_invert_tile(int nb, double tiny, int* bad, const Get& 
     e = 0;
   }
   const double pad = ldexp(1.0, e);
+  double amax = 0.0;
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -420,6 +418,7 @@ __device__ inline void gj_invert_tile(int nb, double tiny, int* bad, const Get& 
       for (int t = 0; t < 4; ++t) {
         const int r = 16 * a + lk + 4 * t, c = 16 * b + lr;
         const bool in = r < nb && c < nb;
+        amax = fmax(amax, in ? fabs(X[a][b][t]) : 0.0);
         X[a][b][t] = in ? X[a][b][t] : (r == c ? pad : 0.0);
         Y[a][b][t] = in ? Y[a][b][t] : (r == c ? pad : 0.0);
       }
@@ -427,7 +426,7 @@ __device__ inline void gj_invert_tile(int nb, double tiny, int* bad, const Get& 
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) amax = fmax(amax, __shfl_xor(amax, off));
   if (lane == 0 && !(pmin > tiny * amax)) *bad = 1;
-  if (shift != 0)
+  if (__builtin_expect(shift != 0, 0))
 #pragma unroll
     for (int x = 0; x < 16; ++x) X[x / 8][x / 4 % 2][x % 4] = ldexp(X[x / 8][x / 4 % 2][x % 4], -shift);
 #pragma unroll
