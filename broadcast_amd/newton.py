@@ -31,9 +31,9 @@ R[K] = [A(K, K-kb) ... A(K, K+kb)], (nblocks, B, (2 kb + 1) B) doubles.
 An i-periodic mesh (the O-mesh) couples the first and last i-lines; it is
 solved with j outermost instead (blocks of one j-line), where the band is
 that of the radial stencil.  Complex matrices, small pivots and CPU tensors
-take torch's pivoted LU of the diagonal blocks.  solve() looks at its residual
-(SOLVE_TOL): entries that grew in the elimination make it factor again,
-downwards only, then with the pivoted LU.
+take torch's pivoted LU of the diagonal blocks.  The residual of a solve
+(SOLVE_TOL) shows entries that grew in the elimination: solve(), or refine()
+after it, then factors again, downwards only, then with the pivoted LU.
 """
 from __future__ import annotations
 
@@ -67,7 +67,7 @@ class BlockBandLU:
     the remaining products of a step run beside it on another stream; the
     library's elimination then also works from both ends of the band at once."""
 
-    def __init__(self, im, jm, outer="i", kb=None, group=1, lookahead=True, pivot=None, diag="inv"):
+    def __init__(self, im, jm, outer="i", kb=None, group=1, lookahead=True, pivot=None, diag="inv", check=True):
         self.t = dev.torch()
         # pivot=None: the project's elimination without pivoting on the device
         # for the diagonal blocks -- diag="inv": their inverses by Gauss-Jordan
@@ -89,6 +89,9 @@ class BlockBandLU:
         self.np = self.nb * self.B                 # padded with identity rows past n
         self.kb = kb
         self.lookahead = lookahead
+        # check: solve() looks at its residual (a caller that gives every
+        # solution to refine() leaves that to it)
+        self.check = check
         self.ends = 2                              # ends of the band the elimination may work from
         self.mid = self.nb                         # block rows eliminated downwards (nb: all)
 
@@ -118,15 +121,17 @@ class BlockBandLU:
             kb = int(d[rest].abs().max()) if bool(rest.any()) else 0
             kb = max(kb, int((-d).max()), 1 if self.nb > 1 else 0)
             self.kb = min(kb, self.nb - 1)
-        # a far block two beyond the band would leave fill in block row 1 that
-        # the band does not hold
-        first = d[K == 0]
-        self.kb = kb = max(self.kb, int(first.max()) - 1 if first.numel() else 0)
-        W = (2 * kb + 1) * B
+        kb = self.kb
         far = d > kb
         if bool((far & (K > 0)).any()) or bool((d < -kb).any()):
             raise ValueError("entry outside the block band")
         self.nfar = int(d[far].max()) - kb if bool(far.any()) else 0
+        if self.nfar > 1:
+            # a far block two beyond the band would leave fill in block row 1
+            # that the band does not hold
+            self.kb = kb = kb + self.nfar - 1
+            self.nfar, far = 1, d > kb
+        W = (2 * kb + 1) * B
         inb = ~far
         R = t.zeros((self.nb, B, W), dtype=data.dtype, device=dv)
         R.view(-1).index_put_((((K * B + rows % B) * W + (d + kb) * B + cols % B)[inb],), data[inb])
@@ -329,14 +334,12 @@ class BlockBandLU:
         b = b.reshape(-1).contiguous()
         if self.np_lu and self.diag == "inv":
             check_vector(b, self.R)
-            if differentiated(b):
-                return self._corrected(b)
-            while self.np_lu:
-                x = self._corrected(b)
-                if self._accurate(x, b):
-                    return x
-                self._safer()
-                self.factor(*self.csr, shift=self.shift)
+            x = self._corrected(b)
+            if not self.check or differentiated(b):
+                return x
+            while not self._accurate(x, b) and self.refactor():
+                x = self._corrected(b) if self.np_lu else self._apply(b)
+            return x
         return self._apply(b)
 
     def _corrected(self, b):
@@ -355,8 +358,8 @@ class BlockBandLU:
         blocks, so the entries may grow in the elimination, which the pivots
         of the tiles do not show; the residual does."""
         t = self.t
-        if t.cuda.is_current_stream_capturing():
-            return True  # (a captured solve cannot ask)
+        if not self.np_lu or t.cuda.is_current_stream_capturing():
+            return True  # (pivoted already; a captured solve cannot ask)
         rn, bn = t.stack((self._residual(x, b).norm(), b.norm())).tolist()
         return rn <= SOLVE_TOL * bn or not math.isfinite(bn)
 
@@ -368,6 +371,15 @@ class BlockBandLU:
         else:
             self.pivot, self.kb = True, None
         self.R = self.F = None
+
+    def refactor(self):
+        """The same matrix factored again the next safer way; False where there
+        is none."""
+        if not self.np_lu or self.diag != "inv":
+            return False
+        self._safer()
+        self.factor(*self.csr, shift=self.shift)
+        return True
 
     def _apply(self, b):
         """The factors applied to b once."""
@@ -493,8 +505,18 @@ def refine(lu, csr, b, x, rtol=1e-12, steps=3):
     """Iterative refinement of x (in place) for A x = b with the factors of
     lu, until ||b - A x|| <= rtol ||b||, a correction no longer halves the
     residual (its rounding floor), or `steps` corrections: the guard of the
-    unpivoted factorization.  Returns (corrections, final relative
-    residual)."""
+    unpivoted factorization.  A residual left above SOLVE_TOL means that
+    entries grew in it: lu factors again a safer way and x is solved anew.
+    Returns (corrections, final relative residual)."""
+    k, rel = correct(lu, csr, b, x, rtol, steps)
+    while rel > SOLVE_TOL and lu.refactor():
+        x.copy_(lu.solve(b))
+        k, rel = correct(lu, csr, b, x, rtol, steps)
+    return k, rel
+
+
+def correct(lu, csr, b, x, rtol, steps):
+    """refine()'s corrections with the factors as they are."""
     bn = float(b.norm())
     k = 0
     r = csr_residual(csr, x, b)
@@ -587,7 +609,7 @@ def newton(flow, w, ite=10, cfl=1e10, tol=1e-10, log=None, verbose=False, growth
         indptr, indices, data = flow.jacobian_csr(w, coefdiag=coefdiag, refresh=True)
         t.cuda.synchronize()
         t1 = time.perf_counter()
-        lu = BlockBandLU(flow.im, flow.jm, outer=outer, group=group).factor(indptr, indices, data)
+        lu = BlockBandLU(flow.im, flow.jm, outer=outer, group=group, check=False).factor(indptr, indices, data)
         t.cuda.synchronize()
         t2 = time.perf_counter()
         rhs = interior(flow, res).reshape(-1)

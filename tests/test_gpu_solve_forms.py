@@ -170,7 +170,7 @@ def test_growth_in_the_upward_elimination_is_noticed():
     """A matrix (condition about 1e3) that only the upward elimination is unstable
     for: the solve is downwards then and accurate.  Tolerance: 40 n cond 2^-53."""
     import torch as t
-    from broadcast_amd.newton import BlockBandLU
+    from broadcast_amd.newton import SOLVE_TOL, BlockBandLU, refine
 
     im, jm, A, _ = band("i", 12, 4, 1)
     B, n = 5 * jm, A.shape[0]
@@ -183,6 +183,13 @@ def test_growth_in_the_upward_elimination_is_noticed():
         x = lu.solve(b)
         assert float((x - ref).norm()) <= 40 * n * cond * 2.0 ** -53 * float(ref.norm())
         assert lu.np_lu and lu.mid == lu.nb
+    # left to refine()
+    lu = BlockBandLU(im, jm, check=False).factor(*to_csr(A))
+    x = lu.solve(b)
+    assert not float((x - ref).norm()) <= 1e-6 * float(ref.norm())
+    assert refine(lu, to_csr(A), b, x)[1] <= SOLVE_TOL
+    assert float((x - ref).norm()) <= 40 * n * cond * 2.0 ** -53 * float(ref.norm())
+    assert lu.np_lu and lu.mid == lu.nb
 
 
 @pytest.mark.parametrize("pivot", [2e-14, 0.0])
