@@ -45,9 +45,12 @@ import numpy as np
 
 from . import device as dev
 
-# residual of a solve, relative to the right-hand side, above which the matrix
-# is factored again a safer way: the solves of the Newton matrices end at 1e-12
-# to 1e-15, and 1e-8 still gives Newton its full step
+# A solve is corrected to a residual of REFINE_TOL times the right-hand side, at
+# most REFINE_STEPS times.  Above SOLVE_TOL after that entries grew in the
+# elimination, which chooses no pivot across the blocks (the pivots of its tiles
+# do not show it), and the matrix is factored again a safer way: the Newton
+# matrices end at 1e-12 to 1e-15, and 1e-8 still gives Newton its full step.
+REFINE_TOL, REFINE_STEPS = 1e-12, 3
 SOLVE_TOL = 1e-8
 
 
@@ -334,12 +337,13 @@ class BlockBandLU:
         b = b.reshape(-1).contiguous()
         if self.np_lu and self.diag == "inv":
             check_vector(b, self.R)
-            x = self._corrected(b)
-            if not self.check or differentiated(b):
-                return x
-            while not self._accurate(x, b) and self.refactor():
-                x = self._corrected(b) if self.np_lu else self._apply(b)
-            return x
+            if not self.check or differentiated(b) or self.t.cuda.is_current_stream_capturing():
+                return self._corrected(b)  # (a captured solve cannot ask for its residual)
+            while self.np_lu:
+                x, rel = self._settled(b)
+                if rel <= SOLVE_TOL:
+                    return x
+                self.refactor()
         return self._apply(b)
 
     def _corrected(self, b):
@@ -353,15 +357,26 @@ class BlockBandLU:
         r = csr_residual(self.csr, x, b)
         return r if self.shift is None else r + self.shift * x
 
-    def _accurate(self, x, b):
-        """||b - A x|| <= SOLVE_TOL ||b||.  No pivot is chosen across the
-        blocks, so the entries may grow in the elimination, which the pivots
-        of the tiles do not show; the residual does."""
-        t = self.t
-        if not self.np_lu or t.cuda.is_current_stream_capturing():
-            return True  # (pivoted already; a captured solve cannot ask)
-        rn, bn = t.stack((self._residual(x, b).norm(), b.norm())).tolist()
-        return rn <= SOLVE_TOL * bn or not math.isfinite(bn)
+    def _settled(self, b):
+        """x and its residual relative to b, corrected as refine() does: while
+        the residual is above REFINE_TOL and a correction halves it."""
+        x = self._corrected(b)
+        r, rel = self._rest(x, b)
+        for _ in range(REFINE_STEPS):
+            if rel <= REFINE_TOL:
+                break
+            y = x + self._apply(r)
+            r, new = self._rest(y, b)
+            if not new <= 0.5 * rel:
+                break
+            x, rel = y, new
+        return x, rel
+
+    def _rest(self, x, b):
+        """b - A x, and its norm relative to b's (0 where that is none)."""
+        r = self._residual(x, b)
+        rn, bn = self.t.stack((r.norm(), b.norm())).tolist()
+        return r, rn / bn if 0.0 < bn < math.inf else 0.0
 
     def _safer(self):
         """The next factorization's way: downwards only, as the flow runs, then
@@ -501,7 +516,7 @@ def csr_residual(csr, x, b):
     return r
 
 
-def refine(lu, csr, b, x, rtol=1e-12, steps=3):
+def refine(lu, csr, b, x, rtol=REFINE_TOL, steps=REFINE_STEPS):
     """Iterative refinement of x (in place) for A x = b with the factors of
     lu, until ||b - A x|| <= rtol ||b||, a correction no longer halves the
     residual (its rounding floor), or `steps` corrections: the guard of the
