@@ -56,14 +56,6 @@ __host__ __device__ constexpr double mid_coef(int SI, int SJ) {
   return along == -2 ? -0.0625 : along == -1 ? 0.5625 : along == 0 ? 0.5625 : along == 1 ? -0.0625 : 0.0;
 }
 
-// wb[q] += c d x / d w_q for a Dual<5>; nothing for a value that does not
-// depend on the seeded cell
-__device__ inline void add_d(double wb[5], const Dual<5>& x, double c) {
-#pragma unroll
-  for (int q = 0; q < 5; ++q) wb[q] += c * x.d[q];
-}
-__device__ inline void add_d(double[5], double, double) {}
-
 // primal of the viscous flux (compact, O4, or 2nd-order): face values and
 // gradients
 struct ViscPrimal {

@@ -555,9 +555,12 @@ int bca_residual_dnc5(bca_ctx* c, double* residu, const double* w, bca_metrics g
 }  // extern "C"
 
 // ---------------------------------------------------------- no-allocation residual
-// Scratch of bca_residual_dnc5_noalloc: the prim, grad and hn planes of the
-// residual pipeline, in one file-scope device array that every GPU the
-// library runs on holds until the process ends.  Host code never passes the
+// Scratch of bca_residual_dnc5_noalloc for a residu that shares memory with w (5
+// planes), in one file-scope device array that every GPU the library runs on
+// holds until the process ends.  Its size, and the count of
+// bca_residual_noalloc_bytes (primitives, gradients and fluxes, 21 planes a
+// cell), are those of a pipeline through memory: the meshes that the entry
+// refuses stay the same.  Host code never passes the
 // array's name to a kernel (on the host it is only a stand-in): it passes
 // the device address hipGetSymbolAddress returned for the current device.
 static __device__ __align__(256) double scratch[BCA_NOALLOC_SCRATCH_BYTES / sizeof(double)];
@@ -1707,7 +1710,8 @@ namespace {
 // place of five: a small mesh's tiles are all resident at once, so the pass takes
 // as long as one workgroup's chain; above, each row forming the tables again
 // costs more.  A full CSR with 32 tiles 438 -> 378 us, 276 (two zones) 576 -> 526,
-// 318 495 -> 474; with 632 848 -> 890 (two zones 1115 -> 1097), 960 1478 -> 1631.
+// 318 495 -> 474; with 632 848 -> 890, 960 1478 -> 1631 (two zones, 632 tiles, gain a
+// little still: 1115 -> 1097; one line for both).
 constexpr unsigned EDGE_SPLIT = 400;
 
 // The pruned CSR of the colored Jacobian without the COO (k_jac_csr_rows).
@@ -1950,7 +1954,10 @@ namespace {
 // most of the chip idle; the two directions are independent until they meet,
 // so every launch carries a step of both: half the chain with the same
 // products.  64 block rows of 480 unknowns, kb = 3: 10.3 ms against 16.7 ms
-// downwards only, of 640: 20.8 / 22.3 ms (there the products fill the chip).
+// downwards only, of 640: 20.8 / 22.3 ms.  Larger blocks fill the chip: 384 of
+// 1280 495 / 532 ms, 192 of 1920 827 / 785 ms.  The upward end loses digits
+// against the flow: 384 x 256 boundary layer, coefdiag 1e-3, residual of one
+// solve 2e-5 against 9e-11 downwards (3e-13 and 1e-13 corrected once).
 // With the products by rocBLAS (and torch's subtractions) one Newton iteration
 // on the 256 x 128 boundary layer took 128 ms, now 72 ms.
 //

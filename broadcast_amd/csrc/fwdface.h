@@ -19,7 +19,7 @@
 //
 // What bounds it: the 600 values a face stores (1.9 GB at 512 x 384 for both
 // families, 0.4 ms at the card's copy rate), at one wave per SIMD (256 VGPRs).
-// 512 x 384: i-faces 0.35 ms, j-faces 0.28 ms beside the ghost tangents, where
+// 512 x 384: i-faces 0.29 ms, j-faces 0.21 ms beside the ghost tangents, where
 // 24 seeded passes per face (each recomputing the face's primal, a launch per
 // offset) took 1.1 ms.  131 x 67: 47 + 50 us for the interior families and
 // 21-27 us for the rows next to the wall, where the seeded passes took 48

@@ -259,9 +259,9 @@ class Flow:
         return indptr, indices[:nnz.value], data[:nnz.value]
 
     def autotune(self, w, jac=None, reps=3):
-        """Choose the launch shapes of the residual faces, the face blocks and
-        the colored assembly for this mesh by timing candidates on w (ghosts
-        as given); later calls on this Flow use them.  Returns the report."""
+        """Choose the launch shapes of the face blocks and the colored assembly
+        for this mesh by timing candidates on w (ghosts as given); later calls
+        on this Flow use them.  Returns the report."""
         split = self.two_zone_split
         nz, zp = (1, int(self.case.kind == "cyl")) if split is None else (2, split)
         scratch = jac if jac is not None else self.t.empty(self.nbentry, dtype=self.t.float64, device="cuda")
